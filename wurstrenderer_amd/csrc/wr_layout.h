@@ -20,8 +20,9 @@ constexpr uint32_t kEmptyChild = 0xFFFFFFFFu;
 constexpr int kMaxLeafTris = 4;
 constexpr uint32_t kMaxTriangles = 1u << 28;  // leaf refs hold 28-bit triangle offsets
 constexpr int kStackDepth = 64;     // traversal stack entries per ray (worst case the builder allows)
-constexpr int kLdsStackDepth = 8;   // entries kept in LDS (4 KB per wave); deeper entries spill to a per-lane global region
-constexpr int kSpillDepth = kStackDepth - kLdsStackDepth;
+constexpr int kLdsSlots = 10;       // stack slots kept in LDS, slot 0 the end mark (5 KB per wave: 32 waves fill
+                                    // a CU's 160 KB); deeper slots spill to a per-lane global region
+constexpr int kSpillDepth = kStackDepth + 1 - kLdsSlots;
 constexpr int kMaxTraversalBlocksPerCU = 32;  // bound on traversal grid size (sizes the spill region)
 
 struct alignas(128) Node4 {
@@ -33,23 +34,26 @@ struct alignas(128) Node4 {
 static_assert(sizeof(Node4) == 128, "Node4 must be one cache line");
 
 // The traversal copy of a Node4: 64 B in four 16-byte rows, so a node visit is
-// four loads instead of seven (traversal is bound by the L1's rate of lane
-// requests, not by arithmetic).  Each child box is stored as 8-bit planes on a
-// per-node, per-axis grid of 256 planes: plane q of axis a stands for the FP32 value
-// fmaf(q, scale_a, origin_a), computed exactly so by the kernels, and the
-// quantiser (k_quantize_nodes) picks every low plane so that this float is <=
-// the child's lo and every high plane so that it is >= its hi: the decoded box
-// contains the Node4 box, and the kernels' slab test runs on these floats
-// unchanged.  Rows: (origin xyz, scale x), (lo_x, hi_x, lo_y, hi_y),
-// (lo_z, hi_z, child 0, child 1), (child 2, child 3, scale y, scale z); byte i
-// of a plane word is child i's plane.  An empty child keeps kEmptyChild (its
-// planes 255 / 0) and is rejected by its ref.
+// four loads instead of seven.  Each child box is stored as 8-bit planes on a
+// per-node, per-axis grid of 256 planes: plane q of axis a lies at
+// origin_a + q * spacing_a (exact arithmetic), and the quantiser
+// (k_quantize_nodes) picks every low plane at or below the child's lo and every
+// high plane at or above its hi.  The kernels read a plane as the
+// half-precision denormal q * 2^-24 and the node stores spacing * 2^24, so one
+// fused multiply-add crosses a plane (node_test).  Each child ref sits in the
+// low word of an aligned pair, where the kernels put the entry distance beside
+// it without a move.  The bytes of a plane word ab, from the lowest, are child
+// a's low plane, b's low, a's high, b's high.  An empty child keeps kEmptyChild
+// (its planes 255 / 0) and is rejected by its ref.
 struct alignas(64) NodeQ {
     float org[3];
-    float scale_x;       // grid spacing
-    uint32_t q[6];       // lo_x, hi_x, lo_y, hi_y, lo_z, hi_z
-    uint32_t child[4];   // as Node4::child
-    float scale_y, scale_z;
+    float scale_x;       // grid spacing * 2^24
+    uint32_t x01, x23, y01, y23;
+    uint32_t child0, z01, child1, z23;   // refs as Node4::child
+    uint32_t child2;
+    float scale_y;
+    uint32_t child3;
+    float scale_z;
 };
 static_assert(sizeof(NodeQ) == 64, "NodeQ is four 16-byte rows");
 

@@ -129,12 +129,13 @@ __global__ void k_rotate(PathBuffers pb, RenderArgs a) {
 }
 // The traversal copy of the BVH4 (NodeQ), one node per thread.  Per axis the
 // grid starts at the smallest lo of the node's children and its spacing is
-// (largest hi - origin) / 255, raised by ulps until plane 255, decoded as the
-// kernels decode it (fmaf(q, scale, origin)), reaches the largest hi.  A child's low plane is the
-// largest q whose decoded value is <= its lo, its high plane the smallest q
-// whose decoded value is >= its hi: q = 0 decodes to the origin (<= every lo)
-// and q = 255 to at least the largest hi, so both exist and the decoded box
-// contains the child's box.
+// (largest hi - origin) / 255, raised by ulps until plane 255 reaches the
+// largest hi.  A child's low plane is the largest q whose plane is <= its lo,
+// its high plane the smallest q whose plane is >= its hi: plane 0 is the origin
+// (<= every lo) and plane 255 is at or above the largest hi, so both exist and
+// the planes contain the child's box.  Planes are compared in FP64 as offsets
+// from the origin: q * spacing is exact there, and a plane - origin difference
+// is rounded by at most 2^-53 of itself, far inside the traversal's margin.
 __global__ void k_quantize_nodes(const Node4 *__restrict__ in, NodeQ *__restrict__ out, uint32_t n) {
     const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= n) return;
@@ -142,6 +143,7 @@ __global__ void k_quantize_nodes(const Node4 *__restrict__ in, NodeQ *__restrict
     const float *lo[3] = {nd.lo_x, nd.lo_y, nd.lo_z}, *hi[3] = {nd.hi_x, nd.hi_y, nd.hi_z};
     NodeQ q;
     float scale[3];
+    uint32_t pl[6];
     for (int a = 0; a < 3; a++) {
         float org = FLT_MAX, top = -FLT_MAX;
         for (int c = 0; c < 4; c++)
@@ -150,34 +152,35 @@ __global__ void k_quantize_nodes(const Node4 *__restrict__ in, NodeQ *__restrict
                 top = fmaxf(top, hi[a][c]);
             }
         if (!(org <= top)) org = top = 0.f;  // no child
-        float sc = fmaxf(float((double(top) - double(org)) / 255.0), FLT_MIN);
-        while (fmaf(255.f, sc, org) < top) sc = nextafterf(sc, INFINITY);
-        uint32_t wl = 0, wh = 0;
+        const double ext = double(top) - double(org);
+        float sc = fmaxf(float(ext / 255.0), FLT_MIN);
+        while (255.0 * double(sc) < ext) sc = nextafterf(sc, INFINITY);
+        uint32_t w[2] = {0u, 0u};  // children 0 and 1, 2 and 3
         for (int c = 0; c < 4; c++) {
             uint32_t ql = 255, qh = 0;  // empty slot
             if (nd.child[c] != kEmptyChild) {
-                const float l = lo[a][c], h = hi[a][c];
-                int a0 = int(fmin(255.0, fmax(0.0, floor((double(l) - org) / sc))));
-                while (a0 > 0 && fmaf(float(a0), sc, org) > l) a0--;
-                while (a0 < 255 && fmaf(float(a0 + 1), sc, org) <= l) a0++;
-                int b0 = int(fmin(255.0, fmax(0.0, ceil((double(h) - org) / sc))));
-                while (b0 < 255 && fmaf(float(b0), sc, org) < h) b0++;
-                while (b0 > 0 && fmaf(float(b0 - 1), sc, org) >= h) b0--;
+                const double l = double(lo[a][c]) - double(org), h = double(hi[a][c]) - double(org), s = double(sc);
+                int a0 = int(fmin(255.0, fmax(0.0, floor(l / s))));
+                while (a0 > 0 && a0 * s > l) a0--;
+                while (a0 < 255 && (a0 + 1) * s <= l) a0++;
+                int b0 = int(fmin(255.0, fmax(0.0, ceil(h / s))));
+                while (b0 < 255 && b0 * s < h) b0++;
+                while (b0 > 0 && (b0 - 1) * s >= h) b0--;
                 ql = uint32_t(a0);
                 qh = uint32_t(b0);
             }
-            wl |= ql << (8 * c);
-            wh |= qh << (8 * c);
+            w[c >> 1] |= (ql << (8 * (c & 1))) | (qh << (16 + 8 * (c & 1)));
         }
         q.org[a] = org;
-        scale[a] = sc;
-        q.q[2 * a] = wl;
-        q.q[2 * a + 1] = wh;
+        scale[a] = sc * 0x1p24f;
+        pl[2 * a] = w[0];
+        pl[2 * a + 1] = w[1];
     }
     q.scale_x = scale[0];
     q.scale_y = scale[1];
     q.scale_z = scale[2];
-    for (int c = 0; c < 4; c++) q.child[c] = nd.child[c];
+    q.x01 = pl[0]; q.x23 = pl[1]; q.y01 = pl[2]; q.y23 = pl[3]; q.z01 = pl[4]; q.z23 = pl[5];
+    q.child0 = nd.child[0]; q.child1 = nd.child[1]; q.child2 = nd.child[2]; q.child3 = nd.child[3];
     out[k] = q;
 }
 
@@ -398,15 +401,19 @@ struct TravTune {
     uint32_t refill = WR_REFILL_LANES;
 };
 
-// The traversal kernels run 8 waves per SIMD without spills: the plain one
-// (k_trace_bounce_fast) in 59 VGPRs (7 waves measured 0.8% slower on the
-// 1.31M-triangle frame, 1.4% in the gap room), the batched and counting
-// instances in 62-64 (the batched one at the compiler's 7 waves made the
-// 32-scene batch 3.5% slower: 1.627 against 1.570 s).
+// Waves per SIMD of the traversal kernels.  The plain one runs 7: its registers
+// then fit without spills, and with the shorter node step the L1's rate of lane
+// requests binds before latency does (1.31M-triangle frame 46.5 ms at 7 waves,
+// 46.7 at 8, 47.5 at 6; gap room 47.4 / 48.4 / 48.6; fog 35.7 / 35.7 / 37.2).
+// The batched instance, whose lanes read different scenes, runs 8 (16 scenes
+// 16.8 ms, 18.0 at 7).
 #ifndef WR_EXTEND_WAVES
-#define WR_EXTEND_WAVES 8
+#define WR_EXTEND_WAVES 7
 #endif
-#define WR_EXTEND_ATTR __attribute__((amdgpu_waves_per_eu(WR_EXTEND_WAVES, WR_EXTEND_WAVES)))
+#ifndef WR_BATCH_WAVES
+#define WR_BATCH_WAVES 8
+#endif
+#define WR_EXTEND_ATTR(W) __attribute__((amdgpu_waves_per_eu(W, W)))
 
 struct WaveRange {
     uint32_t lo = 0, hi = 0;  // wave-uniform
@@ -462,14 +469,15 @@ __device__ __forceinline__ uint32_t spread_chunk(uint32_t n, uint32_t chunk) {
 }
 
 // Closest hit for the n active paths of the current state.  `st_ent` is the
-// block's LDS stack (kLdsStackDepth x kBlock entries).
+// block's LDS stack (kLdsSlots x kBlock entries).
 template <bool COUNT, bool BATCH>
 __device__ __forceinline__ void extend_rays(DScene s1, const BatchJob *__restrict__ jobs, PathBuffers pb, uint2 *spill,
                                             TravTune tune, uint32_t n, uint64_t *st_ent) {
     const uint32_t chunk = spread_chunk(n, tune.chunk);
-    LaneStack<kBlock> st(st_ent + lane_id(), reinterpret_cast<uint32_t *>(st_ent) + lane_id(), spill);
+    LaneStack<kBlock, false> st(st_ent, spill);
     TraversalCounters cnt;
     TravState ts;
+    ts.cur = kEndRef;
     uint32_t p = 0;
     WaveRange wr;
     Geo geo{s1.nodes, s1.tris};
@@ -485,8 +493,8 @@ __device__ __forceinline__ void extend_rays(DScene s1, const BatchJob *__restric
                     const DScene &sj = jobs[pb.cur.meta[p].z >> kBounceBits].s;
                     geo = Geo{sj.nodes, sj.tris};
                 }
-                trav_begin(ts, xyz(o), xyz(d), kRayEps, INFINITY);
-                st.sp = 0;
+                trav_begin(ts, setup_ray(xyz(o), xyz(d), kRayEps), INFINITY);
+                st.reset();
                 active = true;
             }
         }
@@ -494,9 +502,9 @@ __device__ __forceinline__ void extend_rays(DScene s1, const BatchJob *__restric
             if (exhausted) break;
             continue;
         }
-        const bool fin = BATCH ? trav_round<COUNT, kBlock>(geo, ts, st, cnt, active)
-                               : trav_round<COUNT, kBlock>(s1, ts, st, cnt, active);
-        if (active && fin) {
+        if (BATCH) trav_round<COUNT, kBlock>(geo, ts, st, cnt);
+        else trav_round<COUNT, kBlock>(s1, ts, st, cnt);
+        if (active && ts.cur == kEndRef) {
             pb.hit[p] = make_uint2(ts.hit, __float_as_uint(ts.t));
             active = false;
         }
@@ -1138,11 +1146,12 @@ __global__ __launch_bounds__(kShadeBlock) void k_shade_ext(DScene s, PathBuffers
 // node refs (any hit keeps no entry distances).
 template <bool COUNT, bool BATCH>
 __device__ __forceinline__ void shadow_rays(DScene s1, const BatchJob *__restrict__ jobs, PathBuffers pb, uint2 *spill,
-                                            TravTune tune, uint32_t n, uint32_t *st_node) {
+                                            TravTune tune, uint32_t n, uint64_t *st_ent) {
     const uint32_t chunk = spread_chunk(n, tune.chunk);
-    LaneStack<kBlock> st(nullptr, st_node + lane_id(), spill);
+    LaneStack<kBlock, true> st(st_ent, spill);
     TraversalCounters cnt;
     TravState ts;
+    ts.cur = kEndRef;
     uint32_t i = 0;
     WaveRange wr;
     Geo geo{s1.nodes, s1.tris};
@@ -1158,8 +1167,8 @@ __device__ __forceinline__ void shadow_rays(DScene s1, const BatchJob *__restric
                     const DScene &sj = jobs[__float_as_uint(pb.sh_c[i].w)].s;
                     geo = Geo{sj.nodes, sj.tris};
                 }
-                trav_begin(ts, xyz(o), xyz(d), kRayEps, o.w);
-                st.sp = 0;
+                trav_begin(ts, setup_ray(xyz(o), xyz(d), kRayEps), o.w);
+                st.reset();
                 active = true;
             }
         }
@@ -1167,9 +1176,9 @@ __device__ __forceinline__ void shadow_rays(DScene s1, const BatchJob *__restric
             if (exhausted) break;
             continue;
         }
-        const bool fin = BATCH ? trav_round_any<COUNT, kBlock>(geo, ts, st, cnt, active)
-                               : trav_round_any<COUNT, kBlock>(s1, ts, st, cnt, active);
-        if (active && fin) {
+        if (BATCH) trav_round_any<COUNT, kBlock>(geo, ts, st, cnt);
+        else trav_round_any<COUNT, kBlock>(s1, ts, st, cnt);
+        if (active && ts.cur == kEndRef) {
             active = false;
             if (ts.hit == kInvalid) {
                 const float4 c = pb.sh_c[i];
@@ -1208,7 +1217,7 @@ __device__ __forceinline__ void shadow_rays(DScene s1, const BatchJob *__restric
 template <bool COUNT, bool BATCH>
 __device__ __forceinline__ void trace_bounce(DScene s1, const BatchJob *__restrict__ jobs, PathBuffers pb, uint2 *spill,
                                              TravTune tune) {
-    __shared__ uint64_t st_ent[kLdsStackDepth * kBlock];
+    __shared__ uint64_t st_ent[kLdsSlots * kBlock];
     const uint32_t n_ext = active_count(pb.counters);
     const uint32_t n_shd = pb.counters[pb.next.shadow_count];
     const uint32_t g = gridDim.x;
@@ -1216,16 +1225,16 @@ __device__ __forceinline__ void trace_bounce(DScene s1, const BatchJob *__restri
     if (blockIdx.x < ext_blocks) extend_rays<COUNT, BATCH>(s1, jobs, pb, spill, tune, n_ext, st_ent);
     const uint32_t sb = (blockIdx.x + g - ext_blocks) % g;
     if (sb * kBlock < n_shd)
-        shadow_rays<COUNT, BATCH>(s1, jobs, pb, spill, tune, n_shd, reinterpret_cast<uint32_t *>(st_ent));
+        shadow_rays<COUNT, BATCH>(s1, jobs, pb, spill, tune, n_shd, st_ent);
 }
 template <bool COUNT, bool BATCH>
-__global__ __launch_bounds__(kBlock) WR_EXTEND_ATTR void k_trace_bounce(DScene s1, const BatchJob *__restrict__ jobs,
+__global__ __launch_bounds__(kBlock) WR_EXTEND_ATTR(WR_BATCH_WAVES) void k_trace_bounce(DScene s1, const BatchJob *__restrict__ jobs,
                                                                         PathBuffers pb, uint2 *spill, TravTune tune) {
     trace_bounce<COUNT, BATCH>(s1, jobs, pb, spill, tune);
 }
 // The plain kernel of wr_render_nee / wr_render_guided and the other
 // integrators' loops.
-__global__ __launch_bounds__(kBlock) WR_EXTEND_ATTR void k_trace_bounce_fast(DScene s1, PathBuffers pb, uint2 *spill,
+__global__ __launch_bounds__(kBlock) WR_EXTEND_ATTR(WR_EXTEND_WAVES) void k_trace_bounce_fast(DScene s1, PathBuffers pb, uint2 *spill,
                                                                              TravTune tune) {
     trace_bounce<false, false>(s1, nullptr, pb, spill, tune);
 }
@@ -1250,8 +1259,7 @@ __global__ void k_accumulate(const float4 *__restrict__ sample_rad, double *film
 template <bool ANY>
 __global__ __launch_bounds__(kBlock) void k_trace(DScene s, const float4 *__restrict__ rays, uint32_t n, uint2 *hits,
                                                   uint8_t *occ, uint2 *spill) {
-    __shared__ uint64_t st_ent[kLdsStackDepth * kBlock];
-    LaneStack<kBlock> st(st_ent + lane_id(), reinterpret_cast<uint32_t *>(st_ent) + lane_id(), spill);
+    __shared__ uint64_t st_ent[kLdsSlots * kBlock];
     TraversalCounters cnt;
     for (uint32_t base = blockIdx.x * kBlock; base < n; base += gridDim.x * kBlock) {
         const uint32_t i = base + lane_id();
@@ -1259,7 +1267,7 @@ __global__ __launch_bounds__(kBlock) void k_trace(DScene s, const float4 *__rest
             const float4 a = rays[2 * size_t(i)], b = rays[2 * size_t(i) + 1];
             const RaySetup r = setup_ray(xyz(a), xyz(b), a.w);
             float t = b.w;
-            const uint32_t tri = traverse_rounds<ANY, kBlock>(s, r, t, st, cnt);
+            const uint32_t tri = traverse_rounds<ANY, kBlock>(s, r, t, st_ent, spill, cnt);
             if (ANY) occ[i] = tri != kInvalid;
             else hits[i] = make_uint2(tri, __float_as_uint(tri == kInvalid ? INFINITY : t));
         }
@@ -1274,8 +1282,7 @@ __global__ __launch_bounds__(kBlock) void k_trace(DScene s, const float4 *__rest
 // order into the FP64 base film, so the film is bit-reproducible.
 __global__ __launch_bounds__(kBlock) void k_visualize(DScene s, uint32_t wh, uint32_t spp, uint32_t first_sample,
                                                       uint32_t seed, double *film_base, uint2 *spill) {
-    __shared__ uint64_t st_ent[kLdsStackDepth * kBlock];
-    LaneStack<kBlock> st(st_ent + lane_id(), reinterpret_cast<uint32_t *>(st_ent) + lane_id(), spill);
+    __shared__ uint64_t st_ent[kLdsSlots * kBlock];
     TraversalCounters cnt;
     const DCamera &cam = s.cam;
     for (uint32_t pixel = blockIdx.x * kBlock + lane_id(); pixel < wh; pixel += gridDim.x * kBlock) {
@@ -1289,7 +1296,7 @@ __global__ __launch_bounds__(kBlock) void k_visualize(DScene s, uint32_t wh, uin
             const float3 dir = primary_dir(cam, key, px, py, lens, pdfW);
             float t = INFINITY;
             const uint32_t tri = traverse_rounds<false, kBlock>(Geo4{s.fnodes, s.tris}, setup_ray(cpos, dir, kRayEps),
-                                                                t, st, cnt);
+                                                                t, st_ent, spill, cnt);
             if (tri == kInvalid) {
                 if (s.env_select > 0.f) { r += 1.0; g += 1.0; b += 1.0; }  // the envmap vertex is a light vertex
                 continue;
@@ -1357,8 +1364,7 @@ __device__ __forceinline__ float bd_weight(float inv) {
 __global__ __launch_bounds__(kBlock, 4) void k_bdpt(DScene s, uint32_t wh, uint32_t spp, uint32_t first_sample,
                                                  uint32_t seed, int N, double *film_base, double *film_splat,
                                                  float4 *__restrict__ recs, unsigned long long *counts, uint2 *spill) {
-    __shared__ uint64_t st_ent[kLdsStackDepth * kBlock];
-    LaneStack<kBlock> st(st_ent + lane_id(), reinterpret_cast<uint32_t *>(st_ent) + lane_id(), spill);
+    __shared__ uint64_t st_ent[kLdsSlots * kBlock];
     TraversalCounters cnt;
     const DCamera &cam = s.cam;
     const float3 cz = f3(cam.zx, cam.zy, cam.zz);
@@ -1368,12 +1374,12 @@ __global__ __launch_bounds__(kBlock, 4) void k_bdpt(DScene s, uint32_t wh, uint3
     auto occluded = [&](float3 o, float3 d, float len) {
         n_shd++;
         float t = len - kRayEps;
-        return traverse_rounds<true, kBlock>(Geo4{s.fnodes, s.tris}, setup_ray(o, d, kRayEps), t, st, cnt) != kInvalid;
+        return traverse_rounds<true, kBlock>(Geo4{s.fnodes, s.tris}, setup_ray(o, d, kRayEps), t, st_ent, spill, cnt) != kInvalid;
     };
     auto closest = [&](float3 o, float3 d, float &t) {
         n_ext++;
         t = INFINITY;
-        return traverse_rounds<false, kBlock>(Geo4{s.fnodes, s.tris}, setup_ray(o, d, kRayEps), t, st, cnt);
+        return traverse_rounds<false, kBlock>(Geo4{s.fnodes, s.tris}, setup_ray(o, d, kRayEps), t, st_ent, spill, cnt);
     };
     for (uint32_t pixel = blockIdx.x * kBlock + lane_id(); pixel < wh; pixel += gridDim.x * kBlock) {
         const uint32_t px = pixel % uint32_t(cam.W), py = pixel / uint32_t(cam.W);
@@ -1932,6 +1938,7 @@ static int scene_create_impl(wr_device *dev, const wr_scene_desc *d, int builder
     dc.focal = c.focal_distance;
     s->ds.nodes = s->d_qnodes;
     s->ds.fnodes = s->d_nodes;
+    s->ds.n_nodes = uint32_t(s->n_nodes);
     s->ds.tris = s->d_tris;
     s->ds.geom_info = s->d_geom;
     s->ds.mats = s->d_mats;
@@ -1998,8 +2005,7 @@ int wr_scene_bvh_check(wr_scene *s, const wr_scene_desc *d, wr_bvh_stats *st) {
     for (uint32_t i = 0; i < s->n_tris; i++)
         if (tris[i].geom != d->tri_geom[tris[i].orig] || tris[i].orig != s->leaf_to_orig[i])
             return set_error(WR_ERR_DEVICE, "BVH invariant violated: leaf triangle geometry id or order map");
-    // the traversal copy: same refs, and every decoded child box (the kernels'
-    // fmaf(q, scale, origin), IEEE single rounding on both sides) contains the Node4 box
+    // the traversal copy: same refs, and every child's planes (origin + q * spacing) contain its Node4 box
     {
         std::vector<NodeQ> qn(s->n_nodes);
         WR_HIP(hipMemcpy(qn.data(), s->d_qnodes, sizeof(NodeQ) * qn.size(), hipMemcpyDeviceToHost));
@@ -2008,14 +2014,17 @@ int wr_scene_bvh_check(wr_scene *s, const wr_scene_desc *d, wr_bvh_stats *st) {
             const NodeQ &b = qn[i];
             const float *lo[3] = {a.lo_x, a.lo_y, a.lo_z}, *hi[3] = {a.hi_x, a.hi_y, a.hi_z};
             const float sc[3] = {b.scale_x, b.scale_y, b.scale_z};
+            const uint32_t pl[6] = {b.x01, b.x23, b.y01, b.y23, b.z01, b.z23};
+            const uint32_t ref[4] = {b.child0, b.child1, b.child2, b.child3};
             for (int c = 0; c < 4; c++) {
-                if (b.child[c] != a.child[c])
+                if (ref[c] != a.child[c])
                     return set_error(WR_ERR_DEVICE, "BVH invariant violated: quantised node refs differ");
                 if (a.child[c] == kEmptyChild) continue;
                 for (int k = 0; k < 3; k++) {
-                    const float pl = std::fma(float((b.q[2 * k] >> (8 * c)) & 0xFFu), sc[k], b.org[k]);
-                    const float ph = std::fma(float((b.q[2 * k + 1] >> (8 * c)) & 0xFFu), sc[k], b.org[k]);
-                    if (!(pl <= lo[k][c] && ph >= hi[k][c]))
+                    const uint32_t w = pl[2 * k + (c >> 1)] >> (8 * (c & 1));
+                    const double sp = double(sc[k]) * 0x1p-24;
+                    if (!((w & 0xFFu) * sp <= double(lo[k][c]) - double(b.org[k]) &&
+                          ((w >> 16) & 0xFFu) * sp >= double(hi[k][c]) - double(b.org[k])))
                         return set_error(WR_ERR_DEVICE, "BVH invariant violated: quantised box of node " +
                                                             std::to_string(i) + " does not contain its child " +
                                                             std::to_string(c));
