@@ -227,6 +227,10 @@ int wr_film_clear(wr_film *film);
 /* Copies the raw sums to host arrays [H][W][3] (row 0 = top of the image).
  * image = base / spp + splat / (spp * W * H)   (pathnextevent.h:154-157). */
 int wr_film_read(wr_film *film, double *base, double *splat);
+/* The image of the sums, base / base_div + splat / splat_div per value in FP64
+ * (base_div = spp, splat_div = spp * W * H), composed on the device and copied
+ * to the host array rgb[H][W][3]. */
+int wr_film_image(wr_film *film, double base_div, double splat_div, double *rgb);
 
 /* Checks render parameters without touching a GPU: spp, first_sample and
  * max_paths_in_flight >= 0, fetch_chunk <= 4096, refill_lanes <= 64.  Every

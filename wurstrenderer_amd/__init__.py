@@ -136,6 +136,7 @@ EXPORTS = {
     "wr_film_destroy": (None, [P]),
     "wr_film_clear": (C.c_int, [P]),
     "wr_film_read": (C.c_int, [P, P, P]),
+    "wr_film_image": (C.c_int, [P, C.c_double, C.c_double, P]),
     "wr_render_params_validate": (C.c_int, [C.POINTER(RenderParams)]),
     "wr_render_nee": (C.c_int, [P, P, C.POINTER(RenderParams), C.POINTER(RenderStats)]),
     "wr_render_nee_noalloc": (C.c_int, [P, P, C.POINTER(RenderParams), C.POINTER(RenderStats)]),
@@ -451,9 +452,13 @@ class Film:
 
     def image(self):
         """Film::getImage: base/spp + splat/(spp*W*H) (film.h:78-90, pathnextevent.h:154-157)."""
-        base, splat = self.read()
         W, H = self.scene.W, self.scene.H
-        return base / self.spp + splat / (self.spp * W * H)
+        if not self.spp:  # nothing rendered: numpy's 0 / 0
+            base, splat = self.read()
+            return base / self.spp + splat / (self.spp * W * H)
+        rgb = np.empty((H, W, 3), np.float64)
+        _check(lib().wr_film_image(self.h, float(self.spp), float(self.spp * W * H), rgb.ctypes.data))
+        return rgb
 
 
 def render_params(spp=0, num_path_vertices=10, seed=0, use_mis=True, first_sample=0, max_paths_in_flight=0,

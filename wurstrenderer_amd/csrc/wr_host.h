@@ -10,6 +10,7 @@
 #include "../../include/wurst_amd.h"
 #include "wr_device.h"
 #include "wr_layout.h"
+#include "wr_transfer.h"
 
 namespace wr {
 // Thread-local message behind wr_last_error().
@@ -111,6 +112,7 @@ struct wr_device {
     // resident blocks per CU of each kernel (HIP occupancy API), used to size persistent grids
     int occ_rays = 8, occ_shade = 8, occ_generate = 8, occ_trace = 8;
     std::map<const void *, int> occ_cache;  // other kernels, filled on first use
+    TransferRing ring;        // pinned buffers of large host transfers
     void *scratch = nullptr;  // device address of wr_render_nee_noalloc's fixed region on this GPU
 };
 
@@ -127,6 +129,7 @@ struct wr_scene {
     size_t bdpt_bytes = 0;
     int max_trav_blocks = 0;
     int2 *d_geom = nullptr;
+    uint32_t *d_geom_first = nullptr;  // each geometry's first triangle
     DMat *d_mats = nullptr;
     DLight *d_lights = nullptr;
     float4 *d_env = nullptr;            // envmap texels; cdf and pdf follow in d_env_cdf

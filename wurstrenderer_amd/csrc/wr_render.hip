@@ -1255,10 +1255,22 @@ __global__ void k_accumulate(const float4 *__restrict__ sample_rad, double *film
     }
 }
 
+// Film::getImage (film.h:78-90, pathnextevent.h:154-157) of `n` film values:
+// base / spp + splat / (spp W H), written straight to pinned host memory.
+__global__ void k_film_image(const double *__restrict__ base, const double *__restrict__ splat, double base_div,
+                             double splat_div, double *__restrict__ out, uint32_t n) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) out[i] = base[i] / base_div + splat[i] / splat_div;
+}
+
 // ============================================================== trace kernels (parity / benchmark)
-template <bool ANY>
+// Hits leave as (leaf triangle, t) pairs, or, with IDS, as what the host API
+// returns: the geometry, the triangle within it and t in three arrays of n
+// (a triangle record holds its input index and geometry; geom_first is each
+// geometry's first triangle).
+template <bool ANY, bool IDS = false>
 __global__ __launch_bounds__(kBlock) void k_trace(DScene s, const float4 *__restrict__ rays, uint32_t n, uint2 *hits,
-                                                  uint8_t *occ, uint2 *spill) {
+                                                  uint8_t *occ, const uint32_t *__restrict__ geom_first, uint2 *spill) {
     __shared__ uint64_t st_ent[kLdsSlots * kBlock];
     TraversalCounters cnt;
     for (uint32_t base = blockIdx.x * kBlock; base < n; base += gridDim.x * kBlock) {
@@ -1269,7 +1281,17 @@ __global__ __launch_bounds__(kBlock) void k_trace(DScene s, const float4 *__rest
             float t = b.w;
             const uint32_t tri = traverse_rounds<ANY, kBlock>(s, r, t, st_ent, spill, cnt);
             if (ANY) occ[i] = tri != kInvalid;
-            else hits[i] = make_uint2(tri, __float_as_uint(tri == kInvalid ? INFINITY : t));
+            else if (IDS) {
+                uint32_t *out = reinterpret_cast<uint32_t *>(hits);
+                uint32_t geom = kInvalid, prim = kInvalid;
+                if (tri != kInvalid) {
+                    geom = __float_as_uint(s.tris[3 * size_t(tri) + 1].w);
+                    prim = __float_as_uint(s.tris[3 * size_t(tri)].w) - geom_first[geom];
+                }
+                out[i] = geom;
+                out[size_t(n) + i] = prim;
+                out[2 * size_t(n) + i] = __float_as_uint(tri == kInvalid ? INFINITY : t);
+            } else hits[i] = make_uint2(tri, __float_as_uint(tri == kInvalid ? INFINITY : t));
         }
     }
 }
@@ -1663,6 +1685,7 @@ void wr_scene_destroy(wr_scene *s) {
     (void)hipFree(s->d_tris);
     (void)hipFree(s->d_ltris);
     (void)hipFree(s->d_geom);
+    (void)hipFree(s->d_geom_first);
     (void)hipFree(s->d_mats);
     (void)hipFree(s->d_lights);
     (void)hipFree(s->d_env);
@@ -1830,6 +1853,7 @@ static int scene_create_impl(wr_device *dev, const wr_scene_desc *d, int builder
     std::vector<int2> gi(d->n_geoms);
     for (uint32_t g = 0; g < d->n_geoms; g++) gi[g] = make_int2(d->geom_material[g], d->geom_light[g]);
     rc = upload(&s->d_geom, gi.data(), sizeof(int2) * gi.size(), s->device_bytes);
+    if (!rc) rc = upload(&s->d_geom_first, s->geom_first.data(), sizeof(uint32_t) * s->geom_first.size(), s->device_bytes);
     if (rc) return rc;
     std::vector<DMat> mats(d->n_materials);
     for (uint32_t m = 0; m < d->n_materials; m++) {
@@ -2218,12 +2242,36 @@ int wr_film_clear(wr_film *f) {
 
 int wr_film_read(wr_film *f, double *base, double *splat) {
     if (!f) return set_error(WR_ERR_INVALID_ARGUMENT, "film is null");
-    int rc = set_device(f->scene->dev);
+    wr_device *dev = f->scene->dev;
+    int rc = set_device(dev);
     if (rc) return rc;
     const size_t bytes = sizeof(double) * 3 * size_t(f->W) * f->H;
-    WR_HIP(hipStreamSynchronize(f->scene->stream));
-    if (base) WR_HIP(hipMemcpy(base, f->d_base, bytes, hipMemcpyDeviceToHost));
-    if (splat) WR_HIP(hipMemcpy(splat, f->d_splat, bytes, hipMemcpyDeviceToHost));
+    hipStream_t st = f->scene->stream;
+    for (auto &[dst, src] : {std::make_pair(base, f->d_base), std::make_pair(splat, f->d_splat)}) {
+        if (!dst) continue;
+        const char *from = reinterpret_cast<const char *>(src);
+        WR_HIP(dev->ring.download(dev->ordinal, st, dst, bytes, [&](size_t off, size_t n, char *slot) {
+            return hipMemcpyAsync(slot, from + off, n, hipMemcpyDeviceToHost, st);
+        }));
+    }
+    WR_HIP(hipStreamSynchronize(st));
+    return WR_OK;
+}
+
+int wr_film_image(wr_film *f, double base_div, double splat_div, double *rgb) {
+    if (!f || !rgb) return set_error(WR_ERR_INVALID_ARGUMENT, "null argument");
+    wr_device *dev = f->scene->dev;
+    int rc = set_device(dev);
+    if (rc) return rc;
+    const size_t bytes = sizeof(double) * 3 * size_t(f->W) * f->H;
+    hipStream_t st = f->scene->stream;
+    WR_HIP(dev->ring.download(dev->ordinal, st, rgb, bytes, [&](size_t off, size_t n, char *slot) {
+        const size_t first = off / sizeof(double);
+        const uint32_t count = uint32_t(n / sizeof(double));
+        k_film_image<<<(count + 255) / 256, 256, 0, st>>>(f->d_base + first, f->d_splat + first, base_div, splat_div,
+                                                          reinterpret_cast<double *>(slot), count);
+        return hipGetLastError();
+    }));
     return WR_OK;
 }
 
@@ -3032,16 +3080,18 @@ int wr_autotune(const wr_batch_job *jobs, uint32_t n_jobs, const wr_render_param
     return WR_OK;
 }
 
-static int trace_impl(wr_scene *s, const float *d_rays, uint32_t n, void *d_hits, uint8_t *d_occ, bool any, float *ms) {
+static int trace_impl(wr_scene *s, const float *d_rays, uint32_t n, void *d_hits, uint8_t *d_occ, bool any, float *ms,
+                      bool ids = false) {
     int rc = set_device(s->dev);
     if (rc) return rc;
     if (n == 0) { if (ms) *ms = 0.f; return WR_OK; }
     const int grid = trav_grid(s, n, s->dev->occ_trace);
     if (ms) WR_HIP(hipEventRecord(s->ev[0], s->stream));
-    if (any) k_trace<true><<<grid, kBlock, 0, s->stream>>>(s->ds, reinterpret_cast<const float4 *>(d_rays), n, nullptr,
-                                                           d_occ, s->d_spill);
-    else k_trace<false><<<grid, kBlock, 0, s->stream>>>(s->ds, reinterpret_cast<const float4 *>(d_rays), n,
-                                                         reinterpret_cast<uint2 *>(d_hits), nullptr, s->d_spill);
+    const float4 *rays = reinterpret_cast<const float4 *>(d_rays);
+    uint2 *hits = reinterpret_cast<uint2 *>(d_hits);
+    if (any) k_trace<true><<<grid, kBlock, 0, s->stream>>>(s->ds, rays, n, nullptr, d_occ, nullptr, s->d_spill);
+    else if (ids) k_trace<false, true><<<grid, kBlock, 0, s->stream>>>(s->ds, rays, n, hits, nullptr, s->d_geom_first, s->d_spill);
+    else k_trace<false><<<grid, kBlock, 0, s->stream>>>(s->ds, rays, n, hits, nullptr, nullptr, s->d_spill);
     WR_HIP(hipGetLastError());
     if (ms) {
         WR_HIP(hipEventRecord(s->ev[1], s->stream));
@@ -3061,57 +3111,50 @@ int wr_trace_any_device(wr_scene *s, const float *d_rays, uint32_t n, uint8_t *d
     return trace_impl(s, d_rays, n, nullptr, d_occ, true, ms);
 }
 
+// Rays from host arrays: staged up, traced, results staged down.  The device
+// buffer (rays, then results) lives for the call.
+template <class Read>
+static int trace_host(wr_scene *s, const float *rays, uint32_t n, size_t result_bytes, bool any, Read &&read) {
+    int rc = set_device(s->dev);
+    if (rc) return rc;
+    const size_t ray_bytes = sizeof(float) * 8 * size_t(n);
+    char *d = nullptr;
+    WR_HIP(hipMalloc(reinterpret_cast<void **>(&d), ray_bytes + result_bytes));
+    hipError_t e = s->dev->ring.upload(s->dev->ordinal, s->stream, d, rays, ray_bytes);
+    char *d_out = d + ray_bytes;
+    if (e == hipSuccess) {
+        rc = any ? trace_impl(s, reinterpret_cast<const float *>(d), n, nullptr, reinterpret_cast<uint8_t *>(d_out), true, nullptr)
+                 : trace_impl(s, reinterpret_cast<const float *>(d), n, d_out, nullptr, false, nullptr, true);
+        if (rc == WR_OK) e = read(d_out);
+    }
+    (void)hipStreamSynchronize(s->stream);
+    (void)hipFree(d);
+    if (rc) return rc;
+    if (e != hipSuccess) return set_error(WR_ERR_DEVICE, hipGetErrorString(e));
+    return WR_OK;
+}
+
 int wr_trace_closest(wr_scene *s, const float *rays, uint32_t n, uint32_t *geom, uint32_t *prim, float *t) {
     if (!s || (n && (!rays || !geom || !prim || !t))) return set_error(WR_ERR_INVALID_ARGUMENT, "null argument");
     if (n == 0) return WR_OK;
-    int rc = set_device(s->dev);
-    if (rc) return rc;
-    float *d_rays = nullptr;
-    uint2 *d_hits = nullptr;
-    WR_HIP(hipMalloc(&d_rays, sizeof(float) * 8 * size_t(n)));
-    hipError_t e = hipMalloc(&d_hits, sizeof(uint2) * size_t(n));
-    if (e != hipSuccess) { (void)hipFree(d_rays); return set_error(WR_ERR_OUT_OF_MEMORY, hipGetErrorString(e)); }
-    std::vector<uint2> hits(n);
-    e = hipMemcpy(d_rays, rays, sizeof(float) * 8 * size_t(n), hipMemcpyHostToDevice);
-    if (e == hipSuccess) rc = trace_impl(s, d_rays, n, d_hits, nullptr, false, nullptr);
-    if (e == hipSuccess && rc == WR_OK) e = hipStreamSynchronize(s->stream);
-    if (e == hipSuccess && rc == WR_OK) e = hipMemcpy(hits.data(), d_hits, sizeof(uint2) * size_t(n), hipMemcpyDeviceToHost);
-    (void)hipFree(d_rays);
-    (void)hipFree(d_hits);
-    if (rc) return rc;
-    if (e != hipSuccess) return set_error(WR_ERR_DEVICE, hipGetErrorString(e));
-    for (uint32_t i = 0; i < n; i++) {
-        if (hits[i].x == kInvalid) {
-            geom[i] = prim[i] = WR_INVALID_ID;
-            t[i] = INFINITY;
-        } else {
-            const uint32_t orig = s->leaf_to_orig[hits[i].x];
-            geom[i] = s->tri_geom[orig];
-            prim[i] = orig - s->geom_first[geom[i]];
-            std::memcpy(&t[i], &hits[i].y, 4);
-        }
-    }
-    return WR_OK;
+    const size_t bytes = sizeof(uint32_t) * size_t(n);
+    return trace_host(s, rays, n, 3 * bytes, false, [&](const char *d_out) {
+        void *dst[3] = {geom, prim, t};
+        hipError_t e = hipSuccess;
+        for (int k = 0; k < 3 && e == hipSuccess; k++)
+            e = s->dev->ring.download(s->dev->ordinal, s->stream, dst[k], bytes, [&](size_t off, size_t m, char *slot) {
+                return hipMemcpyAsync(slot, d_out + k * bytes + off, m, hipMemcpyDeviceToHost, s->stream);
+            });
+        return e;
+    });
 }
 
 int wr_trace_any(wr_scene *s, const float *rays, uint32_t n, uint8_t *occluded) {
     if (!s || (n && (!rays || !occluded))) return set_error(WR_ERR_INVALID_ARGUMENT, "null argument");
     if (n == 0) return WR_OK;
-    int rc = set_device(s->dev);
-    if (rc) return rc;
-    float *d_rays = nullptr;
-    uint8_t *d_occ = nullptr;
-    WR_HIP(hipMalloc(&d_rays, sizeof(float) * 8 * size_t(n)));
-    hipError_t e = hipMalloc(&d_occ, size_t(n));
-    if (e != hipSuccess) { (void)hipFree(d_rays); return set_error(WR_ERR_OUT_OF_MEMORY, hipGetErrorString(e)); }
-    e = hipMemcpy(d_rays, rays, sizeof(float) * 8 * size_t(n), hipMemcpyHostToDevice);
-    if (e == hipSuccess) rc = trace_impl(s, d_rays, n, nullptr, d_occ, true, nullptr);
-    if (e == hipSuccess && rc == WR_OK) e = hipStreamSynchronize(s->stream);
-    if (e == hipSuccess && rc == WR_OK) e = hipMemcpy(occluded, d_occ, size_t(n), hipMemcpyDeviceToHost);
-    (void)hipFree(d_rays);
-    (void)hipFree(d_occ);
-    if (rc) return rc;
-    if (e != hipSuccess) return set_error(WR_ERR_DEVICE, hipGetErrorString(e));
-    return WR_OK;
+    return trace_host(s, rays, n, n, true, [&](const char *d_out) {
+        return s->dev->ring.download(s->dev->ordinal, s->stream, occluded, n, [&](size_t off, size_t m, char *slot) {
+            return hipMemcpyAsync(slot, d_out + off, m, hipMemcpyDeviceToHost, s->stream);
+        });
+    });
 }
-
