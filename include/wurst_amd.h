@@ -248,7 +248,7 @@ int wr_render_nee(wr_scene *scene, wr_film *film, const wr_render_params *params
  * reference; it is for callers that cannot allocate device memory during the
  * call (code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc).  The film and scene are the caller's; the path pool,
- * per-sample radiance, counters and traversal spill live in a fixed 77 MiB
+ * per-sample radiance, counters and traversal spill live in a fixed 74 MiB
  * region that the library reserves on each GPU it runs on (held until the
  * process ends), so the call makes no hipMalloc/hipFree, creates no events and
  * instantiates no graph.  Limits: a frame of at most 2^20 pixels (passes of at

@@ -48,13 +48,15 @@ constexpr uint32_t kToSplat = 2u << 30;      // light->camera splat (pixel of th
 // Path state in queue order (SoA, double buffered): entry i of the current
 // state is the i-th active path.  Shade writes continuing paths compacted into
 // the next state; regen appends new samples behind them.  Every kernel walks
-// the state in order, so all path-state traffic is coalesced.
+// the state in order, so all path-state traffic is coalesced, and the shade
+// kernel, which reads and writes it all, is close to the rate of a plain copy:
+// an entry is four full 16-byte rows, the integers in the rows' fourth words.
 struct PathState {
-    float4 *ray_o, *ray_d;  // ray to extend
+    float4 *ray_o, *ray_d;  // ray to extend; w: RNG key, sample index in the pass (bits)
     float4 *thr;            // rgb: throughput of the next vertex; w: pdfW of the ray direction
-    float4 *rad;            // rgb: radiance gathered so far (FP32)
-    uint4 *meta;            // x: RNG key, y: sample index in the pass, z: bounce of the next vertex,
-                            // w: 1 + training record of the previous vertex (0: none)
+    float4 *rad;            // rgb: radiance gathered so far (FP32); w: bounce of the next vertex,
+                            // and the job in the bits above kBounceBits (bits)
+    uint32_t *rec;          // 1 + training record of the previous vertex (0: none); guided renders only
     uint32_t shadow_count;  // counter (kShadowA or kShadowB) of the shadow queue that the shade
                             // kernel appends to while this state is current; the two states
                             // hold the two counters and swap them with everything else
@@ -102,6 +104,7 @@ struct RenderArgs {
     int N;                    // num_path_vertices
     int use_mis;
     int nee;                  // 1: PathNeeRenderer (NEE, t = 1 splats); 0: PrimitivePathRenderer (BSDF sampling only)
+    int guided;               // 1: entries carry a training record (PathState::rec)
     int light;                // 1: LightSplattingRenderer (light subpaths connected to the camera)
 };
 

@@ -61,9 +61,9 @@ __device__ __forceinline__ uint32_t wave_append(uint32_t *counter, bool pred) {
     return pred ? base + mbcnt64(mask) : kInvalid;
 }
 
-// Block-aggregated append for kShadeBlock-thread blocks: one atomic per block.
+// Block-aggregated append: one atomic per block of up to kShadeBlock threads.
 // All threads of the block must call it (it synchronises the block).
-constexpr int kShadeBlock = 256;
+constexpr int kShadeBlock = 512;
 constexpr int kWavesPerShadeBlock = kShadeBlock / 64;
 __device__ __forceinline__ uint32_t block_append(uint32_t *counter, bool pred, uint32_t *lds /* kWavesPerShadeBlock+1 */) {
     const unsigned long long mask = __ballot(pred);
@@ -72,7 +72,7 @@ __device__ __forceinline__ uint32_t block_append(uint32_t *counter, bool pred, u
     __syncthreads();
     if (threadIdx.x == 0) {
         uint32_t total = 0;
-        for (int w = 0; w < kWavesPerShadeBlock; w++) {
+        for (uint32_t w = 0; w < blockDim.x / 64; w++) {
             const uint32_t k = lds[w];
             lds[w] = total;
             total += k;
@@ -83,6 +83,43 @@ __device__ __forceinline__ uint32_t block_append(uint32_t *counter, bool pred, u
     const uint32_t pos = lds[kWavesPerShadeBlock] + lds[wave] + mbcnt64(mask);
     __syncthreads();  // lds is reused by the next call
     return pred ? pos : kInvalid;
+}
+
+// The shade kernels' two appends at once: continuing paths (a) and shadow rays
+// (b) share one 64-bit counter, paths in the low word, so a block does one
+// atomic and one round of barriers for both.  Atomics on one address are served
+// one after the other, across all XCDs: with two per 256 threads they, not
+// memory, set k_shade's time on the 1.31M-triangle frame (two per 128 threads:
+// +83%).  `flip` alternates between calls, so that a call's LDS words are not
+// overwritten before every wave has read them.
+struct Append2 {
+    uint32_t a, b;  // positions (valid where the predicate is)
+};
+__device__ __forceinline__ Append2 block_append2(uint32_t *counter, bool pa, bool pb,
+                                                 uint32_t (*lds)[kWavesPerShadeBlock + 2], uint32_t flip) {
+    uint32_t *l = lds[flip & 1u];
+    const unsigned long long ma = __ballot(pa), mb = __ballot(pb);
+    const uint32_t wave = threadIdx.x / 64;
+    if (lane_id() == 0) l[wave] = (uint32_t)__popcll(ma) | (uint32_t)__popcll(mb) << 16;  // block sums stay below 2^16
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        uint32_t total = 0;
+        for (uint32_t w = 0; w < blockDim.x / 64; w++) {
+            const uint32_t k = l[w];
+            l[w] = total;
+            total += k;
+        }
+        unsigned long long base = 0;
+        if (total)
+            base = atomicAdd(reinterpret_cast<unsigned long long *>(counter),
+                             (unsigned long long)(total & 0xFFFFu) | (unsigned long long)(total >> 16) << 32);
+        l[kWavesPerShadeBlock] = uint32_t(base);
+        l[kWavesPerShadeBlock + 1] = uint32_t(base >> 32);
+    }
+    __syncthreads();
+    const uint32_t before = l[wave];
+    return {l[kWavesPerShadeBlock] + (before & 0xFFFFu) + mbcnt64(ma),
+            l[kWavesPerShadeBlock + 1] + (before >> 16) + mbcnt64(mb)};
 }
 
 __device__ __forceinline__ void wave_add_stat(unsigned long long *dst, uint32_t v) {
@@ -105,7 +142,10 @@ __device__ __forceinline__ void plan_fresh(uint32_t *c, const RenderArgs &a) {
     c[kClaimed] += fresh;
 }
 __global__ void k_init(PathBuffers pb, RenderArgs a) {
-    if (threadIdx.x < kNumCounterLines) pb.counters[threadIdx.x * kCounterStride] = 0u;
+    if (threadIdx.x < kNumCounterLines) {
+        pb.counters[threadIdx.x * kCounterStride] = 0u;
+        pb.counters[threadIdx.x * kCounterStride + 1] = 0u;  // kQn's high word
+    }
     __syncthreads();
     if (threadIdx.x == 0) plan_fresh(pb.counters, a);
 }
@@ -119,7 +159,8 @@ __global__ void k_rotate(PathBuffers pb, RenderArgs a) {
     pb.stats[0] += active_count(c);
     pb.stats[1] += c[traced];
     c[kQ] = c[kQn];
-    c[kQn] = 0;
+    c[pb.cur.shadow_count] = c[kQn + 1];
+    c[kQn] = c[kQn + 1] = 0;
     c[traced] = 0;
     for (int x = 0; x < kXcds; x++) {
         c[kFetchExtX + x * kCounterStride] = 0;
@@ -195,7 +236,7 @@ __global__ void k_fill_f64(double *p, size_t n) {
 // A batch renders several (scene, film, parameters) jobs through one path pool
 // and one launch of every kernel per iteration: the pass's samples are the
 // jobs' samples laid end to end (job-major), a path carries its job in the
-// high bits of meta.z (bounce in the low 8), and every per-path lookup reads
+// high bits of rad.w (bounce in the low 8), and every per-path lookup reads
 // the job's scene.  Single-scene kernels (BATCH = false) take the scene as a
 // kernel argument instead, and their job is always 0.
 struct BatchJob {
@@ -258,14 +299,13 @@ __global__ __launch_bounds__(kShadeBlock) void k_regen(DScene s1, const BatchJob
     const uint32_t fresh_n = pb.counters[kFresh];
     const uint32_t sbase = pb.counters[kBase];
     const PathState st = pb.cur;
-    for (uint32_t base = blockIdx.x * kShadeBlock; base < fresh_n; base += gridDim.x * kShadeBlock) {
+    for (uint32_t base = blockIdx.x * blockDim.x; base < fresh_n; base += gridDim.x * blockDim.x) {
         const uint32_t i = base + threadIdx.x;
         const bool fresh = i < fresh_n;
         const uint32_t sidx = sbase + i;
         bool splat = false;
         float4 so = make_float4(0, 0, 0, 0), sd = so, sc = so;
         float4 ro = so, rdir = so, thr = so;
-        uint4 meta = make_uint4(0, 0, 0, 0);
         uint32_t job = 0;
         if (fresh) {
             uint32_t local = sidx, wh = a.wh, first = a.first_sample, seed = a.seed;
@@ -359,15 +399,16 @@ __global__ __launch_bounds__(kShadeBlock) void k_regen(DScene s1, const BatchJob
                 rdir = make_float4(dir.x, dir.y, dir.z, 0.f);
                 thr = make_float4(1.f, 1.f, 1.f, use_mis ? pdfW : 0.f);
             }
-            meta = make_uint4(key, sidx, job << kBounceBits, 0u);
+            ro.w = __uint_as_float(key);
+            rdir.w = __uint_as_float(sidx);
         }
         if (fresh) {
             const uint32_t e = head + i;
             st.ray_o[e] = ro;
             st.ray_d[e] = rdir;
             st.thr[e] = thr;
-            st.rad[e] = make_float4(0.f, 0.f, 0.f, 0.f);
-            st.meta[e] = meta;
+            st.rad[e] = make_float4(0.f, 0.f, 0.f, __uint_as_float(job << kBounceBits));
+            if (a.guided) st.rec[e] = 0u;
         }
         // t = 1 connections join the previous shade kernel's shadow rays
         const uint32_t si = block_append(&pb.counters[pb.next.shadow_count], splat, agg);
@@ -490,7 +531,7 @@ __device__ __forceinline__ void extend_rays(DScene s1, const BatchJob *__restric
                 p = i;
                 const float4 o = pb.cur.ray_o[p], d = pb.cur.ray_d[p];
                 if (BATCH) {
-                    const DScene &sj = jobs[pb.cur.meta[p].z >> kBounceBits].s;
+                    const DScene &sj = jobs[__float_as_uint(pb.cur.rad[p].w) >> kBounceBits].s;
                     geo = Geo{sj.nodes, sj.tris};
                 }
                 trav_begin(ts, setup_ray(xyz(o), xyz(d), kRayEps), INFINITY);
@@ -523,31 +564,32 @@ __device__ __forceinline__ void extend_rays(DScene s1, const BatchJob *__restric
 template <bool BATCH, bool ENV = false>
 __global__ __launch_bounds__(kShadeBlock) void k_shade(DScene s1, const BatchJob *__restrict__ jobs, PathBuffers pb,
                                                        RenderArgs a) {
-    __shared__ uint32_t agg[kWavesPerShadeBlock + 1];
+    __shared__ uint32_t agg[2][kWavesPerShadeBlock + 2];
     const uint32_t n = active_count(pb.counters);
     const PathState cs = pb.cur, ns = pb.next;
-    for (uint32_t base = blockIdx.x * kShadeBlock; base < n; base += gridDim.x * kShadeBlock) {
+    uint32_t flip = 0;
+    for (uint32_t base = blockIdx.x * blockDim.x; base < n; base += gridDim.x * blockDim.x, flip++) {
         const uint32_t i = base + threadIdx.x;
         bool push_shadow = false, cont = false;
         const bool valid = i < n;
         float4 so = make_float4(0, 0, 0, 0), sd = so, sc = so;
         float4 new_o = so, new_d = so, new_thr = so, rad = so;
-        uint4 meta = make_uint4(0, 0, 0, 0);
-        uint32_t job = 0;
+        uint32_t job = 0, key = 0, sidx = 0, bounce = 0;
         if (valid) {
-            meta = cs.meta[i];
+            const float4 ray_d = cs.ray_d[i];
+            const float3 rd = xyz(ray_d);
+            sidx = __float_as_uint(ray_d.w);
             rad = cs.rad[i];
-            job = meta.z >> kBounceBits;
+            bounce = __float_as_uint(rad.w) & kBounceMask;
+            job = __float_as_uint(rad.w) >> kBounceBits;
             const DScene &s = BATCH ? jobs[job].s : s1;
             const int N = BATCH ? jobs[job].N : a.N;
             const int use_mis = BATCH ? jobs[job].use_mis : a.use_mis;
-            const uint32_t bounce = meta.z & kBounceMask;
             const int cNum = int(bounce) + 2;  // camera is vertex 1
             const uint2 h = pb.hit[i];
             if (ENV && h.x == kInvalid && s.env_select > 0.f) {
                 // a miss is the envmap vertex (scene.h:82-88): an emitter hit with Le1 = 1,
                 // Le0 = the lookup, and area pdfs equal to the solid-angle ones
-                const float3 rd = xyz(cs.ray_d[i]);
                 const float4 thr = cs.thr[i];
                 float mis = a.nee ? 0.f : 1.f;
                 if (use_mis) {
@@ -561,7 +603,9 @@ __global__ __launch_bounds__(kShadeBlock) void k_shade(DScene s1, const BatchJob
             }
             if (h.x != kInvalid) {
                 const float t = __uint_as_float(h.y);
-                const float3 ro = xyz(cs.ray_o[i]), rd = xyz(cs.ray_d[i]);
+                const float4 ray_o = cs.ray_o[i];
+                const float3 ro = xyz(ray_o);
+                key = __float_as_uint(ray_o.w);
                 const float4 v0 = s.tris[3 * size_t(h.x) + 0];
                 const float4 v1 = s.tris[3 * size_t(h.x) + 1];
                 const float4 v2 = s.tris[3 * size_t(h.x) + 2];
@@ -570,7 +614,6 @@ __global__ __launch_bounds__(kShadeBlock) void k_shade(DScene s1, const BatchJob
                 const int2 gi = s.geom_info[__float_as_uint(v1.w)];
                 const float4 thr = cs.thr[i];
                 const float3 T = xyz(thr);
-                const uint32_t key = meta.x;
                 if (gi.y >= 0) {
                     // emitter hit: MIS against light sampling (pathnextevent.h:128-146);
                     // without NEE it is the only estimate (weight 1, primitivepath.h:52-56)
@@ -642,28 +685,28 @@ __global__ __launch_bounds__(kShadeBlock) void k_shade(DScene s1, const BatchJob
                     const float3 w = bsdf_sample(m, wi, u01(key, dim), u01(key, dim + 1), wo, pdf);
                     if (!is_black(w)) {
                         const float3 nd = to_world(f, wo);
-                        new_o = make_float4(pos.x, pos.y, pos.z, 0.f);
-                        new_d = make_float4(nd.x, nd.y, nd.z, 0.f);
+                        new_o = make_float4(pos.x, pos.y, pos.z, __uint_as_float(key));
+                        new_d = make_float4(nd.x, nd.y, nd.z, __uint_as_float(sidx));
                         new_thr = make_float4(w.x * T.x, w.y * T.y, w.z * T.z, use_mis ? pdf : 0.f);
                         cont = true;
                     }
                 }
             }
         }
-        const uint32_t qi = block_append(&pb.counters[kQn], cont, agg);
+        const Append2 at = block_append2(&pb.counters[kQn], cont, push_shadow, agg, flip);
+        const uint32_t qi = at.a, si = at.b;
         if (cont) {
             ns.ray_o[qi] = new_o;
             ns.ray_d[qi] = new_d;
             ns.thr[qi] = new_thr;
+            rad.w = __uint_as_float(__float_as_uint(rad.w) + 1u);  // the next bounce
             ns.rad[qi] = rad;
-            ns.meta[qi] = make_uint4(meta.x, meta.y, meta.z + 1, 0u);
         } else if (valid) {
-            pb.sample_rad[meta.y] = rad;
+            pb.sample_rad[sidx] = rad;
         }
-        const uint32_t target = cont ? (kToNextPath | qi) : (kToSample | meta.y);
+        const uint32_t target = cont ? (kToNextPath | qi) : (kToSample | sidx);
         sd.w = __uint_as_float(target);
         sc.w = __uint_as_float(job);
-        const uint32_t si = block_append(&pb.counters[pb.cur.shadow_count], push_shadow, agg);
         if (push_shadow) {
             pb.sh_o[si] = so;
             pb.sh_d[si] = sd;
@@ -682,26 +725,29 @@ __global__ __launch_bounds__(kShadeBlock) void k_shade(DScene s1, const BatchJob
 // An emitter hit ends the subpath.  No medium (the reference's sampler here
 // is not volumetric).
 __global__ __launch_bounds__(kShadeBlock) void k_shade_light(DScene s, PathBuffers pb, RenderArgs a) {
-    __shared__ uint32_t agg[kWavesPerShadeBlock + 1];
+    __shared__ uint32_t agg[2][kWavesPerShadeBlock + 2];
     const uint32_t n = active_count(pb.counters);
     const PathState cs = pb.cur, ns = pb.next;
     const DCamera &cam = s.cam;
-    for (uint32_t base = blockIdx.x * kShadeBlock; base < n; base += gridDim.x * kShadeBlock) {
+    uint32_t flip = 0;
+    for (uint32_t base = blockIdx.x * blockDim.x; base < n; base += gridDim.x * blockDim.x, flip++) {
         const uint32_t i = base + threadIdx.x;
         bool push_shadow = false, cont = false;
         const bool valid = i < n;
         float4 so = make_float4(0, 0, 0, 0), sd = so, sc = so;
         float4 new_o = so, new_d = so, new_thr = so, rad = so;
-        uint4 meta = make_uint4(0, 0, 0, 0);
+        uint32_t sidx = 0;
         if (valid) {
-            meta = cs.meta[i];
+            const float4 ray_d = cs.ray_d[i];
+            sidx = __float_as_uint(ray_d.w);
             rad = cs.rad[i];
-            const uint32_t bounce = meta.z & kBounceMask;
+            const uint32_t bounce = __float_as_uint(rad.w) & kBounceMask;
             const int k = int(bounce) + 2;  // vertex of the light subpath
             const uint2 h = pb.hit[i];
             if (h.x != kInvalid && k <= a.N - 1) {
                 const float t = __uint_as_float(h.y);
-                const float3 ro = xyz(cs.ray_o[i]), rd = xyz(cs.ray_d[i]);
+                const float4 ray_o = cs.ray_o[i];
+                const float3 ro = xyz(ray_o), rd = xyz(ray_d);
                 const float4 v0 = s.tris[3 * size_t(h.x) + 0];
                 const float4 v1 = s.tris[3 * size_t(h.x) + 1];
                 const float4 v2 = s.tris[3 * size_t(h.x) + 2];
@@ -710,7 +756,7 @@ __global__ __launch_bounds__(kShadeBlock) void k_shade_light(DScene s, PathBuffe
                     const float3 pos = ro + rd * t;
                     const float3 ng = normalize3(cross3(xyz(v1) - xyz(v0), xyz(v2) - xyz(v0)));
                     const float3 T = xyz(cs.thr[i]);
-                    const uint32_t key = meta.x;
+                    const uint32_t key = __float_as_uint(ray_o.w);
                     const DMat m = s.mats[gi.x];
                     const Frame f = make_frame(ng);
                     const float3 wi = to_local(f, -rd);
@@ -742,8 +788,8 @@ __global__ __launch_bounds__(kShadeBlock) void k_shade_light(DScene s, PathBuffe
                         const float3 w = bsdf_sample(m, wi, u01(key, dim), u01(key, dim + 1), wo, pdf);
                         if (!is_black(w)) {
                             const float3 nd = to_world(f, wo);
-                            new_o = make_float4(pos.x, pos.y, pos.z, 0.f);
-                            new_d = make_float4(nd.x, nd.y, nd.z, 0.f);
+                            new_o = make_float4(pos.x, pos.y, pos.z, ray_o.w);
+                            new_d = make_float4(nd.x, nd.y, nd.z, ray_d.w);
                             new_thr = make_float4(w.x * T.x, w.y * T.y, w.z * T.z, 0.f);
                             cont = true;
                         }
@@ -751,17 +797,17 @@ __global__ __launch_bounds__(kShadeBlock) void k_shade_light(DScene s, PathBuffe
                 }
             }
         }
-        const uint32_t qi = block_append(&pb.counters[kQn], cont, agg);
+        const Append2 at = block_append2(&pb.counters[kQn], cont, push_shadow, agg, flip);
+        const uint32_t qi = at.a, si = at.b;
         if (cont) {
             ns.ray_o[qi] = new_o;
             ns.ray_d[qi] = new_d;
             ns.thr[qi] = new_thr;
+            rad.w = __uint_as_float(__float_as_uint(rad.w) + 1u);  // the next bounce
             ns.rad[qi] = rad;
-            ns.meta[qi] = make_uint4(meta.x, meta.y, meta.z + 1, 0u);
         } else if (valid) {
-            pb.sample_rad[meta.y] = rad;
+            pb.sample_rad[sidx] = rad;
         }
-        const uint32_t si = block_append(&pb.counters[pb.cur.shadow_count], push_shadow, agg);
         if (push_shadow) {
             pb.sh_o[si] = so;
             pb.sh_d[si] = sd;
@@ -852,17 +898,19 @@ __global__ __launch_bounds__(kInferBlock) __attribute__((amdgpu_waves_per_eu(WR_
         bool need = false, med = false;
         float3 pos = f3(0.f, 0.f, 0.f), ng = f3(0.f, 1.f, 0.f), nf = ng, rd = f3(0.f, 0.f, 1.f);
         int mat = 0;
-        uint4 meta = make_uint4(0, 0, 0, 0);
+        uint32_t key = 0, bounce = 0;
         if (i < n) {
             const uint2 h = hit[i];
-            meta = cs.meta[i];
-            if (int(meta.z) + 2 != N && meta.z < max_bounce) {
+            bounce = __float_as_uint(cs.rad[i].w);
+            if (int(bounce) + 2 != N && bounce < max_bounce) {
+                const float4 ray_o = cs.ray_o[i];
+                key = __float_as_uint(ray_o.w);
                 float tf = 0.f;
-                med = MEDIUM && free_flight(s.med, meta.x, meta.z, h.x != kInvalid ? __uint_as_float(h.y) : INFINITY, tf);
+                med = MEDIUM && free_flight(s.med, key, bounce, h.x != kInvalid ? __uint_as_float(h.y) : INFINITY, tf);
                 if (med) {
                     need = true;
                     rd = xyz(cs.ray_d[i]);
-                    pos = xyz(cs.ray_o[i]) + rd * tf;
+                    pos = xyz(ray_o) + rd * tf;
                     nf = -rd;  // no surface: the incoming direction stands in for the normal
                 } else if (h.x != kInvalid) {
                     const float4 v0 = s.tris[3 * size_t(h.x) + 0];
@@ -873,7 +921,7 @@ __global__ __launch_bounds__(kInferBlock) __attribute__((amdgpu_waves_per_eu(WR_
                         need = true;
                         mat = gi.x;
                         rd = xyz(cs.ray_d[i]);
-                        pos = xyz(cs.ray_o[i]) + rd * __uint_as_float(h.y);
+                        pos = xyz(ray_o) + rd * __uint_as_float(h.y);
                         ng = normalize3(cross3(xyz(v1) - xyz(v0), xyz(v2) - xyz(v0)));
                         nf = dot3(ng, rd) > 0.f ? -ng : ng;
                     }
@@ -887,10 +935,9 @@ __global__ __launch_bounds__(kInferBlock) __attribute__((amdgpu_waves_per_eu(WR_
             if (need) {
                 float wl[guide::kLobes];
                 guide::decode(L, wl);
-                const uint32_t key = meta.x;
                 const LightSample l = sample_light(s, u01(key, kDimLight), u01(key, kDimLight + 1), key);
                 const float3 dl = normalize3(l.pos - pos);
-                const uint32_t dim = kDimBounce0 + kDimsPerBounce * meta.z + kBdBsdf;
+                const uint32_t dim = kDimBounce0 + kDimsPerBounce * bounce + kBdBsdf;
                 const float u0 = u01(key, dim), u1 = u01(key, dim + 1), us = u01(key, dim + 2);
                 float alpha = frac;
                 DMat m{};
@@ -930,34 +977,38 @@ __global__ __launch_bounds__(kInferBlock) __attribute__((amdgpu_waves_per_eu(WR_
 
 template <bool GUIDED, bool MEDIUM>
 __global__ __launch_bounds__(kShadeBlock) void k_shade_ext(DScene s, PathBuffers pb, RenderArgs a, guide::Shade g) {
-    __shared__ uint32_t agg[kWavesPerShadeBlock + 1];
+    __shared__ uint32_t agg[2][kWavesPerShadeBlock + 2];
+    __shared__ uint32_t rec_agg[kWavesPerShadeBlock + 1];
     const uint32_t n = active_count(pb.counters);
     const PathState cs = pb.cur, ns = pb.next;
     const float3 zero = f3(0.f, 0.f, 0.f);
-    for (uint32_t base = blockIdx.x * kShadeBlock; base < n; base += gridDim.x * kShadeBlock) {
+    uint32_t flip = 0;
+    for (uint32_t base = blockIdx.x * blockDim.x; base < n; base += gridDim.x * blockDim.x, flip++) {
         const uint32_t i = base + threadIdx.x;
         const bool valid = i < n;
         // ---- the vertex
-        uint4 meta = make_uint4(0, 0, 0, 0);
+        float4 ray_o = make_float4(0, 0, 0, 0), ray_d = ray_o, rad = ray_o;
         uint2 h = make_uint2(kInvalid, 0u);
         float3 pos = zero, ng = f3(0.f, 1.f, 0.f), rd = f3(0.f, 0.f, 1.f);
         int2 gi = make_int2(0, -1);
         bool in_medium = false;
         float seg_t = 0.f;
         if (valid) {
-            meta = cs.meta[i];
+            ray_o = cs.ray_o[i];
+            ray_d = cs.ray_d[i];
+            rad = cs.rad[i];
             h = pb.hit[i];
-            rd = xyz(cs.ray_d[i]);
+            rd = xyz(ray_d);
             seg_t = h.x != kInvalid ? __uint_as_float(h.y) : INFINITY;
             if (MEDIUM) {
                 float tf = 0.f;
-                in_medium = free_flight(s.med, meta.x, meta.z, seg_t, tf);
+                in_medium = free_flight(s.med, __float_as_uint(ray_o.w), __float_as_uint(rad.w), seg_t, tf);
                 if (in_medium) seg_t = tf;
             }
             if (in_medium) {
-                pos = xyz(cs.ray_o[i]) + rd * seg_t;
+                pos = xyz(ray_o) + rd * seg_t;
             } else if (h.x != kInvalid) {
-                pos = xyz(cs.ray_o[i]) + rd * seg_t;
+                pos = xyz(ray_o) + rd * seg_t;
                 const float4 v0 = s.tris[3 * size_t(h.x) + 0];
                 const float4 v1 = s.tris[3 * size_t(h.x) + 1];
                 const float4 v2 = s.tris[3 * size_t(h.x) + 2];
@@ -966,11 +1017,12 @@ __global__ __launch_bounds__(kShadeBlock) void k_shade_ext(DScene s, PathBuffers
             }
         }
         const bool hit_vertex = valid && !in_medium && h.x != kInvalid;
-        const bool last = int(meta.z) + 2 == a.N;
+        const uint32_t key = __float_as_uint(ray_o.w), sidx = __float_as_uint(ray_d.w), bounce = __float_as_uint(rad.w);
+        const bool last = int(bounce) + 2 == a.N;
         const bool surf = hit_vertex && gi.y < 0 && !last;
         const bool med = valid && in_medium && !last;
         const float3 nf = in_medium ? -rd : (dot3(ng, rd) > 0.f ? -ng : ng);  // faces the incoming ray
-        const bool need = GUIDED && (surf || med) && g.alpha > 0.f && meta.z < g.max_bounce;
+        const bool need = GUIDED && (surf || med) && g.alpha > 0.f && bounce < g.max_bounce;
         float4 gdir = make_float4(0.f, 0.f, 0.f, 0.f);  // k_guide_infer's direction and q there
         float q_nee = 0.f;
         if (GUIDED && need) {
@@ -980,14 +1032,15 @@ __global__ __launch_bounds__(kShadeBlock) void k_shade_ext(DScene s, PathBuffers
         // ---- shading
         bool push_shadow = false, cont = false;
         float4 so = make_float4(0, 0, 0, 0), sd = so, sc = so;
-        float4 new_o = so, new_d = so, new_thr = so, rad = so;
+        float4 new_o = so, new_d = so, new_thr = so;
         float3 wdir = zero, T = zero;
-        const uint32_t key = meta.x, bounce = meta.z;
         float prev_pdfw = 0.f;
         if (valid) {
-            rad = cs.rad[i];
-            // radiance before this vertex closes the record of the previous one
-            if (GUIDED && meta.w) g.rec.rad[meta.w - 1] = rad;
+            if (GUIDED) {
+                // radiance before this vertex closes the record of the previous one
+                const uint32_t prev = cs.rec[i];
+                if (prev) g.rec.rad[prev - 1] = rad;
+            }
             const float4 thr = cs.thr[i];
             prev_pdfw = thr.w;
             T = xyz(thr);
@@ -1096,8 +1149,8 @@ __global__ __launch_bounds__(kShadeBlock) void k_shade_ext(DScene s, PathBuffers
             }
             if (!is_black(w) && pdf > 0.f) {
                 wdir = nd;
-                new_o = make_float4(pos.x, pos.y, pos.z, 0.f);
-                new_d = make_float4(nd.x, nd.y, nd.z, 0.f);
+                new_o = make_float4(pos.x, pos.y, pos.z, ray_o.w);
+                new_d = make_float4(nd.x, nd.y, nd.z, ray_d.w);
                 new_thr = make_float4(w.x * T.x, w.y * T.y, w.z * T.z, a.use_mis ? pdf : 0.f);
                 cont = true;
             }
@@ -1105,9 +1158,9 @@ __global__ __launch_bounds__(kShadeBlock) void k_shade_ext(DScene s, PathBuffers
         uint32_t rec_id = 0;
         if (GUIDED && g.collect) {
             const bool want = cont && bounce < g.max_bounce && float(mix32(key ^ 0x68bc21ebu) >> 8) * 0x1p-24f < g.record_prob;
-            const uint32_t r = block_append(g.rec.count, want, agg);
+            const uint32_t r = block_append(g.rec.count, want, rec_agg);
             if (want && r < g.rec.capacity) {
-                g.rec.pos[r] = make_float4(pos.x, pos.y, pos.z, __uint_as_float(meta.y));
+                g.rec.pos[r] = make_float4(pos.x, pos.y, pos.z, ray_d.w);
                 g.rec.nrm[r] = make_float4(nf.x, nf.y, nf.z, 0.f);
                 g.rec.wo[r] = make_float4(-rd.x, -rd.y, -rd.z, 0.f);
                 g.rec.wi[r] = make_float4(wdir.x, wdir.y, wdir.z, 0.f);
@@ -1116,19 +1169,20 @@ __global__ __launch_bounds__(kShadeBlock) void k_shade_ext(DScene s, PathBuffers
                 rec_id = r + 1;
             }
         }
-        const uint32_t qi = block_append(&pb.counters[kQn], cont, agg);
+        const Append2 at = block_append2(&pb.counters[kQn], cont, push_shadow, agg, flip);
+        const uint32_t qi = at.a, si = at.b;
         if (cont) {
             ns.ray_o[qi] = new_o;
             ns.ray_d[qi] = new_d;
             ns.thr[qi] = new_thr;
+            rad.w = __uint_as_float(bounce + 1u);
             ns.rad[qi] = rad;
-            ns.meta[qi] = make_uint4(meta.x, meta.y, meta.z + 1, rec_id);
+            if (GUIDED) ns.rec[qi] = rec_id;
         } else if (valid) {
-            pb.sample_rad[meta.y] = rad;
+            pb.sample_rad[sidx] = rad;
         }
-        const uint32_t target = cont ? (kToNextPath | qi) : (kToSample | meta.y);
+        const uint32_t target = cont ? (kToNextPath | qi) : (kToSample | sidx);
         sd.w = __uint_as_float(target);
-        const uint32_t si = block_append(&pb.counters[pb.cur.shadow_count], push_shadow, agg);
         if (push_shadow) {
             pb.sh_o[si] = so;
             pb.sh_d[si] = sd;
@@ -2275,15 +2329,15 @@ int wr_film_image(wr_film *f, double base_div, double splat_div, double *rgb) {
     return WR_OK;
 }
 
-// Path pool: two queue-ordered states of 16*5 bytes per path (ray_o, ray_d,
-// thr, rad, meta), the hit records (8 B), two shadow entries (2 * 48 B), and
+// Path pool: two queue-ordered states of 16*4 + 4 bytes per path (ray_o, ray_d,
+// thr, rad, rec), the hit records (8 B), two shadow entries (2 * 48 B), and
 // the per-sample radiance of a pass (16 B per sample).
 // Byte layout of a path pool of `cap` paths and `samples` per-sample slots
 // (every array 256-byte aligned): the state pair, hits, per-sample radiance,
 // shadow queue (2 entries per path), counters (one 256-byte line each), stats.
 constexpr size_t align256(size_t b) { return (b + 255) / 256 * 256; }
 constexpr size_t pool_bytes(size_t cap, size_t samples) {
-    return 10 * align256(16 * cap) + align256(8 * cap) + align256(16 * samples) + 3 * align256(32 * cap) +
+    return 8 * align256(16 * cap) + 2 * align256(4 * cap) + align256(8 * cap) + align256(16 * samples) + 3 * align256(32 * cap) +
            align256(4 * kCounterStride * kNumCounterLines) + align256(64);
 }
 // Points pb's arrays into the pool at `base`; returns the bytes used (pool_bytes).
@@ -2297,7 +2351,7 @@ static size_t pool_layout(char *base, uint32_t cap, uint32_t samples, PathBuffer
         st->ray_d = reinterpret_cast<float4 *>(take(16 * c));
         st->thr = reinterpret_cast<float4 *>(take(16 * c));
         st->rad = reinterpret_cast<float4 *>(take(16 * c));
-        st->meta = reinterpret_cast<uint4 *>(take(16 * c));
+        st->rec = reinterpret_cast<uint32_t *>(take(4 * c));
     }
     pb->hit = reinterpret_cast<uint2 *>(take(8 * c));
     pb->sample_rad = reinterpret_cast<float4 *>(take(16 * size_t(samples)));
@@ -2448,6 +2502,15 @@ int wr_render_params_validate(const wr_render_params *p) {
     return WR_OK;
 }
 
+// Threads per block of the shade and regenerate kernels for a pool of `paths`:
+// kShadeBlock, which halves the appends' atomics against 256, down to one wave
+// where that spreads a small pool over more of the CUs.
+static int shade_block(const wr_device *d, uint64_t paths) {
+    int block = kShadeBlock;
+    while (block > 64 && paths < uint64_t(d->n_cu) * block * 2) block /= 2;
+    return block;
+}
+
 // Estimators of the frame loop.
 enum Estimator { kEstNee, kEstPrimitive, kEstLight };
 // A path pool and traversal spill region that the caller already holds (the
@@ -2552,7 +2615,8 @@ static int render_impl(wr_scene *s, wr_film *f, const wr_render_params *prm, wr_
     };
     auto begin = [&](int kind) { if (prof) marks.push_back({kind, ev_record()}); };
     auto end = [&]() { if (prof) ev_record(); };
-    const int g_regen = std::max(1, std::min<int>((P + kShadeBlock - 1) / kShadeBlock, s->dev->n_cu * s->dev->occ_generate));
+    const int bs = shade_block(s->dev, P);
+    const int g_regen = std::max(1, std::min<int>((P + bs - 1) / bs, s->dev->n_cu * s->dev->occ_generate * (kShadeBlock / bs)));
     // shading kernel: plain, or extended for guiding and/or a medium
     // the light tracer's sampler is not volumetric (lightsplatting.h:34): it sees vacuum
     DScene ds = s->ds;
@@ -2564,8 +2628,8 @@ static int render_impl(wr_scene *s, wr_film *f, const wr_render_params *prm, wr_
     if (g && medium) shade_fn = reinterpret_cast<const void *>(&k_shade_ext<true, true>);
     else if (g) shade_fn = reinterpret_cast<const void *>(&k_shade_ext<true, false>);
     else if (medium) shade_fn = reinterpret_cast<const void *>(&k_shade_ext<false, true>);
-    const int g_shade = std::max(1, std::min<int>((P + kShadeBlock - 1) / kShadeBlock,
-                                                  s->dev->n_cu * occupancy(s->dev, shade_fn, kShadeBlock)));
+    const int g_shade = std::max(1, std::min<int>((P + bs - 1) / bs, s->dev->n_cu * occupancy(s->dev, shade_fn, kShadeBlock) *
+                                                                         (kShadeBlock / bs)));
     int pass = 0;
     const bool fp8 = g && gp->fp8_inference != 0;
     const void *infer_fn = medium ? (fp8 ? reinterpret_cast<const void *>(&k_guide_infer<true, true>)
@@ -2589,6 +2653,7 @@ static int render_impl(wr_scene *s, wr_film *f, const wr_render_params *prm, wr_
         a.N = N;
         a.use_mis = est == kEstNee && prm->use_mis ? 1 : 0;
         a.nee = est == kEstNee ? 1 : 0;
+        a.guided = g ? 1 : 0;
         a.light = est == kEstLight ? 1 : 0;
         guide::Shade gs{};
         float record_prob = 0.f;
@@ -2614,8 +2679,8 @@ static int render_impl(wr_scene *s, wr_film *f, const wr_render_params *prm, wr_
         const uint64_t max_iters = (uint64_t(a.total) / P + 2) * uint64_t(N + 1) + 64;
         auto iteration = [&](const PathBuffers &q) {
             begin(3);
-            if (env) k_regen<false, true><<<g_regen, kShadeBlock, 0, s->stream>>>(ds, nullptr, 0, q, a);
-            else k_regen<false><<<g_regen, kShadeBlock, 0, s->stream>>>(ds, nullptr, 0, q, a);
+            if (env) k_regen<false, true><<<g_regen, bs, 0, s->stream>>>(ds, nullptr, 0, q, a);
+            else k_regen<false><<<g_regen, bs, 0, s->stream>>>(ds, nullptr, 0, q, a);
             end();
             begin(0);
             if (count) k_trace_bounce<true, false><<<g_trav, kBlock, 0, s->stream>>>(ds, nullptr, q, spill, tune);
@@ -2636,12 +2701,12 @@ static int render_impl(wr_scene *s, wr_film *f, const wr_render_params *prm, wr_
                     k_guide_infer<false, false><<<g_infer, kInferBlock, 0, s->stream>>>(ds, q.cur, q.hit, q.counters, N,
                                                                                         net, gs.alpha, gs.max_bounce, gs.draw);
             }
-            if (g && medium) k_shade_ext<true, true><<<g_shade, kShadeBlock, 0, s->stream>>>(ds, q, a, gs);
-            else if (g) k_shade_ext<true, false><<<g_shade, kShadeBlock, 0, s->stream>>>(ds, q, a, gs);
-            else if (medium) k_shade_ext<false, true><<<g_shade, kShadeBlock, 0, s->stream>>>(ds, q, a, gs);
-            else if (est == kEstLight) k_shade_light<<<g_shade, kShadeBlock, 0, s->stream>>>(ds, q, a);
-            else if (env) k_shade<false, true><<<g_shade, kShadeBlock, 0, s->stream>>>(ds, nullptr, q, a);
-            else k_shade<false><<<g_shade, kShadeBlock, 0, s->stream>>>(ds, nullptr, q, a);
+            if (g && medium) k_shade_ext<true, true><<<g_shade, bs, 0, s->stream>>>(ds, q, a, gs);
+            else if (g) k_shade_ext<true, false><<<g_shade, bs, 0, s->stream>>>(ds, q, a, gs);
+            else if (medium) k_shade_ext<false, true><<<g_shade, bs, 0, s->stream>>>(ds, q, a, gs);
+            else if (est == kEstLight) k_shade_light<<<g_shade, bs, 0, s->stream>>>(ds, q, a);
+            else if (env) k_shade<false, true><<<g_shade, bs, 0, s->stream>>>(ds, nullptr, q, a);
+            else k_shade<false><<<g_shade, bs, 0, s->stream>>>(ds, nullptr, q, a);
             end();
             k_rotate<<<1, 1, 0, s->stream>>>(q, a);
         };
@@ -2700,7 +2765,7 @@ int wr_render_nee(wr_scene *s, wr_film *f, const wr_render_params *prm, wr_rende
 // wr_render_nee_noalloc renders through a fixed region of device memory that
 // the library reserves once per GPU instead of the scene's lazily grown path
 // pool: a pool of 2^17 paths with 2^20 per-sample slots (passes of at most
-// 2^20 samples) and the traversal spill of 1024 blocks -- 77 MiB, held by each
+// 2^20 samples) and the traversal spill of 1024 blocks -- 74 MiB, held by each
 // GPU the library runs on until the process ends.  The region is a file-scope
 // device array; its device address on each GPU comes from hipGetSymbolAddress
 // at wr_device_create (the array's name in host code is not a device address).
@@ -2913,15 +2978,16 @@ int wr_render_batch(const wr_batch_job *jobs, uint32_t n_jobs, const wr_render_p
     auto begin = [&](int kind) { if (prof) marks.push_back({kind, ev_record()}); };
     auto end = [&]() { if (prof) ev_record(); };
     wr_device *dev = s0->dev;
-    auto grid = [&](const void *fn, int block) {
-        return std::max(1, std::min<int>((P + block - 1) / block, dev->n_cu * occupancy(dev, fn, block)));
+    const int bs = shade_block(dev, P);
+    auto grid = [&](const void *fn) {
+        return std::max(1, std::min<int>((P + bs - 1) / bs, dev->n_cu * occupancy(dev, fn, kShadeBlock) * (kShadeBlock / bs)));
     };
     bool env = false;
     for (uint32_t j = 0; j < n_jobs; j++) env = env || jobs[j].scene->ds.env_select > 0.f;
     const int g_regen = grid(env ? reinterpret_cast<const void *>(&k_regen<true, true>)
-                                 : reinterpret_cast<const void *>(&k_regen<true>), kShadeBlock);
+                                 : reinterpret_cast<const void *>(&k_regen<true>));
     const int g_shade = grid(env ? reinterpret_cast<const void *>(&k_shade<true, true>)
-                                 : reinterpret_cast<const void *>(&k_shade<true>), kShadeBlock);
+                                 : reinterpret_cast<const void *>(&k_shade<true>));
     const int g_trav =
         trav_grid(s0, 2 * P, occupancy(dev, reinterpret_cast<const void *>(&k_trace_bounce<false, true>), kBlock));
     std::vector<BatchJob> tab;
@@ -2966,16 +3032,16 @@ int wr_render_batch(const wr_batch_job *jobs, uint32_t n_jobs, const wr_render_p
         const uint64_t max_iters = (uint64_t(a.total) / P + 2) * uint64_t(maxN + 1) + 64;
         auto iteration = [&](const PathBuffers &q) {
             begin(3);
-            if (env) k_regen<true, true><<<g_regen, kShadeBlock, 0, s0->stream>>>(s0->ds, d_tab, nt, q, a);
-            else k_regen<true><<<g_regen, kShadeBlock, 0, s0->stream>>>(s0->ds, d_tab, nt, q, a);
+            if (env) k_regen<true, true><<<g_regen, bs, 0, s0->stream>>>(s0->ds, d_tab, nt, q, a);
+            else k_regen<true><<<g_regen, bs, 0, s0->stream>>>(s0->ds, d_tab, nt, q, a);
             end();
             begin(0);
             if (count) k_trace_bounce<true, true><<<g_trav, kBlock, 0, s0->stream>>>(s0->ds, d_tab, q, s0->d_spill, tune);
             else k_trace_bounce<false, true><<<g_trav, kBlock, 0, s0->stream>>>(s0->ds, d_tab, q, s0->d_spill, tune);
             end();
             begin(2);
-            if (env) k_shade<true, true><<<g_shade, kShadeBlock, 0, s0->stream>>>(s0->ds, d_tab, q, a);
-            else k_shade<true><<<g_shade, kShadeBlock, 0, s0->stream>>>(s0->ds, d_tab, q, a);
+            if (env) k_shade<true, true><<<g_shade, bs, 0, s0->stream>>>(s0->ds, d_tab, q, a);
+            else k_shade<true><<<g_shade, bs, 0, s0->stream>>>(s0->ds, d_tab, q, a);
             end();
             k_rotate<<<1, 1, 0, s0->stream>>>(q, a);
         };
