@@ -79,7 +79,8 @@ enum Counter : int {
     kQ = 0 * kCounterStride,         // continuing paths at the head of the current state
     kFresh = 1 * kCounterStride,     // new samples started behind them this iteration
     kQn = 2 * kCounterStride,        // paths continuing into the next state
-    // line 3 is spare
+    kTicket = 3 * kCounterStride,    // blocks of the shade kernel that have finished (the last one ends the
+                                     // iteration); word 1: iterations ended in this pass
     // Shadow queue: the shade kernel of iteration i appends its shadow rays,
     // then the regeneration of iteration i + 1 its t = 1 connections, and the
     // traversal launch of iteration i + 1 traces them beside that iteration's
@@ -105,6 +106,9 @@ struct RenderArgs {
     int use_mis;
     int nee;                  // 1: PathNeeRenderer (NEE, t = 1 splats); 0: PrimitivePathRenderer (BSDF sampling only)
     int guided;               // 1: entries carry a training record (PathState::rec)
+    uint32_t tag;             // pass tag of the progress word
+    unsigned long long *progress;  // pinned host word (null: the host polls the counters): tag << 32 | iterations
+                                   // ended << 1 | drained, written at the end of each iteration
     int light;                // 1: LightSplattingRenderer (light subpaths connected to the camera)
 };
 
@@ -153,7 +157,8 @@ struct wr_scene {
     PathBuffers pb{};
     uint32_t capacity = 0, sample_capacity = 0;
     void *pool = nullptr;
-    uint32_t *h_counters = nullptr;  // pinned host copy of the pool counters
+    uint32_t *h_counters = nullptr;  // pinned host copy of the pool counters; the progress word behind it
+    uint32_t pass_tag = 0;           // passes started
     hipEvent_t ev[2] = {nullptr, nullptr};
 };
 
