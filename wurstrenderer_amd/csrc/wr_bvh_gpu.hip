@@ -126,6 +126,44 @@ __global__ __launch_bounds__(kBB) void k_centroid_final(const float *partial, in
     if (threadIdx.x < 6) cbox[threadIdx.x] = red[threadIdx.x][0];
 }
 
+// ---------------------------------------------------------------- mesh checks
+// The array checks of a scene description (finite vertices, triangle indices and
+// geometries in range, geometries in order) over the uploaded mesh, and the
+// per-block bounds of its vertices -> partial[6 * block].  As host loops these
+// took 2.5 ms of a 1.31M-triangle scene's creation.
+__global__ __launch_bounds__(kBB) void k_check_mesh(const float *verts, uint32_t n_verts, const uint32_t *tris,
+                                                    const uint32_t *tri_geom, uint32_t n, uint32_t n_geoms,
+                                                    float *partial, uint32_t *invalid) {
+    __shared__ float red[6][kBB];
+    float v[6] = {INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY};
+    bool bad = false;
+    const size_t step = size_t(gridDim.x) * kBB, first = size_t(blockIdx.x) * kBB + threadIdx.x;
+    for (size_t i = first; i < n_verts; i += step)
+        for (int k = 0; k < 3; k++) {
+            const float x = verts[3 * i + k];
+            bad |= !(fabsf(x) <= FLT_MAX);
+            v[k] = fminf(v[k], x);
+            v[3 + k] = fmaxf(v[3 + k], x);
+        }
+    for (size_t i = first; i < 3 * size_t(n); i += step) bad |= tris[i] >= n_verts;
+    for (size_t i = first; i < n; i += step) {
+        const uint32_t g = tri_geom[i];
+        bad |= g >= n_geoms || (i > 0 && tri_geom[i - 1] > g);
+    }
+    if (bad) atomicOr(invalid, 1u);
+    for (int k = 0; k < 6; k++) red[k][threadIdx.x] = v[k];
+    __syncthreads();
+    for (int s = kBB / 2; s > 0; s >>= 1) {
+        if ((int)threadIdx.x < s)
+            for (int k = 0; k < 3; k++) {
+                red[k][threadIdx.x] = fminf(red[k][threadIdx.x], red[k][threadIdx.x + s]);
+                red[3 + k][threadIdx.x] = fmaxf(red[3 + k][threadIdx.x], red[3 + k][threadIdx.x + s]);
+            }
+        __syncthreads();
+    }
+    if (threadIdx.x < 6) partial[6 * blockIdx.x + threadIdx.x] = red[threadIdx.x][0];
+}
+
 // ---------------------------------------------------------------- Morton codes
 // 21 bits -> every third bit of 63.
 __device__ __forceinline__ uint64_t spread21(uint32_t v) {
@@ -185,9 +223,29 @@ __device__ __forceinline__ uint32_t pair_hash(uint32_t lo, uint32_t hi, uint32_t
     return uint32_t(x);
 }
 
-// nearest[i]: the cluster in [i - R, i + R] whose union with cluster i has the
-// smallest surface area; equal areas go to the higher pair hash, then to the
-// lower index.
+// The cluster in [i - R, i + R] of m whose union with cluster i has the smallest
+// surface area; equal areas go to the higher pair hash, then to the lower
+// index.  lo[k] and hi[k] are the boxes of cluster i + k.
+__device__ __forceinline__ uint32_t nearest_of(int64_t i, int64_t m, int R, uint32_t seed, const float4 *lo_at, const float4 *hi_at) {
+    const float3 alo = make_float3(lo_at[0].x, lo_at[0].y, lo_at[0].z), ahi = make_float3(hi_at[0].x, hi_at[0].y, hi_at[0].z);
+    float best = INFINITY;
+    uint32_t bh_best = 0;
+    int64_t bj = -1;
+    for (int o = -R; o <= R; o++) {  // ascending j: on a full tie the first (lower) j stays
+        const int64_t j = i + o;
+        if (o == 0 || j < 0 || j >= m) continue;
+        const float4 bl = lo_at[o], bh = hi_at[o];
+        const float3 lo = make_float3(fminf(alo.x, bl.x), fminf(alo.y, bl.y), fminf(alo.z, bl.z));
+        const float3 hi = make_float3(fmaxf(ahi.x, bh.x), fmaxf(ahi.y, bh.y), fmaxf(ahi.z, bh.z));
+        const float a = half_area(lo, hi);
+        if (a > best) continue;
+        const uint32_t h = o < 0 ? pair_hash(uint32_t(j), uint32_t(i), seed) : pair_hash(uint32_t(i), uint32_t(j), seed);
+        if (a < best || h > bh_best) { best = a; bh_best = h; bj = j; }
+    }
+    // non-finite areas (validated input has none) still pair with a neighbour
+    if (bj < 0) bj = i > 0 ? i - 1 : i + 1;
+    return uint32_t(bj);
+}
 __global__ __launch_bounds__(kBB) void k_nearest(const uint32_t *clusters, uint32_t m, const float4 *nlo,
                                                  const float4 *nhi, int R, uint32_t seed, uint32_t *nearest) {
     __shared__ float4 slo[kBB + 2 * kPlocRadiusMax], shi[kBB + 2 * kPlocRadiusMax];
@@ -204,24 +262,7 @@ __global__ __launch_bounds__(kBB) void k_nearest(const uint32_t *clusters, uint3
     const int64_t i = int64_t(blockIdx.x) * kBB + threadIdx.x;
     if (i >= int64_t(m)) return;
     const int me = threadIdx.x + R;
-    const float3 alo = make_float3(slo[me].x, slo[me].y, slo[me].z), ahi = make_float3(shi[me].x, shi[me].y, shi[me].z);
-    float best = INFINITY;
-    uint32_t bh_best = 0;
-    int64_t bj = -1;
-    for (int o = -R; o <= R; o++) {  // ascending j: on a full tie the first (lower) j stays
-        const int64_t j = i + o;
-        if (o == 0 || j < 0 || j >= int64_t(m)) continue;
-        const float4 bl = slo[me + o], bh = shi[me + o];
-        const float3 lo = make_float3(fminf(alo.x, bl.x), fminf(alo.y, bl.y), fminf(alo.z, bl.z));
-        const float3 hi = make_float3(fmaxf(ahi.x, bh.x), fmaxf(ahi.y, bh.y), fmaxf(ahi.z, bh.z));
-        const float a = half_area(lo, hi);
-        if (a > best) continue;
-        const uint32_t h = o < 0 ? pair_hash(uint32_t(j), uint32_t(i), seed) : pair_hash(uint32_t(i), uint32_t(j), seed);
-        if (a < best || h > bh_best) { best = a; bh_best = h; bj = j; }
-    }
-    // non-finite areas (validated input has none) still pair with a neighbour
-    if (bj < 0) bj = i > 0 ? i - 1 : i + 1;
-    nearest[i] = uint32_t(bj);
+    nearest[i] = nearest_of(i, m, R, seed, slo + me, shi + me);
 }
 
 // flags[i]: bit 32 = cluster i merges with its mutual nearest neighbour (the
@@ -236,25 +277,11 @@ __global__ __launch_bounds__(kBB) void k_merge_flags(const uint32_t *nearest, ui
     flags[i] = (uint64_t(merge) << 32) | uint64_t(keep);
 }
 
-// Creates the merged nodes (ids node_base + merge rank) with their SAH cost and
-// leaf decision, and compacts the surviving clusters in order.
-__global__ __launch_bounds__(kBB) void k_merge(const uint32_t *clusters, const uint32_t *nearest, uint32_t m,
-                                               const uint64_t *flags, const uint64_t *incl, uint32_t node_base,
-                                               float4 *nlo, float4 *nhi, uint2 *kids, float4 *wc, uint32_t *wd,
-                                               uint32_t *out) {
-    const uint32_t i = blockIdx.x * kBB + threadIdx.x;
-    if (i >= m) return;
-    const uint64_t f = flags[i];
-    if (!(f & 1u)) return;
-    const uint64_t s = incl[i];
-    const uint32_t pos = uint32_t(s) - 1u;
-    if (!(f >> 32)) {
-        out[pos] = clusters[i];
-        return;
-    }
-    const uint32_t a = clusters[i], b = clusters[nearest[i]];
-    const uint32_t id = node_base + uint32_t(s >> 32) - 1u;
-    const float4 la = nlo[a], ha = nhi[a], lb = nlo[b], hb = nhi[b];
+// Node `id` over nodes a and b with boxes (la, ha) and (lb, hb): box, SAH cost
+// and leaf decision (also returned in nl, nh), children and collapse table.
+__device__ __forceinline__ void merge_nodes(uint32_t a, uint32_t b, float4 la, float4 ha, float4 lb, float4 hb, uint32_t id,
+                                            float4 &nl, float4 &nh, float4 *nlo, float4 *nhi, uint2 *kids, float4 *wc,
+                                            uint32_t *wd) {
     const float3 lo = make_float3(fminf(la.x, lb.x), fminf(la.y, lb.y), fminf(la.z, lb.z));
     const float3 hi = make_float3(fmaxf(ha.x, hb.x), fmaxf(ha.y, hb.y), fmaxf(ha.z, hb.z));
     const uint32_t cnt = (__float_as_uint(ha.w) & ~kLeafMark) + (__float_as_uint(hb.w) & ~kLeafMark);
@@ -262,8 +289,10 @@ __global__ __launch_bounds__(kBB) void k_merge(const uint32_t *clusters, const u
     const float inner = kCt * A + la.w + lb.w;
     const float leaf_cost = kCi * float(cnt) * A;
     const bool leaf = cnt <= uint32_t(kMaxLeafTris) && leaf_cost <= inner;
-    nlo[id] = make_float4(lo.x, lo.y, lo.z, leaf ? leaf_cost : inner);
-    nhi[id] = make_float4(hi.x, hi.y, hi.z, __uint_as_float(cnt | (leaf ? kLeafMark : 0u)));
+    nl = make_float4(lo.x, lo.y, lo.z, leaf ? leaf_cost : inner);
+    nh = make_float4(hi.x, hi.y, hi.z, __uint_as_float(cnt | (leaf ? kLeafMark : 0u)));
+    nlo[id] = nl;
+    nhi[id] = nh;
     kids[id] = make_uint2(a, b);
     // collapse table (a binary SAH leaf stays one wide leaf)
     if (leaf) {
@@ -298,7 +327,120 @@ __global__ __launch_bounds__(kBB) void k_merge(const uint32_t *clusters, const u
         wc[id] = make_float4(c[0], c[1], c[2], c[3]);
         wd[id] = w | dk[4] << 8;
     }
+}
+
+// Creates the merged nodes (ids node_base + merge rank) with their SAH cost and
+// leaf decision, and compacts the surviving clusters in order.
+__global__ __launch_bounds__(kBB) void k_merge(const uint32_t *clusters, const uint32_t *nearest, uint32_t m,
+                                               const uint64_t *flags, const uint64_t *incl, uint32_t node_base,
+                                               float4 *nlo, float4 *nhi, uint2 *kids, float4 *wc, uint32_t *wd,
+                                               uint32_t *out) {
+    const uint32_t i = blockIdx.x * kBB + threadIdx.x;
+    if (i >= m) return;
+    const uint64_t f = flags[i];
+    if (!(f & 1u)) return;
+    const uint64_t s = incl[i];
+    const uint32_t pos = uint32_t(s) - 1u;
+    if (!(f >> 32)) {
+        out[pos] = clusters[i];
+        return;
+    }
+    const uint32_t a = clusters[i], b = clusters[nearest[i]];
+    const uint32_t id = node_base + uint32_t(s >> 32) - 1u;
+    const float4 la = nlo[a], ha = nhi[a], lb = nlo[b], hb = nhi[b];
+    float4 nl, nh;
+    merge_nodes(a, b, la, ha, lb, hb, id, nl, nh, nlo, nhi, kids, wc, wd);
     out[pos] = id;
+}
+
+// The last iterations, from m <= kTailClusters clusters to one, in one block: the
+// same searches, merges and order as the kernels above, with the clusters' boxes
+// in LDS.  Of the 63 iterations over 1.31M triangles, 34 have fewer clusters than
+// this, and each was five launches and a host round trip (35 us) for a few
+// microseconds of work; here one takes 10 us, bound by the search loop of the one
+// CU.  Clustering 2.65 -> 2.1 ms.  2048 is what the LDS holds at two clusters a
+// thread; one iteration at that size costs what the launches of one cost.
+// out: root, node count, iterations, 1 if no progress was made.
+constexpr uint32_t kTailClusters = 2048;
+constexpr int kTailBlock = 1024;
+__global__ __launch_bounds__(kTailBlock) void k_ploc_tail(const uint32_t *clusters, uint32_t m, int R, uint32_t seed,
+                                                          uint32_t node_base, float4 *nlo, float4 *nhi, uint2 *kids,
+                                                          float4 *wc, uint32_t *wd, uint32_t *out) {
+    __shared__ float4 lo[kTailClusters], hi[kTailClusters];
+    __shared__ uint32_t id[kTailClusters], near[kTailClusters], wave_sum[kTailBlock / 64];
+    const uint32_t t = threadIdx.x, wave = t / 64, lane = t % 64;
+    for (uint32_t i = t; i < m; i += kTailBlock) {
+        const uint32_t c = clusters[i];
+        id[i] = c;
+        lo[i] = nlo[c];
+        hi[i] = nhi[c];
+    }
+    __syncthreads();
+    bool stuck = false;
+    while (m > 1 && !stuck) {
+        for (uint32_t i = t; i < m; i += kTailBlock) near[i] = nearest_of(i, m, R, seed, lo + i, hi + i);
+        __syncthreads();
+        // clusters 2t and 2t + 1 are this thread's: (merges, survivors) before them, packed in 16 bits each
+        bool merge[2] = {false, false}, keep[2] = {false, false};
+        uint32_t mine = 0;
+        for (uint32_t k = 0; k < 2; k++) {
+            const uint32_t i = 2 * t + k;
+            if (i >= m) continue;
+            const uint32_t j = near[i];
+            const bool mutual = near[j] == i;
+            merge[k] = mutual && i < j;
+            keep[k] = !(mutual && i > j);
+            mine += (merge[k] ? 1u << 16 : 0u) + (keep[k] ? 1u : 0u);
+        }
+        uint32_t incl = mine;
+        for (int o = 1; o < 64; o <<= 1) {
+            const uint32_t v = __shfl_up(incl, o);
+            if (int(lane) >= o) incl += v;
+        }
+        if (lane == 63) wave_sum[wave] = incl;
+        __syncthreads();
+        uint32_t before = incl - mine, total = 0;
+        for (uint32_t w = 0; w < kTailBlock / 64; w++) {
+            if (w < wave) before += wave_sum[w];
+            total += wave_sum[w];
+        }
+        const uint32_t merges = total >> 16, kept = total & 0xFFFFu;
+        float4 nl[2], nh[2];
+        uint32_t nid[2] = {0, 0}, pos[2] = {0, 0};
+        for (uint32_t k = 0; k < 2; k++) {
+            if (!keep[k]) continue;
+            const uint32_t i = 2 * t + k;
+            pos[k] = before & 0xFFFFu;
+            if (merge[k]) {
+                const uint32_t j = near[i];
+                nid[k] = node_base + (before >> 16);
+                merge_nodes(id[i], id[j], lo[i], hi[i], lo[j], hi[j], nid[k], nl[k], nh[k], nlo, nhi, kids, wc, wd);
+            } else {
+                nid[k] = id[i];
+                nl[k] = lo[i];
+                nh[k] = hi[i];
+            }
+            before += (merge[k] ? 1u << 16 : 0u) + 1u;
+        }
+        __syncthreads();  // everything is read (and the new tables written) before the clusters move
+        for (int k = 0; k < 2; k++)
+            if (keep[k]) {
+                id[pos[k]] = nid[k];
+                lo[pos[k]] = nl[k];
+                hi[pos[k]] = nh[k];
+            }
+        __syncthreads();
+        stuck = merges == 0 || kept != m - merges;
+        node_base += merges;
+        m = kept;
+        seed++;
+    }
+    if (t == 0) {
+        out[0] = id[0];
+        out[1] = node_base;
+        out[2] = seed;
+        out[3] = stuck ? 1u : 0u;
+    }
 }
 
 // ---------------------------------------------------------------- collapse to Node4
@@ -383,7 +525,6 @@ struct CollapseArgs {
     const uint32_t *tris, *tri_geom;
     Node4 *out;
     float4 *tri_out;                     // leaf-order TriRecords (3 float4 each)
-    uint32_t *leaf_orig;                 // leaf order -> input triangle
     uint4 *qnext;
     uint32_t *max_stack;
 };
@@ -431,7 +572,6 @@ __global__ __launch_bounds__(kBB) void k_collapse(CollapseArgs a) {
                                        __uint_as_float(a.tri_geom[t]));
                     r[2] = make_float4(a.verts[3 * size_t(i2)], a.verts[3 * size_t(i2) + 1], a.verts[3 * size_t(i2) + 2],
                                        0.f);
-                    a.leaf_orig[p] = t;
                     p++;
                 } else if (sp + 2 <= kMaxLeafTris + 1) {
                     const uint2 g = a.kids[v];
@@ -459,93 +599,100 @@ __global__ __launch_bounds__(kBB) void k_collapse(CollapseArgs a) {
 
 inline unsigned grid_of(uint64_t n) { return unsigned((n + kBB - 1) / kBB); }
 
-// Device allocations of one build, released on every return path once the
-// build's stream has finished with them.
-struct Scratch {
-    hipStream_t stream = nullptr;
-    std::vector<void *> ptrs;
-    template <typename T>
-    hipError_t alloc(T **p, size_t count) {
-        void *q = nullptr;
-        hipError_t e = hipMalloc(&q, std::max<size_t>(count * sizeof(T), 256));
-        if (e == hipSuccess) ptrs.push_back(q);
-        *p = static_cast<T *>(q);
-        return e;
-    }
-    ~Scratch() {
-        if (stream) (void)hipStreamSynchronize(stream);
-        for (void *p : ptrs) (void)hipFree(p);
-    }
-};
-
 }  // namespace
 
-int build_bvh4_gpu(const float *d_verts, const uint32_t *d_tris, const uint32_t *d_tri_geom, uint32_t n,
-                   hipStream_t stream, int radius, uint32_t *leaf_to_orig, GpuBvhResult *res) {
+int bvh_gpu_plan(uint32_t n, uint32_t n_verts, hipStream_t stream, BuildArena *arena, BuildBuffers *b) {
+    const size_t nn = 2 * size_t(n) - 1;
+    const size_t node_cap = n;
+    arena->want(&b->verts, 3 * size_t(n_verts));
+    arena->want(&b->tris, 3 * size_t(n));
+    arena->want(&b->tri_geom, n);
+    arena->want(&b->partial, 6 * kBoundsBlocks);
+    arena->want(&b->cbox, 6);
+    arena->want(&b->flags32, 1);
+    arena->want(&b->keys, n);
+    arena->want(&b->keys2, n);
+    arena->want(&b->vals, n);
+    arena->want(&b->order, n);
+    arena->want(&b->nlo, nn);
+    arena->want(&b->nhi, nn);
+    arena->want(&b->kids, nn);
+    arena->want(&b->wc, nn);
+    arena->want(&b->wd, nn);
+    arena->want(&b->cl, n);
+    arena->want(&b->cl2, n);
+    arena->want(&b->nearest, n);
+    arena->want(&b->flags, n);
+    arena->want(&b->incl, n);
+    arena->want(&b->q, node_cap);
+    arena->want(&b->q2, node_cap);
+    arena->want(&b->ekid, node_cap);
+    arena->want(&b->eoff, node_cap);
+    arena->want(&b->einner, node_cap);
+    arena->want(&b->eincl, node_cap);
+    arena->want(&b->counts, 8);
+    arena->want(&b->nodes_tmp, node_cap);
+    // library temporary storage, sized for the largest call
+    WR_HIP(rocprim::radix_sort_pairs(nullptr, b->sort_bytes, (uint64_t *)nullptr, (uint64_t *)nullptr, (uint32_t *)nullptr,
+                                     (uint32_t *)nullptr, n, 0, 63, stream));
+    WR_HIP(rocprim::inclusive_scan(nullptr, b->scan64_bytes, (uint64_t *)nullptr, (uint64_t *)nullptr, size_t(n),
+                                   rocprim::plus<uint64_t>(), stream));
+    WR_HIP(rocprim::inclusive_scan(nullptr, b->scan32_bytes, (uint32_t *)nullptr, (uint32_t *)nullptr, node_cap,
+                                   rocprim::plus<uint32_t>(), stream));
+    arena->want(&b->tmp, std::max(b->sort_bytes, std::max(b->scan64_bytes, b->scan32_bytes)));
+    return WR_OK;
+}
+
+int mesh_check_gpu(const BuildBuffers &b, uint32_t n, uint32_t n_verts, uint32_t n_geoms, hipStream_t stream, bool *valid,
+                   float box[6]) {
+    const int blocks = int(std::min<uint64_t>(kBoundsBlocks, std::max<uint64_t>(1, grid_of(3 * uint64_t(std::max(n, n_verts))))));
+    WR_HIP(hipMemsetAsync(b.flags32, 0, sizeof(uint32_t), stream));
+    k_check_mesh<<<blocks, kBB, 0, stream>>>(b.verts, n_verts, b.tris, b.tri_geom, n, n_geoms, b.partial, b.flags32);
+    k_centroid_final<<<1, kBB, 0, stream>>>(b.partial, blocks, b.cbox);
+    WR_HIP(hipGetLastError());
+    uint32_t invalid = 0;
+    WR_HIP(hipMemcpyAsync(&invalid, b.flags32, sizeof invalid, hipMemcpyDeviceToHost, stream));
+    WR_HIP(hipMemcpyAsync(box, b.cbox, 6 * sizeof(float), hipMemcpyDeviceToHost, stream));
+    WR_HIP(hipStreamSynchronize(stream));
+    *valid = invalid == 0;
+    return WR_OK;
+}
+
+// The Node4 of a scene without triangles.
+static int empty_bvh(GpuBvhResult *res) {
+    Node4 nd;
+    for (int i = 0; i < 4; i++) {
+        nd.lo_x[i] = nd.lo_y[i] = nd.lo_z[i] = FLT_MAX;
+        nd.hi_x[i] = nd.hi_y[i] = nd.hi_z[i] = -FLT_MAX;
+        nd.child[i] = kEmptyChild;
+        nd.count[i] = 0;
+    }
+    WR_HIP(hipMalloc(&res->nodes, sizeof(Node4)));
+    WR_HIP(hipMalloc(&res->tris, 128));
+    WR_HIP(hipMemcpy(res->nodes, &nd, sizeof(Node4), hipMemcpyHostToDevice));
+    res->n_nodes = 1;
+    res->max_stack = 1;
+    res->depth = 1;
+    return WR_OK;
+}
+
+int build_bvh4_gpu(wr_device *dev, const BuildBuffers &b, uint32_t n, hipStream_t stream, int radius, GpuBvhResult *res) {
     *res = GpuBvhResult{};
     const int R = radius > 0 ? std::min(radius, kPlocRadiusMax) : kPlocRadius;
     const auto t0 = std::chrono::steady_clock::now();
-    if (n == 0) {
-        Node4 nd;
-        for (int i = 0; i < 4; i++) {
-            nd.lo_x[i] = nd.lo_y[i] = nd.lo_z[i] = FLT_MAX;
-            nd.hi_x[i] = nd.hi_y[i] = nd.hi_z[i] = -FLT_MAX;
-            nd.child[i] = kEmptyChild;
-            nd.count[i] = 0;
-        }
-        WR_HIP(hipMalloc(&res->nodes, sizeof(Node4)));
-        WR_HIP(hipMalloc(&res->tris, 128));
-        WR_HIP(hipMemcpy(res->nodes, &nd, sizeof(Node4), hipMemcpyHostToDevice));
-        res->n_nodes = 1;
-        res->max_stack = 1;
-        res->depth = 1;
-        return WR_OK;
-    }
-    Scratch sc;
-    sc.stream = stream;
-    const size_t nn = 2 * size_t(n) - 1;
-    float *partial, *cbox;
-    uint64_t *keys, *keys2, *flags, *incl;
-    uint32_t *vals, *order, *cl, *cl2, *nearest, *einner, *eincl, *max_stack, *leaf_orig;
-    float4 *nlo, *nhi, *wc;
-    uint32_t *wd;
-    uint2 *kids;
-    uint4 *q, *q2, *ekid, *eoff;
-    Node4 *nodes_tmp;
-    const size_t node_cap = std::max<size_t>(1, n);
-    WR_HIP(sc.alloc(&partial, 6 * kBoundsBlocks));
-    WR_HIP(sc.alloc(&cbox, 6));
-    WR_HIP(sc.alloc(&keys, n));
-    WR_HIP(sc.alloc(&keys2, n));
-    WR_HIP(sc.alloc(&vals, n));
-    WR_HIP(sc.alloc(&order, n));
-    WR_HIP(sc.alloc(&nlo, nn));
-    WR_HIP(sc.alloc(&nhi, nn));
-    WR_HIP(sc.alloc(&kids, nn));
-    WR_HIP(sc.alloc(&wc, nn));
-    WR_HIP(sc.alloc(&wd, nn));
-    WR_HIP(sc.alloc(&cl, n));
-    WR_HIP(sc.alloc(&cl2, n));
-    WR_HIP(sc.alloc(&nearest, n));
-    WR_HIP(sc.alloc(&flags, n));
-    WR_HIP(sc.alloc(&incl, n));
-    WR_HIP(sc.alloc(&q, node_cap));
-    WR_HIP(sc.alloc(&q2, node_cap));
-    WR_HIP(sc.alloc(&ekid, node_cap));
-    WR_HIP(sc.alloc(&eoff, node_cap));
-    WR_HIP(sc.alloc(&einner, node_cap));
-    WR_HIP(sc.alloc(&eincl, node_cap));
-    WR_HIP(sc.alloc(&max_stack, 1));
-    WR_HIP(sc.alloc(&leaf_orig, n));
-    WR_HIP(sc.alloc(&nodes_tmp, node_cap));
-    // library temporary storage, sized for the largest call
-    size_t sort_bytes = 0, scan64_bytes = 0, scan32_bytes = 0;
-    WR_HIP(rocprim::radix_sort_pairs(nullptr, sort_bytes, keys, keys2, vals, order, n, 0, 63, stream));
-    WR_HIP(rocprim::inclusive_scan(nullptr, scan64_bytes, flags, incl, size_t(n), rocprim::plus<uint64_t>(), stream));
-    WR_HIP(rocprim::inclusive_scan(nullptr, scan32_bytes, einner, eincl, node_cap, rocprim::plus<uint32_t>(), stream));
-    void *tmp;
-    const size_t tmp_bytes = std::max(sort_bytes, std::max(scan64_bytes, scan32_bytes));
-    WR_HIP(sc.alloc(reinterpret_cast<uint8_t **>(&tmp), tmp_bytes));
+    if (n == 0) return empty_bvh(res);
+    const size_t nn = 2 * size_t(n) - 1, node_cap = n;
+    const float *d_verts = b.verts;
+    const uint32_t *d_tris = b.tris, *d_tri_geom = b.tri_geom;
+    float *partial = b.partial, *cbox = b.cbox;
+    uint64_t *keys = b.keys, *keys2 = b.keys2, *flags = b.flags, *incl = b.incl;
+    uint32_t *vals = b.vals, *order = b.order, *cl = b.cl, *cl2 = b.cl2, *nearest = b.nearest, *einner = b.einner,
+             *eincl = b.eincl, *tail = b.counts, *max_stack = b.counts + 4, *wd = b.wd;
+    float4 *nlo = b.nlo, *nhi = b.nhi, *wc = b.wc;
+    uint2 *kids = b.kids;
+    uint4 *q = b.q, *q2 = b.q2, *ekid = b.ekid, *eoff = b.eoff;
+    Node4 *nodes_tmp = b.nodes_tmp;
+    void *tmp = b.tmp;
 
     // Morton order
     const int nb = int(std::min<uint64_t>(kBoundsBlocks, grid_of(n)));
@@ -553,7 +700,7 @@ int build_bvh4_gpu(const float *d_verts, const uint32_t *d_tris, const uint32_t 
     k_centroid_final<<<1, kBB, 0, stream>>>(partial, nb, cbox);
     k_morton<<<grid_of(n), kBB, 0, stream>>>(d_verts, d_tris, n, cbox, keys, vals);
     WR_HIP(hipGetLastError());
-    size_t bytes = sort_bytes;
+    size_t bytes = b.sort_bytes;
     WR_HIP(rocprim::radix_sort_pairs(tmp, bytes, keys, keys2, vals, order, n, 0, 63, stream));
     k_leaves<<<grid_of(n), kBB, 0, stream>>>(d_verts, d_tris, n, order, nlo, nhi, kids, wc, wd, cl);
     WR_HIP(hipGetLastError());
@@ -561,11 +708,11 @@ int build_bvh4_gpu(const float *d_verts, const uint32_t *d_tris, const uint32_t 
     // PLOC
     uint32_t m = n, node_base = n, iters = 0;
     uint64_t total = 0;
-    while (m > 1) {
+    while (m > kTailClusters) {
         k_nearest<<<grid_of(m), kBB, 0, stream>>>(cl, m, nlo, nhi, R, iters, nearest);
         k_merge_flags<<<grid_of(m), kBB, 0, stream>>>(nearest, m, flags);
         WR_HIP(hipGetLastError());
-        bytes = scan64_bytes;
+        bytes = b.scan64_bytes;
         WR_HIP(rocprim::inclusive_scan(tmp, bytes, flags, incl, size_t(m), rocprim::plus<uint64_t>(), stream));
         k_merge<<<grid_of(m), kBB, 0, stream>>>(cl, nearest, m, flags, incl, node_base, nlo, nhi, kids, wc, wd,
                                                 cl2);
@@ -580,14 +727,18 @@ int build_bvh4_gpu(const float *d_verts, const uint32_t *d_tris, const uint32_t 
         std::swap(cl, cl2);
         iters++;
     }
-    if (node_base != nn) return set_error(WR_ERR_DEVICE, "GPU BVH build: node count mismatch");
-    uint32_t root = 0;
-    WR_HIP(hipMemcpyAsync(&root, cl, sizeof root, hipMemcpyDeviceToHost, stream));
+    k_ploc_tail<<<1, kTailBlock, 0, stream>>>(cl, m, R, iters, node_base, nlo, nhi, kids, wc, wd, tail);
+    WR_HIP(hipGetLastError());
+    uint32_t ended[4];
+    WR_HIP(hipMemcpyAsync(ended, tail, sizeof ended, hipMemcpyDeviceToHost, stream));
 
     // collapse, level by level (breadth-first node order: children after parents)
-    WR_HIP(hipMalloc(&res->tris, std::max<size_t>(sizeof(TriRecord) * n, 128)));
-    const uint4 q0 = make_uint4(root, 0u, 0u, 0u);
+    WR_HIP(dev->alloc(reinterpret_cast<void **>(&res->tris), std::max<size_t>(sizeof(TriRecord) * n, 128)));
     WR_HIP(hipStreamSynchronize(stream));
+    if (ended[3]) return set_error(WR_ERR_DEVICE, "GPU BVH build: clustering made no progress (non-finite vertices?)");
+    if (ended[1] != nn) return set_error(WR_ERR_DEVICE, "GPU BVH build: node count mismatch");
+    iters = ended[2];
+    const uint4 q0 = make_uint4(ended[0], 0u, 0u, 0u);
     WR_HIP(hipMemcpyAsync(q, &q0, sizeof q0, hipMemcpyHostToDevice, stream));
     WR_HIP(hipMemsetAsync(max_stack, 0, sizeof(uint32_t), stream));
     uint32_t qn = 1, level_base = 0, depth = 0;
@@ -595,12 +746,11 @@ int build_bvh4_gpu(const float *d_verts, const uint32_t *d_tris, const uint32_t 
         const uint32_t next_base = level_base + qn;
         k_expand<<<grid_of(qn), kBB, 0, stream>>>(q, qn, nlo, nhi, kids, wd, ekid, eoff, einner);
         WR_HIP(hipGetLastError());
-        bytes = scan32_bytes;
+        bytes = b.scan32_bytes;
         WR_HIP(rocprim::inclusive_scan(tmp, bytes, einner, eincl, size_t(qn), rocprim::plus<uint32_t>(), stream));
         uint32_t inner_total = 0;
         CollapseArgs ca{q, qn, level_base, next_base, ekid, eoff, einner, eincl, nlo, nhi, kids, wd, n,
-                        d_verts, d_tris, d_tri_geom, nodes_tmp, reinterpret_cast<float4 *>(res->tris), leaf_orig,
-                        q2, max_stack};
+                        d_verts, d_tris, d_tri_geom, nodes_tmp, reinterpret_cast<float4 *>(res->tris), q2, max_stack};
         // this level's nodes end at next_base (checked by the previous level); its
         // children must fit behind them
         WR_HIP(hipMemcpyAsync(&inner_total, eincl + (qn - 1), sizeof inner_total, hipMemcpyDeviceToHost, stream));
@@ -617,9 +767,8 @@ int build_bvh4_gpu(const float *d_verts, const uint32_t *d_tris, const uint32_t 
     const uint32_t n_nodes = level_base;
     uint32_t ms = 0;
     WR_HIP(hipMemcpyAsync(&ms, max_stack, sizeof ms, hipMemcpyDeviceToHost, stream));
-    WR_HIP(hipMalloc(&res->nodes, sizeof(Node4) * n_nodes));
+    WR_HIP(dev->alloc(reinterpret_cast<void **>(&res->nodes), sizeof(Node4) * n_nodes));
     WR_HIP(hipMemcpyAsync(res->nodes, nodes_tmp, sizeof(Node4) * n_nodes, hipMemcpyDeviceToDevice, stream));
-    WR_HIP(hipMemcpyAsync(leaf_to_orig, leaf_orig, sizeof(uint32_t) * n, hipMemcpyDeviceToHost, stream));
     WR_HIP(hipStreamSynchronize(stream));
     res->n_nodes = n_nodes;
     res->max_stack = ms;

@@ -3,8 +3,11 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <map>
+#include <mutex>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "../../include/wurst_amd.h"
@@ -113,12 +116,96 @@ struct RenderArgs {
 };
 
 // ============================================================== host objects
+// Device memory that outlives the calls which use it, kept by a device handle.
+// A caller takes a block and gives it back when its stream has finished with
+// it; blocks are handed to one caller at a time, so streams and threads never
+// share one, and at most `keep` free blocks of at most `most` bytes are held.
+struct BlockPool {
+    struct Block { void *p = nullptr; size_t bytes = 0; };
+    int keep;
+    size_t most;
+    std::mutex m;
+    std::vector<Block> free_blocks;
+    BlockPool(int keep_, size_t most_) : keep(keep_), most(most_) {}
+    ~BlockPool() {
+        for (Block &b : free_blocks) (void)hipFree(b.p);
+    }
+    // the smallest free block of at least `bytes`, else a new one
+    hipError_t take(size_t bytes, Block *out) {
+        {
+            std::lock_guard<std::mutex> lock(m);
+            size_t best = free_blocks.size();
+            for (size_t i = 0; i < free_blocks.size(); i++)
+                if (free_blocks[i].bytes >= bytes &&
+                    (best == free_blocks.size() || free_blocks[i].bytes < free_blocks[best].bytes))
+                    best = i;
+            if (best < free_blocks.size()) {
+                *out = free_blocks[best];
+                free_blocks.erase(free_blocks.begin() + long(best));
+                return hipSuccess;
+            }
+        }
+        const hipError_t e = hipMalloc(&out->p, bytes);
+        if (e != hipSuccess) out->p = nullptr;
+        out->bytes = e == hipSuccess ? bytes : 0;
+        return e;
+    }
+    // gives every free block back to the runtime
+    void trim() {
+        std::lock_guard<std::mutex> lock(m);
+        for (Block &b : free_blocks) (void)hipFree(b.p);
+        free_blocks.clear();
+    }
+    void give(Block b) {
+        if (!b.p) return;
+        Block drop = b;
+        if (b.bytes <= most) {
+            std::lock_guard<std::mutex> lock(m);
+            free_blocks.push_back(b);
+            drop = Block{};
+            if (int(free_blocks.size()) > keep) {  // the smallest goes
+                size_t k = 0;
+                for (size_t i = 1; i < free_blocks.size(); i++)
+                    if (free_blocks[i].bytes < free_blocks[k].bytes) k = i;
+                drop = free_blocks[k];
+                free_blocks.erase(free_blocks.begin() + long(k));
+            }
+        }
+        if (drop.p) (void)hipFree(drop.p);
+    }
+};
+
 struct wr_device {
     int ordinal = 0;
     int n_cu = 256;
     // resident blocks per CU of each kernel (HIP occupancy API), used to size persistent grids
     int occ_rays = 8, occ_shade = 8, occ_generate = 8, occ_trace = 8;
     std::map<const void *, int> occ_cache;  // other kernels, filled on first use
+    BlockPool spills{2, size_t(1) << 30};       // traversal stack spill regions, one per scene
+    BlockPool build_memory{1, size_t(1) << 30}; // mesh copies and scratch of BVH builds
+    void trim() {
+        spills.trim();
+        build_memory.trim();
+    }
+    // hipMalloc that frees the pools' idle blocks where memory runs out
+    hipError_t alloc(void **p, size_t bytes) {
+        hipError_t e = hipMalloc(p, bytes);
+        if (e == hipErrorOutOfMemory) {
+            (void)hipGetLastError();
+            trim();
+            e = hipMalloc(p, bytes);
+        }
+        return e;
+    }
+    hipError_t take(BlockPool &pool, size_t bytes, BlockPool::Block *b) {
+        hipError_t e = pool.take(bytes, b);
+        if (e == hipErrorOutOfMemory) {
+            (void)hipGetLastError();
+            trim();
+            e = pool.take(bytes, b);
+        }
+        return e;
+    }
     TransferRing ring;        // pinned buffers of large host transfers
     void *scratch = nullptr;  // device address of wr_render_nee_noalloc's fixed region on this GPU
 };
@@ -130,8 +217,11 @@ struct wr_scene {
     // device allocations
     Node4 *d_nodes = nullptr;   // the build's BVH4 (checks and statistics)
     NodeQ *d_qnodes = nullptr;  // its quantised copy, which the kernels traverse
-    float4 *d_tris = nullptr, *d_ltris = nullptr;
+    float4 *d_tris = nullptr;
+    void *d_tables = nullptr;   // one allocation behind the five tables below
+    float4 *d_ltris = nullptr;
     uint2 *d_spill = nullptr;   // traversal stack spill: kSpillDepth entries per lane of the largest grid
+    BlockPool::Block spill;     // the block behind it, from the device's pool
     float4 *d_bdpt = nullptr;   // bidirectional light-vertex records (+ 2 ray counters), grown on demand
     size_t bdpt_bytes = 0;
     int max_trav_blocks = 0;
@@ -149,8 +239,8 @@ struct wr_scene {
     int ploc_radius = 0;                // its clustering window (GPU builder; 0 = default)
     uint32_t bvh_depth = 0, bvh_iterations = 0;
     double build_ms = 0.0;
-    // host side: triangle index -> (geom, prim)
-    std::vector<uint32_t> tri_geom, geom_first, leaf_to_orig;
+    // first triangle of each geometry
+    std::vector<uint32_t> geom_first;
     int W = 0, H = 0;
     float box[6] = {0, 0, 0, 0, 0, 0};  // bounds of the vertices (lo xyz, hi xyz)
     // path buffers (lazily sized)
@@ -181,13 +271,62 @@ struct GpuBvhResult {
     uint32_t n_nodes = 0, max_stack = 0, depth = 0, iterations = 0;
     double ms = 0.0;            // wall time of the build
 };
-// Builds from a mesh already in device memory (verts [3n_v], tris [3n], tri_geom [n],
-// indices validated) with a clustering window of `radius` clusters on each side
-// (0: default, at most 64); leaf_to_orig (host, n entries) receives the input
-// triangle of each leaf-order record.  On error the caller frees whatever
+// Temporary device memory of one build: every array is asked for with want(),
+// commit() takes one block for all of them from the device's pool and sets the
+// pointers, and the block goes back when the object dies, after the stream has
+// finished.  (26 allocations and frees took 5 ms of a 15 ms scene creation.)
+struct BuildArena {
+    wr_device *dev;
+    hipStream_t stream;
+    BlockPool::Block block;
+    size_t total = 0;
+    std::vector<std::pair<void **, size_t>> wants;
+    BuildArena(wr_device *d, hipStream_t st) : dev(d), stream(st) {}
+    BuildArena(const BuildArena &) = delete;
+    BuildArena &operator=(const BuildArena &) = delete;
+    template <typename T>
+    void want(T **p, size_t count) {
+        wants.emplace_back(reinterpret_cast<void **>(p), total);
+        total += (std::max<size_t>(count * sizeof(T), 1) + 255) / 256 * 256;
+    }
+    hipError_t commit() {
+        const hipError_t e = dev->take(dev->build_memory, total, &block);
+        if (e == hipSuccess)
+            for (auto &w : wants) *w.first = static_cast<char *>(block.p) + w.second;
+        return e;
+    }
+    ~BuildArena() {
+        (void)hipStreamSynchronize(stream);
+        dev->build_memory.give(block);
+    }
+};
+// The build's arrays, all in a BuildArena.
+struct BuildBuffers {
+    float *verts;                  // the mesh
+    uint32_t *tris, *tri_geom;
+    float *partial, *cbox;         // bounds: per block, then min xyz and max xyz
+    uint32_t *flags32;             // [0]: the mesh is invalid
+    uint64_t *keys, *keys2, *flags, *incl;
+    uint32_t *vals, *order, *cl, *cl2, *nearest, *einner, *eincl, *counts;
+    float4 *nlo, *nhi, *wc;
+    uint32_t *wd;
+    uint2 *kids;
+    uint4 *q, *q2, *ekid, *eoff;
+    Node4 *nodes_tmp;
+    uint8_t *tmp;                  // the library's temporary storage
+    size_t sort_bytes, scan64_bytes, scan32_bytes;
+};
+// Asks for the arrays of a build over n > 0 triangles and n_verts vertices.
+int bvh_gpu_plan(uint32_t n, uint32_t n_verts, hipStream_t stream, BuildArena *arena, BuildBuffers *b);
+// Checks the mesh in the build's arrays as the host checks of a scene do (finite
+// vertices, indices in range, triangles of a geometry contiguous and ordered)
+// and finds the bounds of its vertices (lo xyz, hi xyz).
+int mesh_check_gpu(const BuildBuffers &b, uint32_t n, uint32_t n_verts, uint32_t n_geoms, hipStream_t stream, bool *valid,
+                   float box[6]);
+// Builds from a checked mesh with a clustering window of `radius` clusters on
+// each side (0: default, at most 64).  On error the caller frees whatever
 // out->nodes / out->tris hold.
-int build_bvh4_gpu(const float *d_verts, const uint32_t *d_tris, const uint32_t *d_tri_geom, uint32_t n,
-                   hipStream_t stream, int radius, uint32_t *leaf_to_orig, GpuBvhResult *out);
+int build_bvh4_gpu(wr_device *dev, const BuildBuffers &b, uint32_t n, hipStream_t stream, int radius, GpuBvhResult *out);
 }  // namespace wr
 
 // ============================================================== guiding (wr_guide.hip)

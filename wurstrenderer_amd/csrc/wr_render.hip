@@ -1788,6 +1788,8 @@ int wr_device_create(int ordinal, wr_device **out) {
 
 void wr_device_destroy(wr_device *dev) { delete dev; }
 
+constexpr size_t align256(size_t b) { return (b + 255) / 256 * 256; }
+
 void wr_scene_destroy(wr_scene *s) {
     if (!s) return;
     (void)hipSetDevice(s->dev->ordinal);
@@ -1795,14 +1797,10 @@ void wr_scene_destroy(wr_scene *s) {
     (void)hipFree(s->d_nodes);
     (void)hipFree(s->d_qnodes);
     (void)hipFree(s->d_tris);
-    (void)hipFree(s->d_ltris);
-    (void)hipFree(s->d_geom);
-    (void)hipFree(s->d_geom_first);
-    (void)hipFree(s->d_mats);
-    (void)hipFree(s->d_lights);
+    (void)hipFree(s->d_tables);
     (void)hipFree(s->d_env);
     (void)hipFree(s->d_env_cdf);
-    (void)hipFree(s->d_spill);
+    s->dev->spills.give(s->spill);
     (void)hipFree(s->d_bdpt);
     (void)hipFree(s->pool);
     if (s->h_counters) (void)hipHostFree(s->h_counters);
@@ -1812,13 +1810,15 @@ void wr_scene_destroy(wr_scene *s) {
     delete s;
 }
 
-static int validate_desc(const wr_scene_desc *d) {
+// `arrays`: also the checks over the vertex and triangle arrays, which the GPU
+// build does on the device (mesh_check_gpu).
+static int validate_desc(const wr_scene_desc *d, bool arrays = true) {
     if (!d) return set_error(WR_ERR_INVALID_ARGUMENT, "desc is null");
     if (d->n_tris > 0 && (!d->verts || !d->tris || !d->tri_geom))
         return set_error(WR_ERR_INVALID_ARGUMENT, "null geometry arrays");
     if (d->n_tris >= kMaxTriangles) return set_error(WR_ERR_UNSUPPORTED, "too many triangles (limit 2^28)");
     if (d->n_verts > 0 && !d->verts) return set_error(WR_ERR_INVALID_ARGUMENT, "null vertex array");
-    for (size_t i = 0; i < 3 * size_t(d->n_verts); i++)
+    for (size_t i = 0; arrays && i < 3 * size_t(d->n_verts); i++)
         if (!std::isfinite(d->verts[i])) return set_error(WR_ERR_INVALID_ARGUMENT, "non-finite vertex coordinate");
     if (d->camera.width <= 0 || d->camera.height <= 0) return set_error(WR_ERR_INVALID_ARGUMENT, "bad resolution");
     if ((uint64_t)d->camera.width * d->camera.height >= (1ull << 31))
@@ -1827,10 +1827,10 @@ static int validate_desc(const wr_scene_desc *d) {
         return set_error(WR_ERR_INVALID_ARGUMENT, "focal distance must be > 0 (the JSON key \"radius\" sets it)");
     if (!(d->camera.fovy_deg > 0.f && d->camera.fovy_deg < 180.f))
         return set_error(WR_ERR_INVALID_ARGUMENT, "fovy must be in (0, 180) degrees");
-    for (uint32_t i = 0; i < 3 * d->n_tris; i++)
+    for (uint32_t i = 0; arrays && i < 3 * d->n_tris; i++)
         if (d->tris[i] >= d->n_verts) return set_error(WR_ERR_INVALID_ARGUMENT, "triangle vertex index out of range");
     uint32_t prev = 0;
-    for (uint32_t t = 0; t < d->n_tris; t++) {
+    for (uint32_t t = 0; arrays && t < d->n_tris; t++) {
         if (d->tri_geom[t] >= d->n_geoms) return set_error(WR_ERR_INVALID_ARGUMENT, "tri_geom out of range");
         if (d->tri_geom[t] < prev) return set_error(WR_ERR_INVALID_ARGUMENT, "triangles of a geometry must be contiguous and ordered");
         prev = d->tri_geom[t];
@@ -1874,14 +1874,22 @@ static int upload(T **dst, const void *src, size_t bytes, uint64_t &total) {
     return WR_OK;
 }
 
+// Bounds of the vertices (lo xyz, hi xyz).
+static void scene_bounds(wr_scene *s, const wr_scene_desc *d) {
+    for (int k = 0; k < 3; k++) { s->box[k] = INFINITY; s->box[3 + k] = -INFINITY; }
+    for (uint32_t v = 0; v < d->n_verts; v++)
+        for (int k = 0; k < 3; k++) {
+            s->box[k] = std::min(s->box[k], d->verts[3 * size_t(v) + k]);
+            s->box[3 + k] = std::max(s->box[3 + k], d->verts[3 * size_t(v) + k]);
+        }
+}
+
 // Host SAH build, uploaded.
 static int bvh_host(wr_scene *s, const wr_scene_desc *d) {
     const auto t0 = std::chrono::steady_clock::now();
     BvhBuildResult bvh;
     if (!build_bvh4(d->verts, d->n_verts, d->tris, d->n_tris, d->tri_geom, &bvh))
         return set_error(WR_ERR_OUT_OF_MEMORY, "host allocation failed during BVH build");
-    s->leaf_to_orig.resize(d->n_tris);
-    for (uint32_t i = 0; i < d->n_tris; i++) s->leaf_to_orig[i] = bvh.tris[i].orig;
     s->n_nodes = bvh.n_nodes;
     s->max_stack = bvh.max_stack;
     s->bvh_depth = bvh.depth;
@@ -1892,22 +1900,34 @@ static int bvh_host(wr_scene *s, const wr_scene_desc *d) {
     return rc;
 }
 
-// GPU PLOC build from a temporary device copy of the mesh.
+// GPU checks and PLOC build from a temporary device copy of the mesh; also sets
+// the scene's bounds.
 static int bvh_gpu(wr_scene *s, const wr_scene_desc *d) {
     const auto t0 = std::chrono::steady_clock::now();
     const uint32_t n = d->n_tris;
-    float *dv = nullptr;
-    uint32_t *dt = nullptr, *dg = nullptr;
-    uint64_t mesh_bytes = 0;
     GpuBvhResult g;
-    int rc = upload(&dv, d->verts, sizeof(float) * 3 * size_t(d->n_verts), mesh_bytes);
-    if (!rc) rc = upload(&dt, d->tris, sizeof(uint32_t) * 3 * size_t(n), mesh_bytes);
-    if (!rc) rc = upload(&dg, d->tri_geom, sizeof(uint32_t) * size_t(n), mesh_bytes);
-    s->leaf_to_orig.resize(n);
-    if (!rc) rc = build_bvh4_gpu(dv, dt, dg, n, s->stream, s->ploc_radius, s->leaf_to_orig.data(), &g);
-    (void)hipFree(dv);
-    (void)hipFree(dt);
-    (void)hipFree(dg);
+    int rc = WR_OK;
+    if (n == 0) {
+        if ((rc = validate_desc(d))) return rc;
+        scene_bounds(s, d);
+        rc = build_bvh4_gpu(s->dev, BuildBuffers{}, 0, s->stream, s->ploc_radius, &g);
+    } else {
+        BuildArena arena(s->dev, s->stream);
+        BuildBuffers b{};
+        if ((rc = bvh_gpu_plan(n, d->n_verts, s->stream, &arena, &b))) return rc;
+        WR_HIP(arena.commit());
+        TransferRing &ring = s->dev->ring;
+        WR_HIP(ring.upload(s->dev->ordinal, s->stream, b.verts, d->verts, sizeof(float) * 3 * size_t(d->n_verts)));
+        WR_HIP(ring.upload(s->dev->ordinal, s->stream, b.tris, d->tris, sizeof(uint32_t) * 3 * size_t(n)));
+        WR_HIP(ring.upload(s->dev->ordinal, s->stream, b.tri_geom, d->tri_geom, sizeof(uint32_t) * size_t(n)));
+        bool valid = false;
+        if ((rc = mesh_check_gpu(b, n, d->n_verts, d->n_geoms, s->stream, &valid, s->box))) return rc;
+        if (!valid) {  // the host checks name the fault
+            rc = validate_desc(d);
+            return rc ? rc : set_error(WR_ERR_INVALID_ARGUMENT, "invalid mesh");
+        }
+        rc = build_bvh4_gpu(s->dev, b, n, s->stream, s->ploc_radius, &g);
+    }
     s->d_nodes = g.nodes;
     s->d_tris = reinterpret_cast<float4 *>(g.tris);
     if (rc) return rc;
@@ -1929,44 +1949,41 @@ static int scene_create_impl(wr_device *dev, const wr_scene_desc *d, int builder
     WR_HIP(hipEventCreate(&s->ev[1]));
     s->W = d->camera.width;
     s->H = d->camera.height;
-    for (int k = 0; k < 3; k++) { s->box[k] = INFINITY; s->box[3 + k] = -INFINITY; }
-    for (uint32_t v = 0; v < d->n_verts; v++)
-        for (int k = 0; k < 3; k++) {
-            s->box[k] = std::min(s->box[k], d->verts[3 * size_t(v) + k]);
-            s->box[3 + k] = std::max(s->box[3 + k], d->verts[3 * size_t(v) + k]);
-        }
-    // host tables
-    s->tri_geom.assign(d->tri_geom, d->tri_geom + d->n_tris);
-    s->geom_first.assign(d->n_geoms, kInvalid);
-    for (uint32_t t = 0; t < d->n_tris; t++)
-        if (s->geom_first[d->tri_geom[t]] == kInvalid) s->geom_first[d->tri_geom[t]] = t;
     // BVH
     s->builder = builder;
     s->ploc_radius = radius;
     s->n_tris = d->n_tris;
+    if (builder == WR_BVH_HOST) scene_bounds(s, d);
     rc = builder == WR_BVH_HOST ? bvh_host(s, d) : bvh_gpu(s, d);
     if (rc) return rc;
-    WR_HIP(hipMalloc(&s->d_qnodes, sizeof(NodeQ) * std::max<uint64_t>(s->n_nodes, 1)));
+    // each geometry's first triangle (kInvalid: none); the triangles are in geometry order
+    s->geom_first.assign(d->n_geoms, kInvalid);
+    if (d->n_geoms > d->n_tris / 32) {
+        for (uint32_t t = d->n_tris; t-- > 0;) s->geom_first[d->tri_geom[t]] = t;
+    } else {
+        for (uint32_t g = 0; g < d->n_geoms; g++) {
+            const uint32_t *first = std::lower_bound(d->tri_geom, d->tri_geom + d->n_tris, g);
+            if (first != d->tri_geom + d->n_tris && *first == g) s->geom_first[g] = uint32_t(first - d->tri_geom);
+        }
+    }
+    WR_HIP(dev->alloc(reinterpret_cast<void **>(&s->d_qnodes), sizeof(NodeQ) * std::max<uint64_t>(s->n_nodes, 1)));
     s->device_bytes += sizeof(NodeQ) * s->n_nodes;
     if (s->n_nodes) {
         k_quantize_nodes<<<uint32_t((s->n_nodes + 255) / 256), 256, 0, s->stream>>>(s->d_nodes, s->d_qnodes,
                                                                                     uint32_t(s->n_nodes));
         WR_HIP(hipGetLastError());
-        WR_HIP(hipStreamSynchronize(s->stream));
     }
     if (s->max_stack > (uint32_t)kStackDepth) return set_error(WR_ERR_UNSUPPORTED, "BVH deeper than the traversal stack");
     s->max_trav_blocks = dev->n_cu * kMaxTraversalBlocksPerCU;
     {
         const size_t spill_bytes = sizeof(uint2) * size_t(s->max_trav_blocks) * kBlock * kSpillDepth;
-        WR_HIP(hipMalloc(&s->d_spill, spill_bytes));
+        WR_HIP(dev->take(dev->spills, spill_bytes, &s->spill));
+        s->d_spill = static_cast<uint2 *>(s->spill.p);
         s->device_bytes += spill_bytes;
     }
     // geometry info
     std::vector<int2> gi(d->n_geoms);
     for (uint32_t g = 0; g < d->n_geoms; g++) gi[g] = make_int2(d->geom_material[g], d->geom_light[g]);
-    rc = upload(&s->d_geom, gi.data(), sizeof(int2) * gi.size(), s->device_bytes);
-    if (!rc) rc = upload(&s->d_geom_first, s->geom_first.data(), sizeof(uint32_t) * s->geom_first.size(), s->device_bytes);
-    if (rc) return rc;
     std::vector<DMat> mats(d->n_materials);
     for (uint32_t m = 0; m < d->n_materials; m++) {
         const wr_material &src = d->materials[m];
@@ -1978,8 +1995,6 @@ static int scene_create_impl(wr_device *dev, const wr_scene_desc *d, int builder
         for (int k = 0; k < 3; k++) { dm.rho_d[k] = src.rho_d[k]; dm.rho_s[k] = src.rho_s[k]; }
         dm.rho_d[3] = dm.rho_s[3] = 0.f;
     }
-    rc = upload(&s->d_mats, mats.data(), sizeof(DMat) * mats.size(), s->device_bytes);
-    if (rc) return rc;
     // lights: selection CdfTable over |L|_2, per-light triangle-area CdfTable (FP64 on the host)
     std::vector<DLight> lights(d->n_lights);
     std::vector<float4> ltris;
@@ -2034,9 +2049,29 @@ static int scene_create_impl(wr_device *dev, const wr_scene_desc *d, int builder
         }
     }
     s->h_lights = lights;
-    rc = upload(&s->d_lights, lights.data(), sizeof(DLight) * lights.size(), s->device_bytes);  // >= 128 B allocated
-    if (!rc) rc = upload(&s->d_ltris, ltris.data(), sizeof(float4) * ltris.size(), s->device_bytes);
-    if (rc) return rc;
+    // the tables in one allocation and one copy, each with room for an entry
+    {
+        struct Table { void **p; const void *src; size_t bytes, at; };
+        Table tabs[] = {{reinterpret_cast<void **>(&s->d_geom), gi.data(), sizeof(int2) * gi.size(), 0},
+                        {reinterpret_cast<void **>(&s->d_geom_first), s->geom_first.data(), sizeof(uint32_t) * s->geom_first.size(), 0},
+                        {reinterpret_cast<void **>(&s->d_mats), mats.data(), sizeof(DMat) * mats.size(), 0},
+                        {reinterpret_cast<void **>(&s->d_lights), lights.data(), sizeof(DLight) * lights.size(), 0},
+                        {reinterpret_cast<void **>(&s->d_ltris), ltris.data(), sizeof(float4) * ltris.size(), 0}};
+        size_t total = 0;
+        for (Table &t : tabs) {
+            t.at = total;
+            total += align256(std::max<size_t>(t.bytes, 1));
+            s->device_bytes += t.bytes;
+        }
+        std::vector<char> host(total);
+        WR_HIP(dev->alloc(&s->d_tables, total));
+        for (Table &t : tabs) {
+            if (t.bytes) std::memcpy(host.data() + t.at, t.src, t.bytes);
+            *t.p = static_cast<char *>(s->d_tables) + t.at;
+        }
+        WR_HIP(hipMemcpyAsync(s->d_tables, host.data(), total, hipMemcpyHostToDevice, s->stream));
+        WR_HIP(hipStreamSynchronize(s->stream));  // the tables and the quantised nodes are there for any stream
+    }
     // camera (ThinlensCamera ctor, thinlens.h:40-55; Camera ctor, camera.h:9-17), FP64 then rounded
     const wr_camera &c = d->camera;
     double o[3] = {c.pos[0], c.pos[1], c.pos[2]}, la[3] = {c.lookat[0], c.lookat[1], c.lookat[2]},
@@ -2095,8 +2130,10 @@ int wr_scene_create_ex(wr_device *dev, const wr_scene_desc *desc, const wr_build
     const int radius = params ? params->ploc_radius : 0;
     if (builder != WR_BVH_GPU && builder != WR_BVH_HOST) return set_error(WR_ERR_INVALID_ARGUMENT, "unknown BVH builder");
     if (radius < 0 || radius > 64) return set_error(WR_ERR_INVALID_ARGUMENT, "ploc_radius must be in [0, 64]");
-    int rc = validate_desc(desc);
-    if (rc) return rc;
+    // the GPU build checks the arrays on the device; where anything else is wrong,
+    // the host's checks say what comes first
+    int rc = validate_desc(desc, builder == WR_BVH_HOST);
+    if (rc) return validate_desc(desc);
     wr_scene *s = new wr_scene;
     rc = scene_create_impl(dev, desc, builder, radius, s);
     if (rc) {
@@ -2139,8 +2176,8 @@ int wr_scene_bvh_check(wr_scene *s, const wr_scene_desc *d, wr_bvh_stats *st) {
     const std::string err = verify_bvh4(r, d->verts, d->tris, d->n_tris);
     if (!err.empty()) return set_error(WR_ERR_DEVICE, "BVH invariant violated: " + err);
     for (uint32_t i = 0; i < s->n_tris; i++)
-        if (tris[i].geom != d->tri_geom[tris[i].orig] || tris[i].orig != s->leaf_to_orig[i])
-            return set_error(WR_ERR_DEVICE, "BVH invariant violated: leaf triangle geometry id or order map");
+        if (tris[i].geom != d->tri_geom[tris[i].orig])
+            return set_error(WR_ERR_DEVICE, "BVH invariant violated: leaf triangle geometry id");
     // the traversal copy: same refs, and every child's planes (origin + q * spacing) contain its Node4 box
     {
         std::vector<NodeQ> qn(s->n_nodes);
@@ -2320,8 +2357,8 @@ int wr_film_create(wr_scene *s, wr_film **out) {
     f->W = s->W;
     f->H = s->H;
     const size_t bytes = sizeof(double) * 3 * size_t(f->W) * f->H;
-    hipError_t e = hipMalloc(&f->d_base, bytes);
-    if (e == hipSuccess) e = hipMalloc(&f->d_splat, bytes);
+    hipError_t e = s->dev->alloc(reinterpret_cast<void **>(&f->d_base), bytes);
+    if (e == hipSuccess) e = s->dev->alloc(reinterpret_cast<void **>(&f->d_splat), bytes);
     if (e != hipSuccess) {
         (void)hipFree(f->d_base);
         delete f;
@@ -2392,7 +2429,6 @@ int wr_film_image(wr_film *f, double base_div, double splat_div, double *rgb) {
 // Byte layout of a path pool of `cap` paths and `samples` per-sample slots
 // (every array 256-byte aligned): the state pair, hits, per-sample radiance,
 // shadow queue (2 entries per path), counters (one 256-byte line each), stats.
-constexpr size_t align256(size_t b) { return (b + 255) / 256 * 256; }
 constexpr size_t pool_bytes(size_t cap, size_t samples) {
     return 8 * align256(16 * cap) + 2 * align256(4 * cap) + align256(8 * cap) + align256(16 * samples) + 3 * align256(32 * cap) +
            align256(4 * kCounterStride * kNumCounterLines) + align256(64);
@@ -2438,7 +2474,7 @@ static int ensure_capacity(wr_scene *s, uint32_t cap, uint32_t samples) {
         s->sample_capacity = 0;
     }
     char *p = nullptr;
-    WR_HIP(hipMalloc(reinterpret_cast<void **>(&p), pool_bytes(cap, samples)));
+    WR_HIP(s->dev->alloc(reinterpret_cast<void **>(&p), pool_bytes(cap, samples)));
     s->pool = p;
     pool_layout(p, cap, samples, &s->pb);
     s->capacity = cap;
@@ -2966,7 +3002,7 @@ int wr_render_bdpt(wr_scene *s, wr_film *f, const wr_render_params *prm, wr_rend
         s->device_bytes -= s->bdpt_bytes;
         s->d_bdpt = nullptr;
         s->bdpt_bytes = 0;
-        WR_HIP(hipMalloc(&s->d_bdpt, need));
+        WR_HIP(s->dev->alloc(reinterpret_cast<void **>(&s->d_bdpt), need));
         s->bdpt_bytes = need;
         s->device_bytes += need;
     }
@@ -3281,7 +3317,7 @@ static int trace_host(wr_scene *s, const float *rays, uint32_t n, size_t result_
     if (rc) return rc;
     const size_t ray_bytes = sizeof(float) * 8 * size_t(n);
     char *d = nullptr;
-    WR_HIP(hipMalloc(reinterpret_cast<void **>(&d), ray_bytes + result_bytes));
+    WR_HIP(s->dev->alloc(reinterpret_cast<void **>(&d), ray_bytes + result_bytes));
     hipError_t e = s->dev->ring.upload(s->dev->ordinal, s->stream, d, rays, ray_bytes);
     char *d_out = d + ray_bytes;
     if (e == hipSuccess) {
