@@ -604,9 +604,7 @@ inline unsigned grid_of(uint64_t n) { return unsigned((n + kBB - 1) / kBB); }
 int bvh_gpu_plan(uint32_t n, uint32_t n_verts, hipStream_t stream, BuildArena *arena, BuildBuffers *b) {
     const size_t nn = 2 * size_t(n) - 1;
     const size_t node_cap = n;
-    arena->want(&b->verts, 3 * size_t(n_verts));
-    arena->want(&b->tris, 3 * size_t(n));
-    arena->want(&b->tri_geom, n);
+    arena->want(&b->verts, 3 * size_t(n_verts) + 4 * size_t(n));  // and behind them the triangles and their geometries
     arena->want(&b->partial, 6 * kBoundsBlocks);
     arena->want(&b->cbox, 6);
     arena->want(&b->flags32, 1);

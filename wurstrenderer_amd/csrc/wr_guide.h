@@ -299,7 +299,7 @@ __device__ __forceinline__ void tile_fwd(const u32x4 *ops, const float *bias, in
 #pragma unroll
     for (int v = 0; v < 16; v++) {
         const int o0 = 32 * mt + drow(v, 0);
-        acc[0][v] = o0 + 4 * h < N ? bb[o0] : 0.f;
+        acc[0][v] = o0 < N ? bb[o0] : 0.f;  // o0 + 4 h < N: N is a multiple of 8
     }
     acc[1] = acc[0];
 #pragma unroll
@@ -534,8 +534,8 @@ __device__ __forceinline__ void forward8(const Net &net, const Enc &mine, float 
         for (int v = 0; v < 16; v++) {
             const int o0 = 32 * mt + drow(v, 0);
             if (o0 < kOut) {
-                // this lane's row is o0 + 4 h (its bias bb[o0]); rows past kOut are padding
-                const float b = o0 + 4 * h < kOut ? bb[o0] : 0.f;
+                // this lane's row is o0 + 4 h (its bias bb[o0]), below kOut as o0 is: kOut is a multiple of 8
+                const float b = bb[o0];
                 float lo, hi;
                 rows_to_record(fmaf(acc[mt][0][v], ws * xs[0], b), fmaf(acc[mt][1][v], ws * xs[1], b), lo, hi);
                 out[o0] = lo;
@@ -545,21 +545,35 @@ __device__ __forceinline__ void forward8(const Net &net, const Enc &mine, float 
 }
 
 // ---------------------------------------------------------------- loss gradient
-// One record: loss = -w log q(wi).  Writes dloss/dout[40] to g (which may be
-// o itself) and returns the loss.  Computed in log space: lobes underflow far
-// from their axis.
-__device__ __forceinline__ float loss_grad(const float *o, float3 wi, float w, float *g) {
+// One record: loss = -w log q(wi).  Writes dloss/dout[40] over the outputs in row
+// o and returns the loss.  Computed in log space: lobes underflow far from their
+// axis.  Lanes p and p + 32 share a record and call it together, h = 0 and 1:
+// each does four of the lobes, and the sums over lobes are formed from all eight
+// in order, in both.
+static_assert(kLobes == 8, "half of the lobes per lane half");
+__device__ __forceinline__ void both_halves(const float mine[4], float all[8]) {
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        // swapping a register's upper half with its own lower half leaves one half's values in both
+        const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(mine[j]), __float_as_uint(mine[j]), false, false);
+        all[j] = __uint_as_float(sw[0]);
+        all[4 + j] = __uint_as_float(sw[1]);
+    }
+}
+__device__ __forceinline__ float loss_grad_half(float *row, float3 wi, float w, int h) {
     // hardware exp2 / log2 / reciprocal throughout (about 1 ulp each): the
     // outputs come from a BF16 network, so these errors are far below its own
+    float *o = row + 20 * h;
     float mx = -INFINITY;
-    for (int k = 0; k < kLobes; k++) mx = fmaxf(mx, o[5 * k]);
-    float s = 0.f;
-    for (int k = 0; k < kLobes; k++) s += fexp(o[5 * k] - mx);
+    for (int k = 0; k < kLobes; k++) mx = fmaxf(mx, row[5 * k]);
+    float e[4], all[kLobes], s = 0.f;
+    for (int k = 0; k < 4; k++) e[k] = fexp(o[5 * k] - mx);
+    both_halves(e, all);
+    for (int k = 0; k < kLobes; k++) s += all[k];
     const float lse = mx + flog(s);
-    float lc[kLobes], lam[kLobes], inv[kLobes], dl[kLobes], cs[kLobes];
-    float3 mu[kLobes];
-    float lq_max = -INFINITY;
-    for (int k = 0; k < kLobes; k++) {
+    float lw[4], lc[4], lam[4], inv[4], dl[4], cs[4];
+    float3 mu[4];
+    for (int k = 0; k < 4; k++) {
         const float3 a = f3(o[5 * k + 1], o[5 * k + 2], o[5 * k + 3]);
         const float n2 = dot3(a, a);
         inv[k] = n2 > 1e-24f ? __builtin_amdgcn_rsqf(n2) : 0.f;  // 1 / |a|, 0 for a degenerate axis
@@ -569,24 +583,29 @@ __device__ __forceinline__ float loss_grad(const float *o, float3 wi, float w, f
         lam[k] = fminf(fmaxf(sp, kLambdaMin), kLambdaMax);
         dl[k] = (sp > kLambdaMin && sp < kLambdaMax) ? frcp(1.f + fexp(-raw)) : 0.f;  // dlambda/draw
         cs[k] = dot3(mu[k], wi);
-        lc[k] = (o[5 * k] - lse) + log_vmf_norm_fast(lam[k]) + lam[k] * (cs[k] - 1.f);
-        lq_max = fmaxf(lq_max, lc[k]);
+        lw[k] = o[5 * k] - lse;
+        lc[k] = lw[k] + log_vmf_norm_fast(lam[k]) + lam[k] * (cs[k] - 1.f);
     }
+    both_halves(lc, all);
+    float lq_max = -INFINITY;
+    for (int k = 0; k < kLobes; k++) lq_max = fmaxf(lq_max, all[k]);
+    for (int k = 0; k < 4; k++) e[k] = fexp(lc[k] - lq_max);
+    both_halves(e, all);
     float sq = 0.f;
-    for (int k = 0; k < kLobes; k++) sq += fexp(lc[k] - lq_max);
+    for (int k = 0; k < kLobes; k++) sq += all[k];
     const float logq = lq_max + flog(sq);
-    for (int k = 0; k < kLobes; k++) {
+    for (int k = 0; k < 4; k++) {
         const float gam = fexp(lc[k] - logq);  // responsibility of lobe k
-        g[5 * k] = -w * (gam - fexp(o[5 * k] - lse));
+        o[5 * k] = -w * (gam - fexp(lw[k]));
         // d log c / d lambda = 1/lambda - 2 / (exp(2 lambda) - 1) + (mu.wi - 1)
         const float dlogc = frcp(lam[k]) - 2.f * frcp(fexp(2.f * lam[k]) - 1.f) + (cs[k] - 1.f);
-        g[5 * k + 4] = -w * gam * dlogc * dl[k];
+        o[5 * k + 4] = -w * gam * dlogc * dl[k];
         // d log c / d mu = lambda wi, through mu = a / |a| (zero for a degenerate axis)
         const float3 gm = wi * (gam * lam[k]);
         const float3 ga = (gm - mu[k] * dot3(mu[k], gm)) * inv[k];
-        g[5 * k + 1] = -w * ga.x;
-        g[5 * k + 2] = -w * ga.y;
-        g[5 * k + 3] = -w * ga.z;
+        o[5 * k + 1] = -w * ga.x;
+        o[5 * k + 2] = -w * ga.y;
+        o[5 * k + 3] = -w * ga.z;
     }
     return -w * logq;
 }

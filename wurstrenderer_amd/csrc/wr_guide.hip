@@ -2,7 +2,7 @@
 // its C-ABI (no reference counterpart; the reference has no guiding).
 //
 //   pack      FP32 master weights -> BF16 MFMA operands (forward and backward)
-//   train     per wave of 64 records: forward (MFMA), loss gradient, backward
+//   train     per wave of 32 records: forward (MFMA), loss gradient, backward
 //             data (MFMA) and weight gradients (MFMA over the records), summed
 //             per block in LDS and written as one partial per block
 //   adam      sums the block partials and applies Adam to the FP32 master
@@ -23,7 +23,6 @@ using namespace wr::guide;
 
 namespace {
 
-constexpr int kXt = 72;                  // LDS row stride (bf16) of the transposed tiles
 constexpr int kMaxTrainBlocks = 256;
 constexpr uint32_t kTestBlock = 64;
 
@@ -116,52 +115,98 @@ struct TrainArgs {
     float *loss;                        // [gridDim.x]
 };
 
-// Four waves per block (one per SIMD of a CU) step through the records in
-// lockstep, a tile of 64 per wave.  A wave keeps every layer's input operands
-// in registers (it has a SIMD's whole register file), so LDS holds the current
-// layer's transposed tiles (which the loss stage aliases), 4 x 18 KiB, and a
-// copy of the packed weights and biases, 69 KiB: at one wave per SIMD nothing
-// hides a load's latency, and LDS answers several times sooner than L2.  Each
-// 32 x 32 tile of a weight gradient belongs to one wave, which reduces it over
-// all four waves' staged tiles with MFMA and adds it into the block's slice of
-// the partial sums in global memory: one writer per address, no atomics.
-constexpr int kTrainWaves = 4;
+// Eight waves per block (two per SIMD of a CU) step through the records in
+// lockstep, a tile of 32 per wave.  A wave keeps every layer's input operands
+// in registers, so LDS holds the current layer's transposed tiles (which the
+// loss stage aliases), 8 x 10 KiB, and a copy of the packed weights and biases,
+// 69 KiB, which LDS answers several times sooner than L2; that is one block per
+// CU.  What bounds it is latency: a tile is one chain of MFMA, LDS and
+// transcendental steps, 7,400 cycles of matrix work in 67,000 when four waves
+// of 64 records ran it, one per SIMD; the second wave of a SIMD runs in the
+// gaps of the first (a step over 262,144 records: 112 -> 74 us, with the 32-bit
+// stores and branch-free loads below).  Tiles kept by record and read with the
+// transposing LDS loads took 100 us: twice the reads, each waited for.
+// Each 32 x 32 tile of a weight gradient belongs to one
+// wave, which reduces it over all eight waves' staged tiles with MFMA, in the
+// order of the records, and adds it into the block's slice of the partial sums
+// in global memory: one writer per address, no atomics.
+constexpr int kTrainWaves = 8, kTrainTile = 32;
+constexpr int kXt = kTrainTile + 8;  // row of a transposed tile: 16-byte aligned, 8 rows in distinct banks
 struct TrainLds {
     union {
         struct {
             uint16_t xt[64 * kXt];   // X_l^T of the current layer (BF16 bits): feature-major, records contiguous
             uint16_t dyt[64 * kXt];  // dY_l^T, likewise
         } t;
-        float stage[64 * kStageStride];  // raw outputs, then d loss / d outputs
+        float stage[kTrainTile * kStageStride];  // raw outputs, then d loss / d outputs
     };
 };
 
-// X^T of one layer's input operands into LDS (record-contiguous rows).
+// X^T of one layer's input operands into LDS (record-contiguous rows).  A lane
+// holds two features of one record in a word and its neighbour those of the
+// next record: they exchange words, the even lane stores the first feature of
+// both records and the odd lane the second, one 32-bit store for two 16-bit ones.
 // (Addresses are a per-lane base plus compile-time offsets, so they fold into
 // the LDS instructions' immediates instead of occupying registers.)
 template <int KS>
-__device__ __forceinline__ void store_xt(uint16_t *xt, const u32x4 (*x)[2]) {
-    const int lane = __lane_id(), p = lane & 31, h = lane >> 5;
-    uint16_t *base = xt + 4 * h * kXt + p;
+__device__ __forceinline__ void store_xt(uint16_t *xt, const u32x4 *x) {
+    const int lane = __lane_id(), p = lane & 31, h = lane >> 5, odd = lane & 1;
+    const uint32_t pick = odd ? 0x07060302u : 0x01000504u;
+    uint16_t *base = xt + (4 * h + odd) * kXt + (p & ~1);
 #pragma unroll
     for (int ks = 0; ks < KS; ks++)
 #pragma unroll
-        for (int nt = 0; nt < 2; nt++)
-#pragma unroll
-            for (int e = 0; e < 8; e++)
-                base[kperm(ks, 0, e) * kXt + 32 * nt] = uint16_t(x[ks][nt][e >> 1] >> (16 * (e & 1)));
+        for (int i = 0; i < 4; i++) {
+            const uint32_t mine = x[ks][i];
+            const uint32_t next = __builtin_amdgcn_update_dpp(0, mine, 0xB1 /* quad_perm 1 0 3 2 */, 0xF, 0xF, true);
+            *reinterpret_cast<uint32_t *>(base + kperm(ks, 0, 2 * i) * kXt) = __builtin_amdgcn_perm(mine, next, pick);
+        }
 }
 
-// Backward through layer l of the block's four tiles (one per wave).  dY_l
-// arrives as packed BF16 operands (dy[ks][nt] element e = dY of output
-// kperm(ks, h, e) of record 32 nt + p, the values every product below uses);
+// Both 32-output tiles of a layer for the wave's 32 records (tile_fwd for one
+// record tile): acc[mt] = b + (W_l^T X^T)[32 mt .. 32 mt + 31].
+template <int K>
+__device__ __forceinline__ void tiles_fwd(const u32x4 *ops, const float *bias, int N, const u32x4 *x, f32x16 acc[2]) {
+    const int lane = __lane_id(), h = lane >> 5;
+    const float *bb = bias + 4 * h;
+#pragma unroll
+    for (int mt = 0; mt < 2; mt++)
+#pragma unroll
+        for (int v = 0; v < 16; v++) {
+            const int o0 = 32 * mt + drow(v, 0);
+            acc[mt][v] = o0 < N ? bb[o0] : 0.f;
+        }
+#pragma unroll
+    for (int ks = 0; ks < K / 16; ks++)
+#pragma unroll
+        for (int mt = 0; mt < 2; mt++) acc[mt] = mfma(ops[(mt * (K / 16) + ks) * 64 + lane], x[ks], acc[mt]);
+}
+
+// One hidden layer of the wave's 32 records: input operands x (K inputs) ->
+// output operands xn (bias + ReLU, BF16).
+template <int K>
+__device__ __forceinline__ void layer_to(const Net &net, int l, const u32x4 *x, u32x4 xn[4]) {
+    f32x16 acc[2];
+    tiles_fwd<K>(net.fwd + fwd_offset(l), net.bias + 64 * l, kHid, x, acc);
+#pragma unroll
+    for (int mt = 0; mt < 2; mt++)
+#pragma unroll
+        for (int kk = 0; kk < 2; kk++)
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                xn[2 * mt + kk][i] = pack2_relu(acc[mt][8 * kk + 2 * i], acc[mt][8 * kk + 2 * i + 1]);
+}
+
+// Backward through layer l of the block's eight tiles (one per wave).  dY_l
+// arrives as packed BF16 operands (dy[ks] element e = dY of output
+// kperm(ks, h, e) of record p, the values every product below uses);
 // the layer's input operands are in x.  Adds dW_l and db_l into grad (stores
 // them when first) and, for
 // l > 0, leaves dY_{l-1} (the input's ReLU mask applied) packed in dy.  Every
 // wave of the block calls it together (block barriers inside).
 template <int l>
-__device__ __forceinline__ void backward_layer(const Net &net, TrainLds *wl, float *grad, bool first, float (*bpart)[64],
-                                               const u32x4 (*x)[2], u32x4 dy[4][2]) {
+__device__ __forceinline__ void backward_layer(const Net &net, TrainLds *wl, float *grad, bool first, const u32x4 *x,
+                                               u32x4 dy[4]) {
     constexpr int K = layer_in(l), N = layer_out(l);
     const int lane = __lane_id(), p = lane & 31, h = lane >> 5, wave = threadIdx.x >> 6;
     TrainLds &L = wl[wave];
@@ -173,29 +218,19 @@ __device__ __forceinline__ void backward_layer(const Net &net, TrainLds *wl, flo
     const int mt = wave >> 1, nt = wave & 1;
     const bool mine = wave < kTiles && 32 * nt + p < N;
     float *gb = grad + w_offset(l) + (32 * mt + 4 * h) * N + 32 * nt + p;
-    f32x16 acc;
+    f32x16 acc = f32x16{};
+    if (mine && !first) {
 #pragma unroll
-    for (int v = 0; v < 16; v++) acc[v] = !first && mine ? gb[drow(v, 0) * N] : 0.f;
+        for (int v = 0; v < 16; v++) acc[v] = gb[drow(v, 0) * N];
+    }
     store_xt<4>(L.t.dyt, dy);
     store_xt<K / 16>(L.t.xt, x);
-    wave_sync_lds();
-    // this wave's share of the bias gradient: row sums of its dY^T
-    if (lane < N) {
-        float s[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int r = 0; r < 64; r += 8) {
-            const u32x4 v = *reinterpret_cast<const u32x4 *>(L.t.dyt + lane * kXt + r);
-#pragma unroll
-            for (int i = 0; i < 4; i++) s[i] = add_halves(v[i], s[i]);
-        }
-        bpart[wave][lane] = (s[0] + s[1]) + (s[2] + s[3]);
-    }
     __syncthreads();
     if (wave < kTiles) {
 #pragma unroll
         for (int w2 = 0; w2 < kTrainWaves; w2++)
 #pragma unroll
-            for (int ks = 0; ks < 4; ks++) {
+            for (int ks = 0; ks < kTrainTile / 16; ks++) {
                 const u32x4 av = *reinterpret_cast<const u32x4 *>(wl[w2].t.xt + (32 * mt + p) * kXt + 16 * ks + 8 * h);
                 const u32x4 bv = *reinterpret_cast<const u32x4 *>(wl[w2].t.dyt + (32 * nt + p) * kXt + 16 * ks + 8 * h);
                 acc = mfma(av, bv, acc);
@@ -205,54 +240,44 @@ __device__ __forceinline__ void backward_layer(const Net &net, TrainLds *wl, flo
             for (int v = 0; v < 16; v++) gb[drow(v, 0) * N] = acc[v];
         }
     }
-    // bias: the wave with no weight tile for layer 0, else one per layer in turn
-    if (wave == (kTiles == 2 ? 2 : l & 3) && lane < N) {
-        const float s = (bpart[0][lane] + bpart[1][lane]) + (bpart[2][lane] + bpart[3][lane]);
+    // bias gradient: row sums of the dY^T tiles, per 64 records; a wave with no
+    // weight tile, another one for each layer
+    if (wave == 4 + (l & 3) && lane < N) {
+        float part[4];
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            float s[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int r = 0; r < 64; r += 8) {
+                const u32x4 v = *reinterpret_cast<const u32x4 *>(wl[2 * q + r / kTrainTile].t.dyt + lane * kXt + r % kTrainTile);
+#pragma unroll
+                for (int i = 0; i < 4; i++) s[i] = add_halves(v[i], s[i]);
+            }
+            part[q] = (s[0] + s[1]) + (s[2] + s[3]);
+        }
+        const float s = (part[0] + part[1]) + (part[2] + part[3]);
         grad[b_offset(l) + lane] = first ? s : grad[b_offset(l) + lane] + s;
     }
     if constexpr (l > 0) {
         // backward data: dX^T = W_l dY^T; the input's ReLU mask sits in the same lane
         // and slot as the result, which is packed into dy for the layer below
         const u32x4 *ops = net.bwd + bwd_offset(l);
-        u32x4 nd[4][2];
-#pragma unroll
-        for (int mt = 0; mt < 2; mt++) {
-            f32x16 d0 = f32x16{}, d1 = f32x16{};
-#pragma unroll
-            for (int ks = 0; ks < 4; ks++) {
-                const u32x4 av = ops[(mt * 4 + ks) * 64 + lane];
-                d0 = mfma(av, dy[ks][0], d0);
-                d1 = mfma(av, dy[ks][1], d1);
-            }
-#pragma unroll
-            for (int v = 0; v < 16; v += 2) {
-                // ReLU outputs are >= 0: the mask is "BF16 bits non-zero"
-                const u32x4 &m0 = x[2 * mt + (v >> 3)][0], &m1 = x[2 * mt + (v >> 3)][1];
-                const int w = (v & 7) >> 1;
-                const float a0 = (m0[w] & 0xFFFFu) ? d0[v] : 0.f, b0 = (m0[w] >> 16) ? d0[v + 1] : 0.f;
-                const float a1 = (m1[w] & 0xFFFFu) ? d1[v] : 0.f, b1 = (m1[w] >> 16) ? d1[v + 1] : 0.f;
-                nd[2 * mt + (v >> 3)][0][w] = pack2(a0, b0);
-                nd[2 * mt + (v >> 3)][1][w] = pack2(a1, b1);
-            }
-        }
+        f32x16 d[2] = {f32x16{}, f32x16{}};
 #pragma unroll
         for (int ks = 0; ks < 4; ks++)
 #pragma unroll
-            for (int nt = 0; nt < 2; nt++) dy[ks][nt] = nd[ks][nt];
+            for (int mt = 0; mt < 2; mt++) d[mt] = mfma(ops[(mt * 4 + ks) * 64 + lane], dy[ks], d[mt]);
+#pragma unroll
+        for (int mt = 0; mt < 2; mt++)
+#pragma unroll
+            for (int v = 0; v < 16; v += 2) {
+                // ReLU outputs are >= 0: the mask is "BF16 bits non-zero"
+                const int w = (v & 7) >> 1;
+                const uint32_t m = x[2 * mt + (v >> 3)][w];
+                dy[2 * mt + (v >> 3)][w] = pack2((m & 0xFFFFu) ? d[mt][v] : 0.f, (m >> 16) ? d[mt][v + 1] : 0.f);
+            }
     }
     __syncthreads();  // every wave's tiles are read before the next layer (or record tile) overwrites them
-}
-
-// One hidden layer of the wave's 64 records: input operands x (K inputs) ->
-// output operands xn (bias + ReLU, BF16).
-template <int K>
-__device__ __forceinline__ void layer_to(const Net &net, int l, const u32x4 (*x)[2], u32x4 xn[4][2]) {
-#pragma unroll
-    for (int mt = 0; mt < 2; mt++) {
-        f32x16 acc[2];
-        tile_fwd<K>(net.fwd + fwd_offset(l), net.bias + 64 * l, kHid, x, mt, acc);
-        tile_to_operands(acc, mt, xn);
-    }
 }
 
 __global__ __launch_bounds__(64 * kTrainWaves) void k_train(Net gnet, TrainArgs a) {
@@ -260,8 +285,8 @@ __global__ __launch_bounds__(64 * kTrainWaves) void k_train(Net gnet, TrainArgs 
     __shared__ __attribute__((aligned(16))) u32x4 wfwd[kFwdOps];
     __shared__ __attribute__((aligned(16))) u32x4 wbwd[kBwdOps];
     __shared__ float wbias[kBiasPacked];
-    __shared__ float bpart[kTrainWaves][64];
-    __shared__ float wave_loss[kTrainWaves];
+    __shared__ float lane_loss[kTrainWaves * kTrainTile];
+    __shared__ float wave_loss[kTrainWaves / 2];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, p = lane & 31, h = lane >> 5;
     for (int j = threadIdx.x; j < kFwdOps; j += blockDim.x) wfwd[j] = gnet.fwd[j];
     for (int j = threadIdx.x; j < kBwdOps; j += blockDim.x) wbwd[j] = gnet.bwd[j];
@@ -274,11 +299,12 @@ __global__ __launch_bounds__(64 * kTrainWaves) void k_train(Net gnet, TrainArgs 
     float *grad = a.partials + size_t(blockIdx.x) * kNumParams;
     TrainLds &L = wl[wave];
     float loss = 0.f;
-    const uint32_t tiles = (a.batch + 63) / 64;
-    // groups of kTrainWaves tiles; every wave runs every group (the block
-    // synchronises inside the backward pass), a tile past the end as 64 invalid records
-    for (uint32_t group = blockIdx.x; group * kTrainWaves < tiles; group += gridDim.x) {
-        const uint32_t jr = (group * kTrainWaves + wave) * 64 + lane;
+    constexpr uint32_t kGroup = kTrainWaves * kTrainTile;
+    const uint32_t groups = (a.batch + kGroup - 1) / kGroup;
+    // every wave runs every group (the block synchronises inside the backward
+    // pass), records past the end as invalid ones
+    for (uint32_t group = blockIdx.x; group < groups; group += gridDim.x) {
+        const uint32_t jr = group * kGroup + wave * kTrainTile + p;
         const bool first = group == blockIdx.x;
         const bool valid = jr < a.batch;
         Enc enc;
@@ -296,80 +322,83 @@ __global__ __launch_bounds__(64 * kTrainWaves) void k_train(Net gnet, TrainArgs 
         }
         // forward; the inputs of layers 0, 2 and 4 stay in registers (checkpoints),
         // those of layers 1 and 3 are recomputed during the backward pass
-        u32x4 x0[2][2], x2[4][2], x4[4][2];
-        input_operands(enc, x0);
+        u32x4 x0[2], x2[4], x4[4];
+#pragma unroll
+        for (int ks = 0; ks < 2; ks++)
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                x0[ks][i] = pack2(feature_h(enc, kperm(ks, 0, 2 * i), h), feature_h(enc, kperm(ks, 0, 2 * i + 1), h));
         {
-            u32x4 x1[4][2];
+            u32x4 x1[4];
             layer_to<kIn>(net, 0, x0, x1);
             layer_to<kHid>(net, 1, x1, x2);
         }
         {
-            u32x4 x3[4][2];
+            u32x4 x3[4];
             layer_to<kHid>(net, 2, x2, x3);
             layer_to<kHid>(net, 3, x3, x4);
         }
-#pragma unroll
-        for (int mt = 0; mt < 2; mt++) {
+        {
             f32x16 acc[2];
-            tile_fwd<kHid>(net.fwd + fwd_offset(4), net.bias + 64 * 4, kOut, x4, mt, acc);
+            tiles_fwd<kHid>(net.fwd + fwd_offset(4), net.bias + 64 * 4, kOut, x4, acc);
             float *sb = L.stage + p * kStageStride + 4 * h;
 #pragma unroll
-            for (int v = 0; v < 16; v++) {
-                const int o0 = 32 * mt + drow(v, 0);
-                if (o0 + 4 * h < kOut) {
-                    sb[o0] = acc[0][v];
-                    sb[32 * kStageStride + o0] = acc[1][v];
+            for (int mt = 0; mt < 2; mt++)
+#pragma unroll
+                for (int v = 0; v < 16; v++) {
+                    const int o0 = 32 * mt + drow(v, 0);
+                    if (o0 < kOut) sb[o0] = acc[mt][v];
                 }
-            }
         }
         wave_sync_lds();
-        // loss gradient of this lane's record, written over its outputs
+        // loss gradient of the record, written over its outputs, half of the lobes in each lane half
         {
-            float *row = L.stage + lane * kStageStride;
-            const float l = loss_grad(row, wi, w, row);
+            const float l = loss_grad_half(L.stage + p * kStageStride, wi, w, h);
             if (valid) loss += l;
             else
-                for (int k = 0; k < kOut; k++) row[k] = 0.f;
+                for (int k = 0; k < kOut / 2; k++) L.stage[p * kStageStride + kOut / 2 * h + k] = 0.f;
         }
         wave_sync_lds();
-        // dY_4 as packed operands: element e of dy[ks][nt] is output kperm(ks, h, e) of record 32 nt + p
-        u32x4 dacc[4][2];
+        // dY_4 as packed operands: element e of dy[ks] is output kperm(ks, h, e) of record p
+        u32x4 dacc[4];
         {
             const float *sb = L.stage + p * kStageStride + 4 * h;
 #pragma unroll
             for (int ks = 0; ks < 4; ks++)
 #pragma unroll
-                for (int nt = 0; nt < 2; nt++)
-#pragma unroll
-                    for (int i = 0; i < 4; i++) {
-                        // output kperm(ks, h, e) = kperm(ks, 0, e) + 4 h; outputs >= 40 are padding
-                        const int o0 = kperm(ks, 0, 2 * i), o1 = kperm(ks, 0, 2 * i + 1);
-                        const float v0 = o0 + 4 * h < kOut ? sb[32 * nt * kStageStride + o0] : 0.f;
-                        const float v1 = o1 + 4 * h < kOut ? sb[32 * nt * kStageStride + o1] : 0.f;
-                        dacc[ks][nt][i] = pack2(v0, v1);
-                    }
+                for (int i = 0; i < 4; i++) {
+                    // output kperm(ks, h, e) = kperm(ks, 0, e) + 4 h; outputs >= 40 are padding
+                    const int o0 = kperm(ks, 0, 2 * i), o1 = kperm(ks, 0, 2 * i + 1);
+                    dacc[ks][i] = pack2(o0 < kOut ? sb[o0] : 0.f, o1 < kOut ? sb[o1] : 0.f);
+                }
         }
         wave_sync_lds();  // the stage is read before the transposed tiles overwrite it
-        backward_layer<4>(net, wl, grad, first, bpart, x4, dacc);
+        backward_layer<4>(net, wl, grad, first, x4, dacc);
         {
-            u32x4 x3[4][2];
+            u32x4 x3[4];
             layer_to<kHid>(net, 2, x2, x3);
-            backward_layer<3>(net, wl, grad, first, bpart, x3, dacc);
+            backward_layer<3>(net, wl, grad, first, x3, dacc);
         }
-        backward_layer<2>(net, wl, grad, first, bpart, x2, dacc);
+        backward_layer<2>(net, wl, grad, first, x2, dacc);
         {
-            u32x4 x1[4][2];
+            u32x4 x1[4];
             layer_to<kIn>(net, 0, x0, x1);
-            backward_layer<1>(net, wl, grad, first, bpart, x1, dacc);
+            backward_layer<1>(net, wl, grad, first, x1, dacc);
         }
-        backward_layer<0>(net, wl, grad, first, bpart, x0, dacc);
+        backward_layer<0>(net, wl, grad, first, x0, dacc);
     }
-    for (int off = 32; off > 0; off >>= 1) loss += __shfl_xor(loss, off);
-    if (lane == 0) wave_loss[wave] = loss;
+    // both lane halves hold their record's loss: summed over 64 records, then over the block
+    if (h == 0) lane_loss[wave * kTrainTile + p] = loss;
+    __syncthreads();
+    if (threadIdx.x < kTrainWaves * kTrainTile) {
+        loss = lane_loss[threadIdx.x];
+        for (int off = 32; off > 0; off >>= 1) loss += __shfl_xor(loss, off);
+        if (lane == 0) wave_loss[wave] = loss;
+    }
     __syncthreads();
     if (threadIdx.x == 0) {
         float s = 0.f;
-        for (int k = 0; k < kTrainWaves; k++) s += wave_loss[k];
+        for (int k = 0; k < kTrainWaves / 2; k++) s += wave_loss[k];
         a.loss[blockIdx.x] = s;
     }
 }
@@ -419,6 +448,22 @@ __global__ __launch_bounds__(kAdamBlock) void k_adam(AdamArgs a) {
     const float p = a.params[j] - a.lr_t * m / (sqrtf(v) + a.eps_t);
     a.params[j] = p;
     if (a.avg) a.avg[j] = a.avg_decay * a.avg[j] + (1.f - a.avg_decay) * p;
+}
+
+// ---------------------------------------------------------------- unpack
+// Records from host arrays: raw holds pos, nrm, wo, wi (3 floats a record) and
+// the weights one behind the other; out holds pos, nrm, wo and (wi, weight) as
+// float4 arrays.  Bound by memory (30 MB, 10 us at 262144 records), where packing
+// on one host thread and the copy of the packed array took 1.0 ms; with the
+// arrays' own upload it is 0.45 ms.
+__global__ __launch_bounds__(256) void k_unpack(const float *raw, uint32_t n, float4 *out) {
+    const uint32_t r = blockIdx.x * 256 + threadIdx.x;
+    if (r >= n) return;
+    const size_t N = n;
+    for (int k = 0; k < 4; k++) {
+        const float *v = raw + 3 * (k * N + r);
+        out[k * N + r] = make_float4(v[0], v[1], v[2], k == 3 ? raw[12 * N + r] : 0.f);
+    }
 }
 
 // ---------------------------------------------------------------- finalize
@@ -608,8 +653,8 @@ int train_step(wr_guide *g, const float4 *pos, const float4 *nrm, const float4 *
     a.n = n; a.start = start; a.batch = batch; a.wscale = wscale;
     a.partials = g->d_partials;
     a.loss = g->d_loss;
-    const int tiles = int((batch + 63) / 64);
-    const int blocks = std::max(1, std::min((tiles + kTrainWaves - 1) / kTrainWaves, g->train_blocks));
+    constexpr uint32_t kGroup = kTrainWaves * kTrainTile;
+    const int blocks = std::max(1, std::min(int((batch + kGroup - 1) / kGroup), g->train_blocks));
     k_train<<<blocks, 64 * kTrainWaves, 0, st>>>(net_view(g), a);
     WR_HIP(hipGetLastError());
     g->last_blocks = blocks;
@@ -650,23 +695,21 @@ int train_step(wr_guide *g, const float4 *pos, const float4 *nrm, const float4 *
     return WR_OK;
 }
 
-// Host records -> temporary device arrays (float4 each).
+// Host records -> temporary device arrays (float4 each): the caller's arrays go
+// up as they are and k_unpack spreads them.
 struct DeviceRecords {
     float4 *buf = nullptr;
     float4 *pos = nullptr, *nrm = nullptr, *wo = nullptr, *wi = nullptr;
     ~DeviceRecords() { if (buf) (void)hipFree(buf); }
-    int upload(hipStream_t st, const float *p, const float *nr, const float *o, const float *i, const float *w, uint32_t n) {
-        std::vector<float4> h(4 * size_t(n));
-        for (uint32_t r = 0; r < n; r++) {
-            h[r] = make_float4(p[3 * r], p[3 * r + 1], p[3 * r + 2], 0.f);
-            h[n + r] = make_float4(nr[3 * r], nr[3 * r + 1], nr[3 * r + 2], 0.f);
-            h[2 * size_t(n) + r] = make_float4(o[3 * r], o[3 * r + 1], o[3 * r + 2], 0.f);
-            h[3 * size_t(n) + r] = make_float4(i[3 * r], i[3 * r + 1], i[3 * r + 2], w[r]);
-        }
-        WR_HIP(hipMalloc(reinterpret_cast<void **>(&buf), sizeof(float4) * h.size()));
-        WR_HIP(hipMemcpyAsync(buf, h.data(), sizeof(float4) * h.size(), hipMemcpyHostToDevice, st));
-        WR_HIP(hipStreamSynchronize(st));
+    int upload(wr_device *dev, hipStream_t st, const float *p, const float *nr, const float *o, const float *i,
+               const float *w, uint32_t n) {
+        const size_t row = 3 * sizeof(float) * size_t(n), raw = 4 * row + sizeof(float) * size_t(n);
+        WR_HIP(dev->alloc(reinterpret_cast<void **>(&buf), 4 * sizeof(float4) * size_t(n) + raw));
         pos = buf; nrm = buf + n; wo = buf + 2 * size_t(n); wi = buf + 3 * size_t(n);
+        float *d_raw = reinterpret_cast<float *>(buf + 4 * size_t(n));
+        WR_HIP(dev->ring.upload(dev->ordinal, st, d_raw, {{p, row}, {nr, row}, {o, row}, {i, row}, {w, raw - 4 * row}}));
+        k_unpack<<<(n + 255) / 256, 256, 0, st>>>(d_raw, n, buf);
+        WR_HIP(hipGetLastError());
         return WR_OK;
     }
 };
@@ -994,7 +1037,7 @@ int wr_guide_gradient(wr_guide *g, const float *pos, const float *nrm, const flo
     if (rc) return rc;
     if (n == 0) return set_error(WR_ERR_INVALID_ARGUMENT, "no records");
     DeviceRecords dr;
-    rc = dr.upload(g->scene->stream, pos, nrm, wo, wi, weight, n);
+    rc = dr.upload(g->scene->dev, g->scene->stream, pos, nrm, wo, wi, weight, n);
     if (rc) return rc;
     float *dg = nullptr;
     WR_HIP(hipMalloc(reinterpret_cast<void **>(&dg), sizeof(float) * kNumParams));
@@ -1018,7 +1061,7 @@ int wr_guide_train(wr_guide *g, const float *pos, const float *nrm, const float 
     if (rc) return rc;
     if (n == 0) return set_error(WR_ERR_INVALID_ARGUMENT, "no records");
     DeviceRecords dr;
-    rc = dr.upload(g->scene->stream, pos, nrm, wo, wi, weight, n);
+    rc = dr.upload(g->scene->dev, g->scene->stream, pos, nrm, wo, wi, weight, n);
     if (rc) return rc;
     for (uint32_t k = 0; k < steps; k++) {
         rc = train_step(g, dr.pos, dr.nrm, dr.wo, dr.wi, n, 0, n, 1.f / float(n), nullptr,

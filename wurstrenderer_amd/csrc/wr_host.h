@@ -302,8 +302,8 @@ struct BuildArena {
 };
 // The build's arrays, all in a BuildArena.
 struct BuildBuffers {
-    float *verts;                  // the mesh
-    uint32_t *tris, *tri_geom;
+    float *verts;                  // the mesh: one array, so that it goes up in one transfer
+    uint32_t *tris, *tri_geom;     // inside it, set by the caller of bvh_gpu_plan after commit()
     float *partial, *cbox;         // bounds: per block, then min xyz and max xyz
     uint32_t *flags32;             // [0]: the mesh is invalid
     uint64_t *keys, *keys2, *flags, *incl;

@@ -1916,10 +1916,12 @@ static int bvh_gpu(wr_scene *s, const wr_scene_desc *d) {
         BuildBuffers b{};
         if ((rc = bvh_gpu_plan(n, d->n_verts, s->stream, &arena, &b))) return rc;
         WR_HIP(arena.commit());
-        TransferRing &ring = s->dev->ring;
-        WR_HIP(ring.upload(s->dev->ordinal, s->stream, b.verts, d->verts, sizeof(float) * 3 * size_t(d->n_verts)));
-        WR_HIP(ring.upload(s->dev->ordinal, s->stream, b.tris, d->tris, sizeof(uint32_t) * 3 * size_t(n)));
-        WR_HIP(ring.upload(s->dev->ordinal, s->stream, b.tri_geom, d->tri_geom, sizeof(uint32_t) * size_t(n)));
+        b.tris = reinterpret_cast<uint32_t *>(b.verts + 3 * size_t(d->n_verts));
+        b.tri_geom = b.tris + 3 * size_t(n);
+        WR_HIP(s->dev->ring.upload(s->dev->ordinal, s->stream, b.verts,
+                                   {{d->verts, sizeof(float) * 3 * size_t(d->n_verts)},
+                                    {d->tris, sizeof(uint32_t) * 3 * size_t(n)},
+                                    {d->tri_geom, sizeof(uint32_t) * size_t(n)}}));
         bool valid = false;
         if ((rc = mesh_check_gpu(b, n, d->n_verts, d->n_geoms, s->stream, &valid, s->box))) return rc;
         if (!valid) {  // the host checks name the fault

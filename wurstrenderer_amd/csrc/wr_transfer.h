@@ -21,6 +21,7 @@
 #include <atomic>
 #include <cstring>
 #include <exception>
+#include <initializer_list>
 #include <mutex>
 #include <thread>
 #include <vector>
@@ -54,17 +55,30 @@ struct TransferRing {
         return run(ordinal, stream, bytes, true, issue,
                    [out](size_t off, size_t n, char *slot) { std::memcpy(out + off, slot, n); });
     }
-    // Host to device on `stream`; src may be reused when it returns, and the
-    // copies are complete.
-    hipError_t upload(int ordinal, hipStream_t stream, void *device, const void *src, size_t bytes) {
-        const char *in = static_cast<const char *>(src);
+    // Host to device on `stream`: the parts, one behind the other.  The sources
+    // may be reused when it returns, and the copies are complete.
+    struct Part { const void *src; size_t bytes; };
+    hipError_t upload(int ordinal, hipStream_t stream, void *device, std::initializer_list<Part> parts) {
         char *out = static_cast<char *>(device);
+        size_t total = 0;
+        for (const Part &p : parts) total += p.bytes;
         return run(
-            ordinal, stream, bytes, false,
+            ordinal, stream, total, false,
             [out, stream](size_t off, size_t n, char *slot) {
                 return hipMemcpyAsync(out + off, slot, n, hipMemcpyHostToDevice, stream);
             },
-            [in](size_t off, size_t n, char *slot) { std::memcpy(slot, in + off, n); });
+            [&parts](size_t off, size_t n, char *slot) {
+                for (const Part &p : parts) {  // the piece of each part that lies in [off, off + n)
+                    const size_t m = off < p.bytes ? std::min(n, p.bytes - off) : 0;
+                    if (m) std::memcpy(slot, static_cast<const char *>(p.src) + off, m);
+                    slot += m;
+                    n -= m;
+                    off = off < p.bytes ? 0 : off - p.bytes;
+                }
+            });
+    }
+    hipError_t upload(int ordinal, hipStream_t stream, void *device, const void *src, size_t bytes) {
+        return upload(ordinal, stream, device, {Part{src, bytes}});
     }
 
 private:
