@@ -319,6 +319,14 @@ __device__ __forceinline__ float3 primary_dir(const DCamera &cam, uint32_t key, 
     return primary_dir_u(cam, u01(key, kDimPixel), u01(key, kDimPixel + 1), px, py, lens, pdfW);
 }
 
+// A path vertex's outcome: the shadow ray it sends (origin and length, direction
+// and target, contribution and job) and the ray that continues the path.
+struct Vertex {
+    float4 so = make_float4(0, 0, 0, 0), sd = so, sc = so;
+    float4 o = so, d = so, thr = so;
+    bool shadow = false, cont = false;
+};
+
 // ============================================================== regenerate
 // Fills the pool behind the continuing paths with the next unclaimed samples:
 // createLightSubpath + createCameraSubpath up to the first ray, with the t = 1
@@ -328,6 +336,85 @@ __device__ __forceinline__ float3 primary_dir(const DCamera &cam, uint32_t key, 
 // generalsubpathsampler.h:185-268): its light vertex connects to the camera
 // with weight 1, and its first ray leaves the light in a cosine-distributed
 // direction (DiffuseAreaLight::sampleLe1CosByPdf, contribution 1).
+template <bool ENV>
+__device__ __forceinline__ void start_path(const DScene &s, const RenderArgs &a, int use_mis, uint32_t key, uint32_t px,
+                                           uint32_t py, uint32_t job, Vertex &out) {
+    const DCamera &cam = s.cam;
+    // camera vertex (sampleWe0ByPdf)
+    const float3 lens = lens_point(cam, key);
+    const float3 cpos = cam_to_world(cam, lens) + f3(cam.ox, cam.oy, cam.oz);
+    const float3 cz = f3(cam.zx, cam.zy, cam.zz);
+    // t = 1 connection
+    const LightSample l = sample_light<ENV>(s, u01(key, kDimLight), u01(key, kDimLight + 1), key);
+    if (ENV && a.nee && l.env) {
+        // an envmap vertex: the camera looks along its direction; G = |cos| at
+        // the camera only, Le1 = 1, visibility to infinity (path.h:64-76, scene.h:98-101)
+        const float3 d = l.pos;
+        const float G = fabsf(dot3(cz, d));
+        float rx = 0.f, ry = 0.f;
+        const float we1 = G != 0.f ? camera_we1(cam, lens, d, rx, ry) : 0.f;
+        if (we1 != 0.f) {
+            float mis = 1.f;
+            if (use_mis) {
+                const float c = cam_to_local(cam, d).z;
+                const float camPdfA = cam.per_pixel_norm / (c * c * c);
+                mis = l.pdfA / (l.pdfA + camPdfA);
+            }
+            const float3 c = l.contrib * (mis * we1 * G);
+            if (!is_black(c)) {
+                const uint32_t target = kToSplat | (uint32_t(ry) * uint32_t(cam.W) + uint32_t(rx));
+                out.so = make_float4(cpos.x, cpos.y, cpos.z, INFINITY);
+                out.sd = make_float4(d.x, d.y, d.z, __uint_as_float(target));
+                out.sc = make_float4(c.x, c.y, c.z, __uint_as_float(job));
+                out.shadow = true;
+            }
+        }
+    } else if (a.nee || a.light) {
+        const float3 uv = cpos - l.pos;
+        const float len2 = dot3(uv, uv);
+        const float len = sqrtf(len2);
+        const float3 nuv = uv * (1.0f / len);
+        const float cos_l = dot3(l.n, nuv);
+        const float G = fabsf(cos_l) * fabsf(dot3(cz, nuv)) / len2;
+        if (G != 0.f && cos_l >= 0.f) {
+            float rx, ry;
+            const float3 wcam = -nuv;
+            const float we1 = camera_we1(cam, lens, wcam, rx, ry);
+            if (we1 != 0.f) {
+                float mis = 1.f;
+                if (use_mis) {
+                    const float c = cam_to_local(cam, wcam).z;
+                    float camPdfA = cam.per_pixel_norm / (c * c * c) * fabsf(cos_l) / len2;
+                    if (s.med.on) camPdfA *= pass_pdf(s.med, len);
+                    mis = l.pdfA / (l.pdfA + camPdfA);
+                }
+                const float k = mis * we1 * G * kInvPi;
+                float3 c = l.contrib * k;
+                if (s.med.on) c = c * transmittance(s.med, len);  // attenuated connection
+                const uint32_t target = kToSplat | (uint32_t(ry) * uint32_t(cam.W) + uint32_t(rx));
+                out.so = make_float4(l.pos.x, l.pos.y, l.pos.z, len - kRayEps);
+                out.sd = make_float4(nuv.x, nuv.y, nuv.z, __uint_as_float(target));
+                out.sc = make_float4(c.x, c.y, c.z, __uint_as_float(job));
+                out.shadow = true;
+            }
+        }
+    }
+    if (a.light) {
+        // the light subpath's first ray (pdf not needed: no MIS)
+        const float3 dir =
+            to_world(make_frame(l.n), cosine_hemisphere(u01(key, kDimPixel), u01(key, kDimPixel + 1)));
+        out.o = make_float4(l.pos.x, l.pos.y, l.pos.z, 0.f);
+        out.d = make_float4(dir.x, dir.y, dir.z, 0.f);
+        out.thr = make_float4(l.contrib.x, l.contrib.y, l.contrib.z, 0.f);
+    } else {
+        // primary ray (samplePerPixelWe1CosByPdf)
+        float pdfW;
+        const float3 dir = primary_dir(cam, key, px, py, lens, pdfW);
+        out.o = make_float4(cpos.x, cpos.y, cpos.z, 0.f);
+        out.d = make_float4(dir.x, dir.y, dir.z, 0.f);
+        out.thr = make_float4(1.f, 1.f, 1.f, use_mis ? pdfW : 0.f);
+    }
+}
 template <bool BATCH, bool ENV = false>
 __global__ __launch_bounds__(kShadeBlock) void k_regen(DScene s1, const BatchJob *__restrict__ jobs, uint32_t n_jobs,
                                                        PathBuffers pb, RenderArgs a) {
@@ -340,9 +427,7 @@ __global__ __launch_bounds__(kShadeBlock) void k_regen(DScene s1, const BatchJob
         const uint32_t i = base + threadIdx.x;
         const bool fresh = i < fresh_n;
         const uint32_t sidx = sbase + i;
-        bool splat = false;
-        float4 so = make_float4(0, 0, 0, 0), sd = so, sc = so;
-        float4 ro = so, rdir = so, thr = so;
+        Vertex v;
         uint32_t job = 0;
         if (fresh) {
             uint32_t local = sidx, wh = a.wh, first = a.first_sample, seed = a.seed;
@@ -362,97 +447,24 @@ __global__ __launch_bounds__(kShadeBlock) void k_regen(DScene s1, const BatchJob
             const uint32_t sample = first + local / wh;
             const uint32_t px = pixel % uint32_t(cam.W), py = pixel / uint32_t(cam.W);
             const uint32_t key = path_key(seed, pixel, sample);
-            // camera vertex (sampleWe0ByPdf)
-            const float3 lens = lens_point(cam, key);
-            const float3 cpos = cam_to_world(cam, lens) + f3(cam.ox, cam.oy, cam.oz);
-            const float3 cz = f3(cam.zx, cam.zy, cam.zz);
-            // t = 1 connection
-            const LightSample l = sample_light<ENV>(s, u01(key, kDimLight), u01(key, kDimLight + 1), key);
-            if (ENV && a.nee && l.env) {
-                // an envmap vertex: the camera looks along its direction; G = |cos| at
-                // the camera only, Le1 = 1, visibility to infinity (path.h:64-76, scene.h:98-101)
-                const float3 d = l.pos;
-                const float G = fabsf(dot3(cz, d));
-                float rx = 0.f, ry = 0.f;
-                const float we1 = G != 0.f ? camera_we1(cam, lens, d, rx, ry) : 0.f;
-                if (we1 != 0.f) {
-                    float mis = 1.f;
-                    if (use_mis) {
-                        const float c = cam_to_local(cam, d).z;
-                        const float camPdfA = cam.per_pixel_norm / (c * c * c);
-                        mis = l.pdfA / (l.pdfA + camPdfA);
-                    }
-                    const float3 c = l.contrib * (mis * we1 * G);
-                    if (!is_black(c)) {
-                        const uint32_t target = kToSplat | (uint32_t(ry) * uint32_t(cam.W) + uint32_t(rx));
-                        so = make_float4(cpos.x, cpos.y, cpos.z, INFINITY);
-                        sd = make_float4(d.x, d.y, d.z, __uint_as_float(target));
-                        sc = make_float4(c.x, c.y, c.z, __uint_as_float(job));
-                        splat = true;
-                    }
-                }
-            } else if (a.nee || a.light) {
-                const float3 uv = cpos - l.pos;
-                const float len2 = dot3(uv, uv);
-                const float len = sqrtf(len2);
-                const float3 nuv = uv * (1.0f / len);
-                const float cos_l = dot3(l.n, nuv);
-                const float G = fabsf(cos_l) * fabsf(dot3(cz, nuv)) / len2;
-                if (G != 0.f && cos_l >= 0.f) {
-                    float rx, ry;
-                    const float3 wcam = -nuv;
-                    const float we1 = camera_we1(cam, lens, wcam, rx, ry);
-                    if (we1 != 0.f) {
-                        float mis = 1.f;
-                        if (use_mis) {
-                            const float c = cam_to_local(cam, wcam).z;
-                            float camPdfA = cam.per_pixel_norm / (c * c * c) * fabsf(cos_l) / len2;
-                            if (s.med.on) camPdfA *= pass_pdf(s.med, len);
-                            mis = l.pdfA / (l.pdfA + camPdfA);
-                        }
-                        const float k = mis * we1 * G * kInvPi;
-                        float3 c = l.contrib * k;
-                        if (s.med.on) c = c * transmittance(s.med, len);  // attenuated connection
-                        const uint32_t target = kToSplat | (uint32_t(ry) * uint32_t(cam.W) + uint32_t(rx));
-                        so = make_float4(l.pos.x, l.pos.y, l.pos.z, len - kRayEps);
-                        sd = make_float4(nuv.x, nuv.y, nuv.z, __uint_as_float(target));
-                        sc = make_float4(c.x, c.y, c.z, __uint_as_float(job));
-                        splat = true;
-                    }
-                }
-            }
-            if (a.light) {
-                // the light subpath's first ray (pdf not needed: no MIS)
-                const float3 dir =
-                    to_world(make_frame(l.n), cosine_hemisphere(u01(key, kDimPixel), u01(key, kDimPixel + 1)));
-                ro = make_float4(l.pos.x, l.pos.y, l.pos.z, 0.f);
-                rdir = make_float4(dir.x, dir.y, dir.z, 0.f);
-                thr = make_float4(l.contrib.x, l.contrib.y, l.contrib.z, 0.f);
-            } else {
-                // primary ray (samplePerPixelWe1CosByPdf)
-                float pdfW;
-                const float3 dir = primary_dir(cam, key, px, py, lens, pdfW);
-                ro = make_float4(cpos.x, cpos.y, cpos.z, 0.f);
-                rdir = make_float4(dir.x, dir.y, dir.z, 0.f);
-                thr = make_float4(1.f, 1.f, 1.f, use_mis ? pdfW : 0.f);
-            }
-            ro.w = __uint_as_float(key);
-            rdir.w = __uint_as_float(sidx);
+            start_path<ENV>(s, a, use_mis, key, px, py, job, v);
+            v.o.w = __uint_as_float(key);
+            v.d.w = __uint_as_float(sidx);
         }
         if (fresh) {
             const uint32_t e = head + i;
-            store_once(&st.ray_o[e], ro);
-            store_once(&st.ray_d[e], rdir);
-            store_once(&st.thr[e], thr);
+            store_once(&st.ray_o[e], v.o);
+            store_once(&st.ray_d[e], v.d);
+            store_once(&st.thr[e], v.thr);
             store_once(&st.rad[e], make_float4(0.f, 0.f, 0.f, __uint_as_float(job << kBounceBits)));
             if (a.guided) st.rec[e] = 0u;
         }
         // t = 1 connections join the previous shade kernel's shadow rays
-        const uint32_t si = block_append(&pb.counters[pb.next.shadow_count], splat, agg);
-        if (splat) {
-            store_once(&pb.sh_o[si], so);
-            store_once(&pb.sh_d[si], sd);
-            store_once(&pb.sh_c[si], sc);
+        const uint32_t si = block_append(&pb.counters[pb.next.shadow_count], v.shadow, agg);
+        if (v.shadow) {
+            store_once(&pb.sh_o[si], v.so);
+            store_once(&pb.sh_d[si], v.sd);
+            store_once(&pb.sh_c[si], v.sc);
         }
     }
 }
@@ -613,9 +625,122 @@ __device__ __forceinline__ void extend_rays(DScene s1, const BatchJob *__restric
 
 // ============================================================== shade
 // One vertex of randomWalk with the PathNeeRenderer callback
-// (generalsubpathsampler.h:34-130, pathnextevent.h:100-149).  Continuing
-// paths are compacted into the next state; a finished path stores its
-// radiance in its sample's slot of the pass.
+// (generalsubpathsampler.h:34-130, pathnextevent.h:100-149): the hit h of the
+// ray with direction rd, the radiance and bounce in rad, and origin and
+// throughput from load_o and load_thr, which are called only where they are needed.
+template <bool ENV, class LoadO, class LoadThr>
+__device__ __forceinline__ void shade_vertex(const DScene &s, const RenderArgs &a, int N, int use_mis, uint2 h, float3 rd,
+                                             uint32_t sidx, float4 &rad, LoadO &&load_o, LoadThr &&load_thr, Vertex &out) {
+    const uint32_t bounce = __float_as_uint(rad.w) & kBounceMask;
+    const int cNum = int(bounce) + 2;  // camera is vertex 1
+    if (ENV && h.x == kInvalid && s.env_select > 0.f) {
+        // a miss is the envmap vertex (scene.h:82-88): an emitter hit with Le1 = 1,
+        // Le0 = the lookup, and area pdfs equal to the solid-angle ones
+        const float4 thr = load_thr();
+        float mis = a.nee ? 0.f : 1.f;
+        if (use_mis) {
+            const float lightPdfA = s.env_select * env_pdf_dir(s, rd);
+            mis = thr.w / (lightPdfA + thr.w);
+        }
+        const float3 c = xyz(thr) * env_eval(s, rd) * mis;
+        rad.x += c.x;
+        rad.y += c.y;
+        rad.z += c.z;
+    }
+    if (h.x != kInvalid) {
+        const float t = __uint_as_float(h.y);
+        const float4 ray_o = load_o();
+        const float3 ro = xyz(ray_o);
+        const uint32_t key = __float_as_uint(ray_o.w);
+        const float4 v0 = s.tris[3 * size_t(h.x) + 0];
+        const float4 v1 = s.tris[3 * size_t(h.x) + 1];
+        const float4 v2 = s.tris[3 * size_t(h.x) + 2];
+        const float3 pos = ro + rd * t;
+        const float3 ng = normalize3(cross3(xyz(v1) - xyz(v0), xyz(v2) - xyz(v0)));
+        const int2 gi = s.geom_info[__float_as_uint(v1.w)];
+        const float4 thr = load_thr();
+        const float3 T = xyz(thr);
+        if (gi.y >= 0) {
+            // emitter hit: MIS against light sampling (pathnextevent.h:128-146);
+            // without NEE it is the only estimate (weight 1, primitivepath.h:52-56)
+            const float cos_l = -dot3(ng, rd);
+            if (cos_l >= 0.f) {
+                const DLight &L = s.lights[gi.y];
+                float mis = a.nee ? 0.f : 1.f;
+                if (use_mis) {
+                    const float cPdfA = thr.w * fabsf(cos_l) / (t * t);
+                    const float lightPdfA = L.pdf_select * L.inv_area;
+                    mis = cPdfA / (lightPdfA + cPdfA);
+                }
+                rad.x += mis * T.x * L.L[0];
+                rad.y += mis * T.y * L.L[1];
+                rad.z += mis * T.z * L.L[2];
+            }
+        } else if (cNum != N) {
+            const DMat m = s.mats[gi.x];
+            const Frame f = make_frame(ng);
+            const float3 wi = to_local(f, -rd);
+            // NEE with MIS (pathnextevent.h:106-127)
+            const LightSample l = sample_light<ENV>(s, u01(key, kDimLight), u01(key, kDimLight + 1), key);
+            if (ENV && a.nee && l.env) {
+                // toward an envmap vertex: G = |cos| at the surface, visibility to infinity
+                const float3 nuv = l.pos;
+                const float G = fabsf(dot3(ng, nuv));
+                const float3 wo = to_local(f, nuv);
+                const float3 fs = G != 0.f ? bsdf_eval(m, wi, wo) : f3(0.f, 0.f, 0.f);
+                if (!is_black(fs)) {
+                    const float mis = use_mis ? l.pdfA / (l.pdfA + bsdf_pdf(m, wi, wo)) : 1.f;
+                    const float3 c = T * fs * l.contrib * (mis * G);
+                    if (!is_black(c)) {
+                        out.so = make_float4(pos.x, pos.y, pos.z, INFINITY);
+                        out.sd = make_float4(nuv.x, nuv.y, nuv.z, 0.f);
+                        out.sc = make_float4(c.x, c.y, c.z, 0.f);
+                        out.shadow = true;
+                    }
+                }
+            }
+            const float3 uv = l.pos - pos;
+            const float len2 = dot3(uv, uv);
+            const float len = sqrtf(len2);
+            const float3 nuv = uv * (1.0f / len);
+            const float cos_lv = -dot3(l.n, nuv);
+            const float G = fabsf(dot3(ng, nuv)) * fabsf(cos_lv) / len2;
+            if (a.nee && !(ENV && l.env) && G != 0.f && cos_lv >= 0.f) {
+                const float3 wo = to_local(f, nuv);
+                const float3 fs = bsdf_eval(m, wi, wo);
+                if (!is_black(fs)) {
+                    float mis = 1.f;
+                    if (use_mis) {
+                        const float bsdfPdfA = bsdf_pdf(m, wi, wo) * fabsf(cos_lv) / len2;
+                        mis = l.pdfA / (l.pdfA + bsdfPdfA);
+                    }
+                    const float k = mis * G * kInvPi;
+                    const float3 c = T * fs * l.contrib * k;
+                    if (!is_black(c)) {
+                        out.so = make_float4(pos.x, pos.y, pos.z, len - kRayEps);
+                        out.sd = make_float4(nuv.x, nuv.y, nuv.z, 0.f);
+                        out.sc = make_float4(c.x, c.y, c.z, 0.f);
+                        out.shadow = true;
+                    }
+                }
+            }
+            // BSDF sampling (generalsubpathsampler.h:81-130); here cNum < N
+            const uint32_t dim = kDimBounce0 + kDimsPerBounce * bounce + kBdBsdf;
+            float3 wo;
+            float pdf = 0.f;
+            const float3 w = bsdf_sample(m, wi, u01(key, dim), u01(key, dim + 1), wo, pdf);
+            if (!is_black(w)) {
+                const float3 nd = to_world(f, wo);
+                out.o = make_float4(pos.x, pos.y, pos.z, __uint_as_float(key));
+                out.d = make_float4(nd.x, nd.y, nd.z, __uint_as_float(sidx));
+                out.thr = make_float4(w.x * T.x, w.y * T.y, w.z * T.z, use_mis ? pdf : 0.f);
+                out.cont = true;
+            }
+        }
+    }
+}
+// The vertices of all active paths.  Continuing paths are compacted into the
+// next state; a finished path stores its radiance in its sample's slot of the pass.
 template <bool BATCH, bool ENV = false>
 __global__ __launch_bounds__(kShadeBlock) void k_shade(DScene s1, const BatchJob *__restrict__ jobs, PathBuffers pb,
                                                        RenderArgs a) {
@@ -625,147 +750,41 @@ __global__ __launch_bounds__(kShadeBlock) void k_shade(DScene s1, const BatchJob
     uint32_t flip = 0;
     for (uint32_t base = blockIdx.x * blockDim.x; base < n; base += gridDim.x * blockDim.x, flip++) {
         const uint32_t i = base + threadIdx.x;
-        bool push_shadow = false, cont = false;
         const bool valid = i < n;
-        float4 so = make_float4(0, 0, 0, 0), sd = so, sc = so;
-        float4 new_o = so, new_d = so, new_thr = so, rad = so;
-        uint32_t job = 0, key = 0, sidx = 0, bounce = 0;
+        Vertex v;
+        float4 rad = make_float4(0, 0, 0, 0);
+        uint32_t job = 0, sidx = 0;
         if (valid) {
             const float4 ray_d = load_once(&cs.ray_d[i]);
             const float3 rd = xyz(ray_d);
             sidx = __float_as_uint(ray_d.w);
             rad = load_once(&cs.rad[i]);
-            bounce = __float_as_uint(rad.w) & kBounceMask;
             job = __float_as_uint(rad.w) >> kBounceBits;
             const DScene &s = BATCH ? jobs[job].s : s1;
             const int N = BATCH ? jobs[job].N : a.N;
             const int use_mis = BATCH ? jobs[job].use_mis : a.use_mis;
-            const int cNum = int(bounce) + 2;  // camera is vertex 1
             const uint2 h = load_once(&pb.hit[i]);
-            if (ENV && h.x == kInvalid && s.env_select > 0.f) {
-                // a miss is the envmap vertex (scene.h:82-88): an emitter hit with Le1 = 1,
-                // Le0 = the lookup, and area pdfs equal to the solid-angle ones
-                const float4 thr = load_once(&cs.thr[i]);
-                float mis = a.nee ? 0.f : 1.f;
-                if (use_mis) {
-                    const float lightPdfA = s.env_select * env_pdf_dir(s, rd);
-                    mis = thr.w / (lightPdfA + thr.w);
-                }
-                const float3 c = xyz(thr) * env_eval(s, rd) * mis;
-                rad.x += c.x;
-                rad.y += c.y;
-                rad.z += c.z;
-            }
-            if (h.x != kInvalid) {
-                const float t = __uint_as_float(h.y);
-                const float4 ray_o = load_once(&cs.ray_o[i]);
-                const float3 ro = xyz(ray_o);
-                key = __float_as_uint(ray_o.w);
-                const float4 v0 = s.tris[3 * size_t(h.x) + 0];
-                const float4 v1 = s.tris[3 * size_t(h.x) + 1];
-                const float4 v2 = s.tris[3 * size_t(h.x) + 2];
-                const float3 pos = ro + rd * t;
-                const float3 ng = normalize3(cross3(xyz(v1) - xyz(v0), xyz(v2) - xyz(v0)));
-                const int2 gi = s.geom_info[__float_as_uint(v1.w)];
-                const float4 thr = load_once(&cs.thr[i]);
-                const float3 T = xyz(thr);
-                if (gi.y >= 0) {
-                    // emitter hit: MIS against light sampling (pathnextevent.h:128-146);
-                    // without NEE it is the only estimate (weight 1, primitivepath.h:52-56)
-                    const float cos_l = -dot3(ng, rd);
-                    if (cos_l >= 0.f) {
-                        const DLight &L = s.lights[gi.y];
-                        float mis = a.nee ? 0.f : 1.f;
-                        if (use_mis) {
-                            const float cPdfA = thr.w * fabsf(cos_l) / (t * t);
-                            const float lightPdfA = L.pdf_select * L.inv_area;
-                            mis = cPdfA / (lightPdfA + cPdfA);
-                        }
-                        rad.x += mis * T.x * L.L[0];
-                        rad.y += mis * T.y * L.L[1];
-                        rad.z += mis * T.z * L.L[2];
-                    }
-                } else if (cNum != N) {
-                    const DMat m = s.mats[gi.x];
-                    const Frame f = make_frame(ng);
-                    const float3 wi = to_local(f, -rd);
-                    // NEE with MIS (pathnextevent.h:106-127)
-                    const LightSample l = sample_light<ENV>(s, u01(key, kDimLight), u01(key, kDimLight + 1), key);
-                    if (ENV && a.nee && l.env) {
-                        // toward an envmap vertex: G = |cos| at the surface, visibility to infinity
-                        const float3 nuv = l.pos;
-                        const float G = fabsf(dot3(ng, nuv));
-                        const float3 wo = to_local(f, nuv);
-                        const float3 fs = G != 0.f ? bsdf_eval(m, wi, wo) : f3(0.f, 0.f, 0.f);
-                        if (!is_black(fs)) {
-                            const float mis = use_mis ? l.pdfA / (l.pdfA + bsdf_pdf(m, wi, wo)) : 1.f;
-                            const float3 c = T * fs * l.contrib * (mis * G);
-                            if (!is_black(c)) {
-                                so = make_float4(pos.x, pos.y, pos.z, INFINITY);
-                                sd = make_float4(nuv.x, nuv.y, nuv.z, 0.f);
-                                sc = make_float4(c.x, c.y, c.z, 0.f);
-                                push_shadow = true;
-                            }
-                        }
-                    }
-                    const float3 uv = l.pos - pos;
-                    const float len2 = dot3(uv, uv);
-                    const float len = sqrtf(len2);
-                    const float3 nuv = uv * (1.0f / len);
-                    const float cos_lv = -dot3(l.n, nuv);
-                    const float G = fabsf(dot3(ng, nuv)) * fabsf(cos_lv) / len2;
-                    if (a.nee && !(ENV && l.env) && G != 0.f && cos_lv >= 0.f) {
-                        const float3 wo = to_local(f, nuv);
-                        const float3 fs = bsdf_eval(m, wi, wo);
-                        if (!is_black(fs)) {
-                            float mis = 1.f;
-                            if (use_mis) {
-                                const float bsdfPdfA = bsdf_pdf(m, wi, wo) * fabsf(cos_lv) / len2;
-                                mis = l.pdfA / (l.pdfA + bsdfPdfA);
-                            }
-                            const float k = mis * G * kInvPi;
-                            const float3 c = T * fs * l.contrib * k;
-                            if (!is_black(c)) {
-                                so = make_float4(pos.x, pos.y, pos.z, len - kRayEps);
-                                sd = make_float4(nuv.x, nuv.y, nuv.z, 0.f);
-                                sc = make_float4(c.x, c.y, c.z, 0.f);
-                                push_shadow = true;
-                            }
-                        }
-                    }
-                    // BSDF sampling (generalsubpathsampler.h:81-130); here cNum < N
-                    const uint32_t dim = kDimBounce0 + kDimsPerBounce * bounce + kBdBsdf;
-                    float3 wo;
-                    float pdf = 0.f;
-                    const float3 w = bsdf_sample(m, wi, u01(key, dim), u01(key, dim + 1), wo, pdf);
-                    if (!is_black(w)) {
-                        const float3 nd = to_world(f, wo);
-                        new_o = make_float4(pos.x, pos.y, pos.z, __uint_as_float(key));
-                        new_d = make_float4(nd.x, nd.y, nd.z, __uint_as_float(sidx));
-                        new_thr = make_float4(w.x * T.x, w.y * T.y, w.z * T.z, use_mis ? pdf : 0.f);
-                        cont = true;
-                    }
-                }
-            }
+            shade_vertex<ENV>(s, a, N, use_mis, h, rd, sidx, rad, [&] { return load_once(&cs.ray_o[i]); },
+                              [&] { return load_once(&cs.thr[i]); }, v);
         }
-        const Append2 at = block_append2(&pb.counters[kQn], cont, push_shadow, agg, flip);
+        const Append2 at = block_append2(&pb.counters[kQn], v.cont, v.shadow, agg, flip);
         const uint32_t qi = at.a, si = at.b;
-        if (cont) {
-            store_once(&ns.ray_o[qi], new_o);
-            store_once(&ns.ray_d[qi], new_d);
-            store_once(&ns.thr[qi], new_thr);
+        if (v.cont) {
+            store_once(&ns.ray_o[qi], v.o);
+            store_once(&ns.ray_d[qi], v.d);
+            store_once(&ns.thr[qi], v.thr);
             rad.w = __uint_as_float(__float_as_uint(rad.w) + 1u);  // the next bounce
             store_once(&ns.rad[qi], rad);
         } else if (valid) {
             store_once(&pb.sample_rad[sidx], rad);
         }
-        const uint32_t target = cont ? (kToNextPath | qi) : (kToSample | sidx);
-        sd.w = __uint_as_float(target);
-        sc.w = __uint_as_float(job);
-        if (push_shadow) {
-            store_once(&pb.sh_o[si], so);
-            store_once(&pb.sh_d[si], sd);
-            store_once(&pb.sh_c[si], sc);
+        const uint32_t target = v.cont ? (kToNextPath | qi) : (kToSample | sidx);
+        v.sd.w = __uint_as_float(target);
+        v.sc.w = __uint_as_float(job);
+        if (v.shadow) {
+            store_once(&pb.sh_o[si], v.so);
+            store_once(&pb.sh_d[si], v.sd);
+            store_once(&pb.sh_c[si], v.sc);
         }
     }
     end_iteration(pb, a);
@@ -1344,6 +1363,117 @@ __global__ __launch_bounds__(kBlock) WR_EXTEND_ATTR(WR_BATCH_WAVES) void k_trace
                                                                         PathBuffers pb, uint2 *spill, TravTune tune) {
     trace_bounce<COUNT, BATCH>(s1, jobs, pb, spill, tune);
 }
+// ============================================================== small passes
+// A pass of few samples, start to end in one launch.  Its iterations are bound
+// by the latency of their launches and queues (about 25 us each, of which a
+// traversal over a short queue takes 12), so a block of two waves keeps 64 paths
+// in registers: the first wave starts them, traces their closest hits and
+// shades; the second traces the shadow rays that the first one left in LDS, at
+// the same time.  The arithmetic and the order in which a sample's radiance is
+// summed are those of k_regen, k_trace_bounce_fast and k_shade.
+//
+// Lanes whose paths have ended stay idle, so the queues win once there are
+// enough rays to fill the chip several times over.  Queues / this kernel, in
+// ms, by samples of the pass:
+//                          16,384         131,044        262,144        1,048,576
+//   Cornell box            0.333 / 0.169  0.535 / 0.237  0.494 / 0.348  1.66 / 1.09
+//   1.31M-triangle frame   1.54  / 0.59   2.27  / 0.95   2.34  / 1.28   3.14 / 4.98
+//   gap room               2.31  / 1.33   2.99  / 1.68   3.21  / 3.07   7.8  / 14.2
+//   clutter, 5k triangles                                0.85  / 0.66   2.15 / 2.21
+// It takes passes of up to 2^18 samples, and no more than one block per pair of
+// spill slices, so each block has one tile.  Six waves per SIMD: their registers
+// still hold everything, and 131,072 to 262,144 samples run up to 30% faster
+// than at four (gap room 3.58 -> 3.07 ms).
+constexpr uint32_t kSmallPassSamples = 1u << 18;
+template <bool ENV>
+__global__ __launch_bounds__(2 * kBlock) WR_EXTEND_ATTR(6) void k_small_pass(DScene s, PathBuffers pb, RenderArgs a, uint2 *spill) {
+    __shared__ uint64_t st_ent[2][kLdsSlots * kBlock];
+    __shared__ float4 sh_o[kBlock], sh_d[kBlock], sh_c[kBlock];
+    __shared__ uint32_t sent[kBlock], seen[kBlock];  // a shadow ray of lane l; it adds to its path
+    __shared__ uint32_t more;
+    const uint32_t wave = threadIdx.x / kBlock, lane = lane_id();
+    const DCamera &cam = s.cam;
+    uint2 *my_spill = spill + size_t(blockIdx.x + wave) * (kSpillDepth * kBlock);  // slice 2 blockIdx.x + wave
+    TraversalCounters cnt;
+    uint32_t rays = 0;
+    const uint32_t sidx = blockIdx.x * kBlock + lane;
+    bool alive = false, pending = false;  // pending: ended, its last shadow ray is on its way
+    Vertex v;
+    float4 rad = make_float4(0, 0, 0, 0);
+    if (wave == 0) {
+        alive = sidx < a.total;
+        if (alive) {
+            const uint32_t pixel = sidx % a.wh;
+            const uint32_t key = path_key(a.seed, pixel, a.first_sample + sidx / a.wh);
+            start_path<ENV>(s, a, a.use_mis, key, pixel % uint32_t(cam.W), pixel / uint32_t(cam.W), 0u, v);
+            v.o.w = __uint_as_float(key);
+        }
+        sent[lane] = v.shadow;
+        if (v.shadow) { sh_o[lane] = v.so; sh_d[lane] = v.sd; sh_c[lane] = v.sc; }
+    }
+    for (bool first = true;; first = false) {
+        __syncthreads();  // the shadow rays and `more` are written
+        if (!first && !more) break;
+        uint2 h = make_uint2(kInvalid, 0u);
+        if (wave == 0) {
+            if (alive) {
+                float t = INFINITY;
+                h.x = traverse_rounds<false, kBlock>(s, setup_ray(xyz(v.o), xyz(v.d), kRayEps), t, st_ent[0], my_spill, cnt);
+                h.y = __float_as_uint(t);
+                rays++;
+            }
+        } else {
+            bool adds = false;
+            if (sent[lane]) {
+                const float4 o = sh_o[lane], d = sh_d[lane];
+                float t = o.w;
+                const bool visible = traverse_rounds<true, kBlock>(s, setup_ray(xyz(o), xyz(d), kRayEps), t, st_ent[1],
+                                                                   my_spill, cnt) == kInvalid;
+                const uint32_t target = __float_as_uint(d.w);
+                const bool splat = (target & ~kTargetMask) == kToSplat;
+                if (visible && splat) {
+                    const float4 c = sh_c[lane];
+                    double *dst = pb.film_splat + 3 * size_t(target & kTargetMask);
+                    atomicAdd(dst + 0, double(c.x));
+                    atomicAdd(dst + 1, double(c.y));
+                    atomicAdd(dst + 2, double(c.z));
+                }
+                adds = visible && !splat;
+                rays++;
+            }
+            seen[lane] = adds;
+        }
+        __syncthreads();  // the shadow rays are traced
+        if (wave != 0) continue;
+        if (seen[lane]) {
+            const float4 c = sh_c[lane];
+            rad.x += c.x; rad.y += c.y; rad.z += c.z;
+        }
+        bool ended = pending, shadow = false;
+        pending = false;
+        if (alive) {
+            const float4 o = v.o, thr = v.thr;
+            Vertex nv;
+            shade_vertex<ENV>(s, a, a.N, a.use_mis, h, xyz(v.d), sidx, rad, [&] { return o; }, [&] { return thr; }, nv);
+            shadow = nv.shadow;
+            alive = nv.cont;
+            ended = !alive && !shadow;
+            pending = !alive && shadow;
+            rad.w = __uint_as_float(__float_as_uint(rad.w) + 1u);  // the next bounce
+            if (shadow) {
+                nv.sd.w = __uint_as_float(kToSample);
+                sh_o[lane] = nv.so; sh_d[lane] = nv.sd; sh_c[lane] = nv.sc;
+            }
+            v = nv;
+        }
+        sent[lane] = shadow;
+        if (ended) store_once(&pb.sample_rad[sidx], rad);
+        const bool go = __ballot(alive || pending) != 0;
+        if (lane == 0) more = go;
+    }
+    wave_add_stat(&pb.stats[wave], rays);
+}
+
 // The plain kernel of wr_render_nee / wr_render_guided and the other
 // integrators' loops.
 __global__ __launch_bounds__(kBlock) WR_EXTEND_ATTR(WR_EXTEND_WAVES) void k_trace_bounce_fast(DScene s1, PathBuffers pb, uint2 *spill,
@@ -2765,6 +2895,10 @@ static int render_impl(wr_scene *s, wr_film *f, const wr_render_params *prm, wr_
                                          : reinterpret_cast<const void *>(&k_guide_infer<false, false>));
     const int g_infer = std::max(1, std::min<int>((P + kInferBlock - 1) / kInferBlock,
                                                   s->dev->n_cu * occupancy(s->dev, infer_fn, kInferBlock)));
+    // passes that k_small_pass takes: the plain estimators, unless traversal
+    // counters, per-kernel times or graph replays of the iterations are asked for
+    const bool small_passes = est != kEstLight && !g && !medium && !count && !prof && !use_graph;
+    const uint32_t small_tiles = std::min(kSmallPassSamples / kBlock, uint32_t(fixed ? fixed->trav_blocks : s->max_trav_blocks) / 2);
     guide::Net net{};
     // up to P closest-hit rays and 2P shadow rays (one per path and one per new sample)
     int g_trav = trav_grid(s, 2 * P, s->dev->occ_rays);
@@ -2797,7 +2931,14 @@ static int render_impl(wr_scene *s, wr_film *f, const wr_render_params *prm, wr_
                                   gp->max_guided_bounce ? gp->max_guided_bounce : 0xFFFFFFFFu, &gs);
             if (rc) return rc;
         }
-        k_init<<<1, 64, 0, s->stream>>>(pb, a);
+        const uint32_t tiles = (a.total + kBlock - 1) / kBlock;
+        const bool small = small_passes && a.total <= P && tiles <= small_tiles;
+        if (small) {
+            if (env) k_small_pass<true><<<tiles, 2 * kBlock, 0, s->stream>>>(ds, pb, a, spill);
+            else k_small_pass<false><<<tiles, 2 * kBlock, 0, s->stream>>>(ds, pb, a, spill);
+        } else {
+            k_init<<<1, 64, 0, s->stream>>>(pb, a);
+        }
         WR_HIP(hipGetLastError());
         // Each iteration refills the pool, extends every active path by one
         // vertex and resolves the shadow rays of the previous iteration's
@@ -2841,7 +2982,7 @@ static int render_impl(wr_scene *s, wr_film *f, const wr_render_params *prm, wr_
             else k_shade<false><<<g_shade, bs, 0, s->stream>>>(ds, nullptr, q, a);
             end();
         };
-        rc = drain(s, pb, max_iters, use_graph, host_counters, a.progress, a.tag, iteration);
+        rc = small ? WR_OK : drain(s, pb, max_iters, use_graph, host_counters, a.progress, a.tag, iteration);
         if (rc) return rc;
         begin(4);
         k_accumulate<<<std::max<uint32_t>(1, std::min<uint32_t>((wh + 255) / 256, uint32_t(s->dev->n_cu) * 8)), 256, 0,
