@@ -4,8 +4,9 @@ same passes through the path queues (a path pool one smaller than the pass).
 Both do the same arithmetic on each sample and sum it in the same order, so base
 films are equal bit for bit and ray counts are equal; the splat film is FP64
 atomics in varying order and agrees to rounding (1e-11).  Sizes: one pixel, edges
-of the 64-path tiles, several samples per pixel, and both sides of the limit of
-2^18 samples."""
+of the 64-path tiles, several samples per pixel, shares that restart lanes (above
+2^18 samples), and both sides of the limits (2^22 samples up to 2^11 triangles,
+2^20 up to 2^16, else 2^18)."""
 import ctypes as C
 
 import numpy as np
@@ -21,6 +22,7 @@ SCENES = {
     "spheres": lambda r: scenes.icospheres(2, n_spheres=12, level=3, resolution=r),
     "env": lambda r: scenes.icospheres(2, n_spheres=12, level=3, resolution=r).with_envmap((0.3, 0.4, 0.5)),
     "clutter": lambda r: scenes.cornell_clutter(3, 12_000, r),
+    "room": lambda r: scenes.guide_room(4, n_spheres=49, level=4, resolution=r),
 }
 
 
@@ -36,7 +38,8 @@ def _films(gs, render, total, spp, **kw):
 
 @pytest.mark.parametrize("kind", list(SCENES))
 @pytest.mark.parametrize("size,spp,vertices", [((1, 2), 1, 8), ((9, 7), 1, 2), ((64, 1), 1, 3), ((13, 5), 1, 8), ((63, 65), 3, 10),
-                                               ((512, 512), 1, 12), ((512, 513), 1, 6)])
+                                               ((512, 512), 1, 12), ((512, 513), 1, 6),
+                                               ((1024, 1024), 1, 9), ((1024, 1025), 1, 4)])
 def test_small_passes_equal_the_queues(gpu_device, kind, size, spp, vertices):
     print(f"small pass: {kind} {size} spp={spp} N={vertices}", flush=True)
     gs = wr.GpuScene(gpu_device, SCENES[kind](size))
@@ -46,6 +49,15 @@ def test_small_passes_equal_the_queues(gpu_device, kind, size, spp, vertices):
         np.testing.assert_array_equal(a[0], b[0])
         np.testing.assert_allclose(a[1], b[1], rtol=1e-11, atol=1e-300)
         assert a[2:] == b[2:]
+
+
+@pytest.mark.parametrize("spp", [16, 17])
+def test_shares_up_to_the_limit_of_a_tiny_scene(gpu_device, spp):
+    print(f"small pass: cornell 512x512 spp={spp}", flush=True)
+    gs = wr.GpuScene(gpu_device, SCENES["cornell"]((512, 512)))
+    a, b = _films(gs, wr.render_nee, 512 * 512 * spp, spp, num_path_vertices=12)
+    np.testing.assert_array_equal(a[0], b[0])
+    assert a[2:] == b[2:]
 
 
 def test_small_pass_in_the_fixed_region(gpu_device):

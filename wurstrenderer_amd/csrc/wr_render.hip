@@ -1372,21 +1372,36 @@ __global__ __launch_bounds__(kBlock) WR_EXTEND_ATTR(WR_BATCH_WAVES) void k_trace
 // the same time.  The arithmetic and the order in which a sample's radiance is
 // summed are those of k_regen, k_trace_bounce_fast and k_shade.
 //
-// Lanes whose paths have ended stay idle, so the queues win once there are
-// enough rays to fill the chip several times over.  Queues / this kernel, in
-// ms, by samples of the pass:
-//                          16,384         131,044        262,144        1,048,576
-//   Cornell box            0.333 / 0.169  0.535 / 0.237  0.494 / 0.348  1.66 / 1.09
-//   1.31M-triangle frame   1.54  / 0.59   2.27  / 0.95   2.34  / 1.28   3.14 / 4.98
-//   gap room               2.31  / 1.33   2.99  / 1.68   3.21  / 3.07   7.8  / 14.2
-//   clutter, 5k triangles                                0.85  / 0.66   2.15 / 2.21
-// It takes passes of up to 2^18 samples, and no more than one block per pair of
-// spill slices, so each block has one tile.  Six waves per SIMD: their registers
-// still hold everything, and 131,072 to 262,144 samples run up to 30% faster
-// than at four (gap room 3.58 -> 3.07 ms).
-constexpr uint32_t kSmallPassSamples = 1u << 18;
+// A block has per_block consecutive samples: a tile of 64, or, where the pass
+// has more tiles than the spill region has pairs of slices, an equal share of
+// the pass for each resident block, which starts the next samples in the lanes
+// whose paths have ended once kRestartLanes of them have.
+//
+// A wave steps at the pace of its slowest ray, where the queues refill lanes
+// inside a traversal; with enough rays to fill the chip several times over they
+// win, the earlier the more the lengths of the traversals differ.  Queues / this
+// kernel, in ms, by samples of the pass (12 to 18 path vertices):
+//                          16,384       131,044      262,144      1,048,576    4,194,304
+//   Cornell box, 36         0.33 / 0.17  0.53 / 0.25  0.59 / 0.42  1.83 / 1.11  5.25 / 3.72
+//   clutter, 1,000                                   0.75 / 0.55  2.05 / 1.36  5.47 / 4.61
+//   clutter, 5,000                                   0.84 / 0.65  2.17 / 1.68  5.61 / 5.79
+//   clutter, 40,000                                  0.97 / 0.70  2.31 / 1.95  5.71 / 6.79
+//   clutter, 200,000                                 1.16 / 0.84  2.57 / 2.33  6.15 / 8.05
+//   spheres, 1.31M         1.54 / 0.59  2.27 / 0.95  2.34 / 1.27  3.09 / 2.40
+//   gap room, 1.0M         2.31 / 1.33  2.99 / 1.68  3.21 / 3.04  7.70 / 10.4
+// (16,777,216 in the Cornell box 14.2 / 14.2), hence small_pass_samples.  Six
+// waves per SIMD: the registers still hold everything, and 262,144 samples of
+// the gap room take 3.6 ms at four.  Restarting at 1 / 8 / 16 / 32 idle lanes:
+// 3.91 / 3.78 / 3.72 / 3.96 ms in the box at 4,194,304 samples.
+constexpr uint32_t kRestartLanes = 16;
+// Largest pass of k_small_pass in a scene of n_tris triangles; passes of at most
+// a tile per pair of spill slices (2^18 samples; 2^15 in the fixed region, whose
+// 512 blocks would leave most of the chip idle with more) always take it.
+static uint32_t small_pass_samples(uint32_t n_tris) {
+    return n_tris <= 1u << 11 ? 1u << 22 : n_tris <= 1u << 16 ? 1u << 20 : 0u;
+}
 template <bool ENV>
-__global__ __launch_bounds__(2 * kBlock) WR_EXTEND_ATTR(6) void k_small_pass(DScene s, PathBuffers pb, RenderArgs a, uint2 *spill) {
+__global__ __launch_bounds__(2 * kBlock) WR_EXTEND_ATTR(6) void k_small_pass(DScene s, PathBuffers pb, RenderArgs a, uint32_t per_block, uint2 *spill) {
     __shared__ uint64_t st_ent[2][kLdsSlots * kBlock];
     __shared__ float4 sh_o[kBlock], sh_d[kBlock], sh_c[kBlock];
     __shared__ uint32_t sent[kBlock], seen[kBlock];  // a shadow ray of lane l; it adds to its path
@@ -1396,24 +1411,40 @@ __global__ __launch_bounds__(2 * kBlock) WR_EXTEND_ATTR(6) void k_small_pass(DSc
     uint2 *my_spill = spill + size_t(blockIdx.x + wave) * (kSpillDepth * kBlock);  // slice 2 blockIdx.x + wave
     TraversalCounters cnt;
     uint32_t rays = 0;
-    const uint32_t sidx = blockIdx.x * kBlock + lane;
+    uint32_t next = min(blockIdx.x * per_block, a.total);  // wave 0: the block's next sample
+    const uint32_t end = min(next + per_block, a.total);
     bool alive = false, pending = false;  // pending: ended, its last shadow ray is on its way
+    bool shadow = false;                  // v.so, v.sd, v.sc is a shadow ray to trace
+    uint32_t sidx = 0;
     Vertex v;
     float4 rad = make_float4(0, 0, 0, 0);
-    if (wave == 0) {
-        alive = sidx < a.total;
-        if (alive) {
-            const uint32_t pixel = sidx % a.wh;
-            const uint32_t key = path_key(a.seed, pixel, a.first_sample + sidx / a.wh);
-            start_path<ENV>(s, a, a.use_mis, key, pixel % uint32_t(cam.W), pixel / uint32_t(cam.W), 0u, v);
-            v.o.w = __uint_as_float(key);
+    for (;;) {
+        if (wave == 0) {
+            const unsigned long long idle = __ballot(!alive && !pending);
+            const uint32_t k = (uint32_t)__popcll(idle);
+            if (next < end && k >= kRestartLanes) {
+                if (!alive && !pending) {
+                    sidx = next + mbcnt64(idle);
+                    alive = sidx < end;
+                    v = Vertex{};
+                    rad = make_float4(0, 0, 0, 0);
+                    if (alive) {
+                        const uint32_t pixel = sidx % a.wh;
+                        const uint32_t key = path_key(a.seed, pixel, a.first_sample + sidx / a.wh);
+                        start_path<ENV>(s, a, a.use_mis, key, pixel % uint32_t(cam.W), pixel / uint32_t(cam.W), 0u, v);
+                        v.o.w = __uint_as_float(key);
+                    }
+                    shadow = v.shadow;
+                }
+                next = min(next + k, end);
+            }
+            sent[lane] = shadow;
+            if (shadow) { sh_o[lane] = v.so; sh_d[lane] = v.sd; sh_c[lane] = v.sc; }
+            const bool go = __ballot(alive || pending) != 0;
+            if (lane == 0) more = go;
         }
-        sent[lane] = v.shadow;
-        if (v.shadow) { sh_o[lane] = v.so; sh_d[lane] = v.sd; sh_c[lane] = v.sc; }
-    }
-    for (bool first = true;; first = false) {
         __syncthreads();  // the shadow rays and `more` are written
-        if (!first && !more) break;
+        if (!more) break;
         uint2 h = make_uint2(kInvalid, 0u);
         if (wave == 0) {
             if (alive) {
@@ -1449,27 +1480,21 @@ __global__ __launch_bounds__(2 * kBlock) WR_EXTEND_ATTR(6) void k_small_pass(DSc
             const float4 c = sh_c[lane];
             rad.x += c.x; rad.y += c.y; rad.z += c.z;
         }
-        bool ended = pending, shadow = false;
-        pending = false;
+        bool ended = pending;
+        pending = shadow = false;
         if (alive) {
             const float4 o = v.o, thr = v.thr;
             Vertex nv;
             shade_vertex<ENV>(s, a, a.N, a.use_mis, h, xyz(v.d), sidx, rad, [&] { return o; }, [&] { return thr; }, nv);
-            shadow = nv.shadow;
-            alive = nv.cont;
+            nv.sd.w = __uint_as_float(kToSample);
+            v = nv;
+            shadow = v.shadow;
+            alive = v.cont;
             ended = !alive && !shadow;
             pending = !alive && shadow;
             rad.w = __uint_as_float(__float_as_uint(rad.w) + 1u);  // the next bounce
-            if (shadow) {
-                nv.sd.w = __uint_as_float(kToSample);
-                sh_o[lane] = nv.so; sh_d[lane] = nv.sd; sh_c[lane] = nv.sc;
-            }
-            v = nv;
         }
-        sent[lane] = shadow;
         if (ended) store_once(&pb.sample_rad[sidx], rad);
-        const bool go = __ballot(alive || pending) != 0;
-        if (lane == 0) more = go;
     }
     wave_add_stat(&pb.stats[wave], rays);
 }
@@ -2898,7 +2923,9 @@ static int render_impl(wr_scene *s, wr_film *f, const wr_render_params *prm, wr_
     // passes that k_small_pass takes: the plain estimators, unless traversal
     // counters, per-kernel times or graph replays of the iterations are asked for
     const bool small_passes = est != kEstLight && !g && !medium && !count && !prof && !use_graph;
-    const uint32_t small_tiles = std::min(kSmallPassSamples / kBlock, uint32_t(fixed ? fixed->trav_blocks : s->max_trav_blocks) / 2);
+    const void *small_fn = env ? reinterpret_cast<const void *>(&k_small_pass<true>) : reinterpret_cast<const void *>(&k_small_pass<false>);
+    const uint32_t small_blocks = uint32_t(s->dev->n_cu * occupancy(s->dev, small_fn, 2 * kBlock));
+    const uint32_t small_slices = uint32_t(fixed ? fixed->trav_blocks : s->max_trav_blocks) / 2;
     guide::Net net{};
     // up to P closest-hit rays and 2P shadow rays (one per path and one per new sample)
     int g_trav = trav_grid(s, 2 * P, s->dev->occ_rays);
@@ -2932,10 +2959,14 @@ static int render_impl(wr_scene *s, wr_film *f, const wr_render_params *prm, wr_
             if (rc) return rc;
         }
         const uint32_t tiles = (a.total + kBlock - 1) / kBlock;
-        const bool small = small_passes && a.total <= P && tiles <= small_tiles;
+        const bool small = small_passes && a.total <= P &&
+                           (tiles <= small_slices || (!fixed && a.total <= small_pass_samples(s->n_tris)));
         if (small) {
-            if (env) k_small_pass<true><<<tiles, 2 * kBlock, 0, s->stream>>>(ds, pb, a, spill);
-            else k_small_pass<false><<<tiles, 2 * kBlock, 0, s->stream>>>(ds, pb, a, spill);
+            // a tile per block as long as there are spill slices, else resident blocks with equal shares
+            const uint32_t grid = tiles <= small_slices ? tiles : std::min(small_blocks, small_slices);
+            const uint32_t per_block = tiles <= small_slices ? kBlock : (a.total + grid - 1) / grid;
+            if (env) k_small_pass<true><<<grid, 2 * kBlock, 0, s->stream>>>(ds, pb, a, per_block, spill);
+            else k_small_pass<false><<<grid, 2 * kBlock, 0, s->stream>>>(ds, pb, a, per_block, spill);
         } else {
             k_init<<<1, 64, 0, s->stream>>>(pb, a);
         }
