@@ -124,9 +124,10 @@ struct BlockPool {
     struct Block { void *p = nullptr; size_t bytes = 0; };
     int keep;
     size_t most;
+    bool close_fit;  // blocks of more than twice the size asked for are not handed out
     std::mutex m;
     std::vector<Block> free_blocks;
-    BlockPool(int keep_, size_t most_) : keep(keep_), most(most_) {}
+    BlockPool(int keep_, size_t most_, bool close_fit_ = false) : keep(keep_), most(most_), close_fit(close_fit_) {}
     ~BlockPool() {
         for (Block &b : free_blocks) (void)hipFree(b.p);
     }
@@ -136,7 +137,7 @@ struct BlockPool {
             std::lock_guard<std::mutex> lock(m);
             size_t best = free_blocks.size();
             for (size_t i = 0; i < free_blocks.size(); i++)
-                if (free_blocks[i].bytes >= bytes &&
+                if (free_blocks[i].bytes >= bytes && (!close_fit || free_blocks[i].bytes / 2 <= bytes) &&
                     (best == free_blocks.size() || free_blocks[i].bytes < free_blocks[best].bytes))
                     best = i;
             if (best < free_blocks.size()) {
@@ -182,9 +183,11 @@ struct wr_device {
     int occ_rays = 8, occ_shade = 8, occ_generate = 8, occ_trace = 8;
     std::map<const void *, int> occ_cache;  // other kernels, filled on first use
     BlockPool spills{2, size_t(1) << 30};       // traversal stack spill regions, one per scene
+    BlockPool geometry{3, size_t(512) << 20, true};  // nodes (both copies) and triangles of GPU-built scenes
     BlockPool build_memory{1, size_t(1) << 30}; // mesh copies and scratch of BVH builds
     void trim() {
         spills.trim();
+        geometry.trim();
         build_memory.trim();
     }
     // hipMalloc that frees the pools' idle blocks where memory runs out
@@ -222,6 +225,7 @@ struct wr_scene {
     float4 *d_ltris = nullptr;
     uint2 *d_spill = nullptr;   // traversal stack spill: kSpillDepth entries per lane of the largest grid
     BlockPool::Block spill;     // the block behind it, from the device's pool
+    BlockPool::Block nodes_block, tris_block, qnodes_block;  // behind the geometry, if it came from the pool
     float4 *d_bdpt = nullptr;   // bidirectional light-vertex records (+ 2 ray counters), grown on demand
     size_t bdpt_bytes = 0;
     int max_trav_blocks = 0;
@@ -268,6 +272,7 @@ namespace wr {
 struct GpuBvhResult {
     Node4 *nodes = nullptr;     // device, n_nodes, breadth-first (root = 0, children after parents)
     TriRecord *tris = nullptr;  // device, leaf order
+    BlockPool::Block nodes_block, tris_block;  // the blocks of the device's geometry pool behind them, if any
     uint32_t n_nodes = 0, max_stack = 0, depth = 0, iterations = 0;
     double ms = 0.0;            // wall time of the build
 };
