@@ -223,6 +223,11 @@ __device__ __forceinline__ uint32_t pair_hash(uint32_t lo, uint32_t hi, uint32_t
     return uint32_t(x);
 }
 
+struct ClusterBuffers {
+    uint32_t *buf[2];
+};
+constexpr uint32_t kTailClusters = 2048;
+constexpr int kMergeBlock = 1024, kPlocBatch = 6;
 // The cluster in [i - R, i + R] of m whose union with cluster i has the smallest
 // surface area; equal areas go to the higher pair hash, then to the lower
 // index.  lo[k] and hi[k] are the boxes of cluster i + k.
@@ -246,8 +251,11 @@ __device__ __forceinline__ uint32_t nearest_of(int64_t i, int64_t m, int R, uint
     if (bj < 0) bj = i > 0 ? i - 1 : i + 1;
     return uint32_t(bj);
 }
-__global__ __launch_bounds__(kBB) void k_nearest(const uint32_t *clusters, uint32_t m, const float4 *nlo,
-                                                 const float4 *nhi, int R, uint32_t seed, uint32_t *nearest) {
+__global__ __launch_bounds__(kBB) void k_nearest(const PlocState *st, ClusterBuffers cl, const float4 *nlo,
+                                                 const float4 *nhi, int R, uint32_t *nearest) {
+    const uint32_t m = st->m, seed = st->iteration;
+    if (m <= kTailClusters || blockIdx.x * kBB >= m) return;
+    const uint32_t *clusters = cl.buf[st->which];
     __shared__ float4 slo[kBB + 2 * kPlocRadiusMax], shi[kBB + 2 * kPlocRadiusMax];
     const int64_t base = int64_t(blockIdx.x) * kBB - R;
     for (int s = threadIdx.x; s < kBB + 2 * R; s += kBB) {
@@ -265,16 +273,27 @@ __global__ __launch_bounds__(kBB) void k_nearest(const uint32_t *clusters, uint3
     nearest[i] = nearest_of(i, m, R, seed, slo + me, shi + me);
 }
 
-// flags[i]: bit 32 = cluster i merges with its mutual nearest neighbour (the
-// lower index of the pair owns the merge); bit 0 = cluster i survives.
-__global__ __launch_bounds__(kBB) void k_merge_flags(const uint32_t *nearest, uint32_t m, uint64_t *flags) {
-    const uint32_t i = blockIdx.x * kBB + threadIdx.x;
-    if (i >= m) return;
+// What cluster i does: bit 16: it merges with its nearest (and keeps its place),
+// bit 0: it keeps its place.  Two clusters merge if each is the other's nearest.
+__device__ __forceinline__ uint32_t merge_role(const uint32_t *nearest, uint32_t i, uint32_t m) {
+    if (i >= m) return 0u;
     const uint32_t j = nearest[i];
     const bool mutual = nearest[j] == i;
-    const bool merge = mutual && i < j;
-    const bool keep = !(mutual && i > j);
-    flags[i] = (uint64_t(merge) << 32) | uint64_t(keep);
+    return (mutual && i < j ? 1u << 16 : 0u) + (mutual && i > j ? 0u : 1u);
+}
+// merges and places of each block of clusters -> sums[block] (16 bits each)
+__global__ __launch_bounds__(kMergeBlock) void k_merge_count(const PlocState *st, const uint32_t *nearest, uint32_t *sums) {
+    __shared__ uint32_t part[kMergeBlock / 64];
+    const uint32_t m = st->m;
+    if (m <= kTailClusters || blockIdx.x * kMergeBlock >= m) return;
+    uint32_t v = merge_role(nearest, blockIdx.x * kMergeBlock + threadIdx.x, m);
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+    if (threadIdx.x % 64 == 0) part[threadIdx.x / 64] = v;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < kMergeBlock / 64; w++) v += part[w];
+        sums[blockIdx.x] = v;
+    }
 }
 
 // Node `id` over nodes a and b with boxes (la, ha) and (lb, hb): box, SAH cost
@@ -329,24 +348,63 @@ __device__ __forceinline__ void merge_nodes(uint32_t a, uint32_t b, float4 la, f
     }
 }
 
-// Creates the merged nodes (ids node_base + merge rank) with their SAH cost and
-// leaf decision, and compacts the surviving clusters in order.
-__global__ __launch_bounds__(kBB) void k_merge(const uint32_t *clusters, const uint32_t *nearest, uint32_t m,
-                                               const uint64_t *flags, const uint64_t *incl, uint32_t node_base,
-                                               float4 *nlo, float4 *nhi, uint2 *kids, float4 *wc, uint32_t *wd,
-                                               uint32_t *out) {
-    const uint32_t i = blockIdx.x * kBB + threadIdx.x;
-    if (i >= m) return;
-    const uint64_t f = flags[i];
-    if (!(f & 1u)) return;
-    const uint64_t s = incl[i];
-    const uint32_t pos = uint32_t(s) - 1u;
-    if (!(f >> 32)) {
+// Creates the merged nodes (ids base + merge rank) and compacts the clusters in
+// place order into the other buffer; the last block writes the next state.
+// Every block adds up the sums of the blocks before it (at most 1,280 words
+// from L2 at 1.31M triangles), which saves the launches of a scan.
+__global__ __launch_bounds__(kMergeBlock) void k_merge(const PlocState *st, PlocState *next, ClusterBuffers cl,
+                                                       const uint32_t *nearest, const uint32_t *sums, float4 *nlo,
+                                                       float4 *nhi, uint2 *kids, float4 *wc, uint32_t *wd) {
+    __shared__ uint64_t part[kMergeBlock / 64];
+    const PlocState s = *st;
+    if (s.m <= kTailClusters) {  // nothing left to do here
+        if (blockIdx.x == 0 && threadIdx.x == 0) *next = s;
+        return;
+    }
+    if (blockIdx.x * kMergeBlock >= s.m) return;
+    const uint32_t *clusters = cl.buf[s.which];
+    uint32_t *out = cl.buf[s.which ^ 1u];
+    const uint32_t t = threadIdx.x, wave = t / 64, lane = t % 64;
+    // merges (high word) and places (low word) before this block
+    uint64_t before = 0;
+    for (uint32_t b = t; b < blockIdx.x; b += kMergeBlock) {
+        const uint32_t v = sums[b];
+        before += uint64_t(v >> 16) << 32 | (v & 0xFFFFu);
+    }
+    for (int o = 32; o > 0; o >>= 1) before += __shfl_xor(before, o);
+    if (lane == 0) part[wave] = before;
+    __syncthreads();
+    before = 0;
+    for (int w = 0; w < kMergeBlock / 64; w++) before += part[w];
+    __syncthreads();
+    // and before this cluster
+    const uint32_t i = blockIdx.x * kMergeBlock + t;
+    const uint32_t role = merge_role(nearest, i, s.m);
+    uint32_t incl = role;
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t v = __shfl_up(incl, o);
+        if (int(lane) >= o) incl += v;
+    }
+    if (lane == 63) part[wave] = incl;
+    __syncthreads();
+    uint32_t in_block = incl - role, total = 0;
+    for (uint32_t w = 0; w < kMergeBlock / 64; w++) {
+        if (w < wave) in_block += uint32_t(part[w]);
+        total += uint32_t(part[w]);
+    }
+    if ((blockIdx.x + 1) * kMergeBlock >= s.m && t == 0) {
+        const uint32_t merges = uint32_t(before >> 32) + (total >> 16), kept = uint32_t(before) + (total & 0xFFFFu);
+        const bool stuck = merges == 0 || kept != s.m - merges;
+        *next = PlocState{stuck ? 0u : kept, s.base + merges, s.iteration + 1, s.which ^ 1u, stuck ? 1u : 0u};
+    }
+    if (!(role & 1u)) return;
+    const uint32_t pos = uint32_t(before) + (in_block & 0xFFFFu);
+    if (!(role >> 16)) {
         out[pos] = clusters[i];
         return;
     }
     const uint32_t a = clusters[i], b = clusters[nearest[i]];
-    const uint32_t id = node_base + uint32_t(s >> 32) - 1u;
+    const uint32_t id = s.base + uint32_t(before >> 32) + (in_block >> 16);
     const float4 la = nlo[a], ha = nhi[a], lb = nlo[b], hb = nhi[b];
     float4 nl, nh;
     merge_nodes(a, b, la, ha, lb, hb, id, nl, nh, nlo, nhi, kids, wc, wd);
@@ -361,11 +419,11 @@ __global__ __launch_bounds__(kBB) void k_merge(const uint32_t *clusters, const u
 // CU.  Clustering 2.65 -> 2.1 ms.  2048 is what the LDS holds at two clusters a
 // thread; one iteration at that size costs what the launches of one cost.
 // out: root, node count, iterations, 1 if no progress was made.
-constexpr uint32_t kTailClusters = 2048;
 constexpr int kTailBlock = 1024;
-__global__ __launch_bounds__(kTailBlock) void k_ploc_tail(const uint32_t *clusters, uint32_t m, int R, uint32_t seed,
-                                                          uint32_t node_base, float4 *nlo, float4 *nhi, uint2 *kids,
-                                                          float4 *wc, uint32_t *wd, uint32_t *out) {
+__global__ __launch_bounds__(kTailBlock) void k_ploc_tail(const PlocState *st, ClusterBuffers cl, int R, float4 *nlo,
+                                                          float4 *nhi, uint2 *kids, float4 *wc, uint32_t *wd, uint32_t *out) {
+    const uint32_t *clusters = cl.buf[st->which];
+    uint32_t m = st->m, node_base = st->base, seed = st->iteration;
     __shared__ float4 lo[kTailClusters], hi[kTailClusters];
     __shared__ uint32_t id[kTailClusters], near[kTailClusters], wave_sum[kTailBlock / 64];
     const uint32_t t = threadIdx.x, wave = t / 64, lane = t % 64;
@@ -620,8 +678,8 @@ int bvh_gpu_plan(uint32_t n, uint32_t n_verts, hipStream_t stream, BuildArena *a
     arena->want(&b->cl, n);
     arena->want(&b->cl2, n);
     arena->want(&b->nearest, n);
-    arena->want(&b->flags, n);
-    arena->want(&b->incl, n);
+    arena->want(&b->sums, (size_t(n) + kMergeBlock - 1) / kMergeBlock);
+    arena->want(&b->ploc, 2);
     arena->want(&b->q, node_cap);
     arena->want(&b->q2, node_cap);
     arena->want(&b->ekid, node_cap);
@@ -633,11 +691,9 @@ int bvh_gpu_plan(uint32_t n, uint32_t n_verts, hipStream_t stream, BuildArena *a
     // library temporary storage, sized for the largest call
     WR_HIP(rocprim::radix_sort_pairs(nullptr, b->sort_bytes, (uint64_t *)nullptr, (uint64_t *)nullptr, (uint32_t *)nullptr,
                                      (uint32_t *)nullptr, n, 0, 63, stream));
-    WR_HIP(rocprim::inclusive_scan(nullptr, b->scan64_bytes, (uint64_t *)nullptr, (uint64_t *)nullptr, size_t(n),
-                                   rocprim::plus<uint64_t>(), stream));
     WR_HIP(rocprim::inclusive_scan(nullptr, b->scan32_bytes, (uint32_t *)nullptr, (uint32_t *)nullptr, node_cap,
                                    rocprim::plus<uint32_t>(), stream));
-    arena->want(&b->tmp, std::max(b->sort_bytes, std::max(b->scan64_bytes, b->scan32_bytes)));
+    arena->want(&b->tmp, std::max(b->sort_bytes, b->scan32_bytes));
     return WR_OK;
 }
 
@@ -683,8 +739,8 @@ int build_bvh4_gpu(wr_device *dev, const BuildBuffers &b, uint32_t n, hipStream_
     const float *d_verts = b.verts;
     const uint32_t *d_tris = b.tris, *d_tri_geom = b.tri_geom;
     float *partial = b.partial, *cbox = b.cbox;
-    uint64_t *keys = b.keys, *keys2 = b.keys2, *flags = b.flags, *incl = b.incl;
-    uint32_t *vals = b.vals, *order = b.order, *cl = b.cl, *cl2 = b.cl2, *nearest = b.nearest, *einner = b.einner,
+    uint64_t *keys = b.keys, *keys2 = b.keys2;
+    uint32_t *vals = b.vals, *order = b.order, *nearest = b.nearest, *einner = b.einner,
              *eincl = b.eincl, *tail = b.counts, *max_stack = b.counts + 4, *wd = b.wd;
     float4 *nlo = b.nlo, *nhi = b.nhi, *wc = b.wc;
     uint2 *kids = b.kids;
@@ -700,32 +756,28 @@ int build_bvh4_gpu(wr_device *dev, const BuildBuffers &b, uint32_t n, hipStream_
     WR_HIP(hipGetLastError());
     size_t bytes = b.sort_bytes;
     WR_HIP(rocprim::radix_sort_pairs(tmp, bytes, keys, keys2, vals, order, n, 0, 63, stream));
-    k_leaves<<<grid_of(n), kBB, 0, stream>>>(d_verts, d_tris, n, order, nlo, nhi, kids, wc, wd, cl);
+    k_leaves<<<grid_of(n), kBB, 0, stream>>>(d_verts, d_tris, n, order, nlo, nhi, kids, wc, wd, b.cl);
     WR_HIP(hipGetLastError());
 
     // PLOC
-    uint32_t m = n, node_base = n, iters = 0;
-    uint64_t total = 0;
-    while (m > kTailClusters) {
-        k_nearest<<<grid_of(m), kBB, 0, stream>>>(cl, m, nlo, nhi, R, iters, nearest);
-        k_merge_flags<<<grid_of(m), kBB, 0, stream>>>(nearest, m, flags);
-        WR_HIP(hipGetLastError());
-        bytes = b.scan64_bytes;
-        WR_HIP(rocprim::inclusive_scan(tmp, bytes, flags, incl, size_t(m), rocprim::plus<uint64_t>(), stream));
-        k_merge<<<grid_of(m), kBB, 0, stream>>>(cl, nearest, m, flags, incl, node_base, nlo, nhi, kids, wc, wd,
-                                                cl2);
-        WR_HIP(hipGetLastError());
-        WR_HIP(hipMemcpyAsync(&total, incl + (m - 1), sizeof total, hipMemcpyDeviceToHost, stream));
+    const ClusterBuffers cl{{b.cl, b.cl2}};
+    PlocState state{n, n, 0, 0, 0};
+    PlocState *d_state = b.ploc, *d_next = b.ploc + 1;
+    WR_HIP(hipMemcpyAsync(d_state, &state, sizeof state, hipMemcpyHostToDevice, stream));
+    while (state.m > kTailClusters) {
+        const uint32_t merge_blocks = (state.m + kMergeBlock - 1) / kMergeBlock;
+        for (int k = 0; k < kPlocBatch; k++) {
+            k_nearest<<<grid_of(state.m), kBB, 0, stream>>>(d_state, cl, nlo, nhi, R, nearest);
+            k_merge_count<<<merge_blocks, kMergeBlock, 0, stream>>>(d_state, nearest, b.sums);
+            k_merge<<<merge_blocks, kMergeBlock, 0, stream>>>(d_state, d_next, cl, nearest, b.sums, nlo, nhi, kids, wc, wd);
+            WR_HIP(hipGetLastError());
+            std::swap(d_state, d_next);
+        }
+        WR_HIP(hipMemcpyAsync(&state, d_state, sizeof state, hipMemcpyDeviceToHost, stream));
         WR_HIP(hipStreamSynchronize(stream));
-        const uint32_t merges = uint32_t(total >> 32), kept = uint32_t(total);
-        if (merges == 0 || kept != m - merges || node_base + merges > nn)
-            return set_error(WR_ERR_DEVICE, "GPU BVH build: clustering made no progress (non-finite vertices?)");
-        node_base += merges;
-        m = kept;
-        std::swap(cl, cl2);
-        iters++;
+        if (state.stuck) return set_error(WR_ERR_DEVICE, "GPU BVH build: clustering made no progress (non-finite vertices?)");
     }
-    k_ploc_tail<<<1, kTailBlock, 0, stream>>>(cl, m, R, iters, node_base, nlo, nhi, kids, wc, wd, tail);
+    k_ploc_tail<<<1, kTailBlock, 0, stream>>>(d_state, cl, R, nlo, nhi, kids, wc, wd, tail);
     WR_HIP(hipGetLastError());
     uint32_t ended[4];
     WR_HIP(hipMemcpyAsync(ended, tail, sizeof ended, hipMemcpyDeviceToHost, stream));
@@ -736,7 +788,7 @@ int build_bvh4_gpu(wr_device *dev, const BuildBuffers &b, uint32_t n, hipStream_
     WR_HIP(hipStreamSynchronize(stream));
     if (ended[3]) return set_error(WR_ERR_DEVICE, "GPU BVH build: clustering made no progress (non-finite vertices?)");
     if (ended[1] != nn) return set_error(WR_ERR_DEVICE, "GPU BVH build: node count mismatch");
-    iters = ended[2];
+    const uint32_t iters = ended[2];
     const uint4 q0 = make_uint4(ended[0], 0u, 0u, 0u);
     WR_HIP(hipMemcpyAsync(q, &q0, sizeof q0, hipMemcpyHostToDevice, stream));
     WR_HIP(hipMemsetAsync(max_stack, 0, sizeof(uint32_t), stream));

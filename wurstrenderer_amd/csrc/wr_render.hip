@@ -1365,7 +1365,7 @@ __global__ __launch_bounds__(kBlock) WR_EXTEND_ATTR(WR_BATCH_WAVES) void k_trace
 }
 // ============================================================== small passes
 // A pass of few samples, start to end in one launch.  Its iterations are bound
-// by the latency of their launches and queues (about 25 us each, of which a
+// by the latency of their launches and queues (about 28 us each, of which a
 // traversal over a short queue takes 12), so a block of two waves keeps 64 paths
 // in registers: the first wave starts them, traces their closest hits and
 // shades; the second traces the shadow rays that the first one left in LDS, at
