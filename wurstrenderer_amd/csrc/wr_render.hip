@@ -7,21 +7,23 @@
 //
 //   regen     start the next unclaimed samples behind the continuing paths:
 //             light vertex, camera ray, light->camera (t = 1) connection
-//   extend    closest hit for every active path                (BVH4 traversal)
+//   trace     closest hit for every active path, and any hit for the NEE and
+//             t = 1 rays of the iteration before; visible ones add their
+//             contribution (quantised BVH4 traversal)
 //   shade     emitter hit with MIS, NEE with MIS, BSDF sample; continuing paths
 //             are compacted into the next state, a finished path stores its
-//             radiance under its sample index
-//   shadow    any hit for NEE and t = 1 rays; add visible contributions
-//   rotate    the next state becomes current (device-side counters)
+//             radiance under its sample index; the last block to finish ends
+//             the iteration (the next state becomes current)
 //   (per pass) accumulate: per-pixel FP64 sums of the samples' radiance
 //
 // Refilling the pool as paths end keeps every kernel's queue full until the
 // last samples drain.  Path state is stored in queue order, so every kernel
-// reads and writes it contiguously; compaction is one atomic per wave (ballot
-// + mbcnt).  Every kernel reads its work count from device memory, and the
-// host polls the counters only every few iterations.  Radiance is gathered in
-// FP32 per path and summed per pixel in FP64 in sample order (reproducible);
-// t = 1 splats go to the FP64 splat film with atomics.
+// reads and writes it contiguously; compaction is one atomic per block of up to
+// 512 threads.  Every kernel reads its work count from device memory, and the
+// host follows a pass through a pinned progress word that the device writes.
+// Small passes take one kernel from start to end instead (k_small_pass).
+// Radiance is gathered in FP32 per path and summed per pixel in FP64 in sample
+// order (reproducible); t = 1 splats go to the FP64 splat film with atomics.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -2683,9 +2685,8 @@ static uint64_t default_pool_fit(const wr_scene *s, uint64_t want, uint64_t samp
 
 // Runs wavefront iterations until the pool drains and both shadow queues are
 // traced.  launch(pb) issues one iteration (refill, one traversal launch for
-// the closest-hit rays and the previous shadow queue, shade, rotate) for the
-// state pb; the host
-// polls the device counters every kPoll iterations.  With a graph, the two
+// the closest-hit rays and the previous shadow queue, shade) for the state pb;
+// without `progress` the host polls the device counters every kPoll iterations.  With a graph, the two
 // iterations of a state round trip (cur -> next -> cur) are captured once and
 // replayed, so a pass costs one graph launch per two iterations.  Every
 // kernel reads its work counts from device memory, which is what makes the
