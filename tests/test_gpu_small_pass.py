@@ -51,6 +51,17 @@ def test_small_passes_equal_the_queues(gpu_device, kind, size, spp, vertices):
         assert a[2:] == b[2:]
 
 
+@pytest.mark.parametrize("vertices", [255, 256, 300])
+def test_more_vertices_than_the_bounce_counter_holds(gpu_device, vertices):
+    """Above 255 vertices the queues render the pass, which bound the iterations
+    of paths that the 8-bit bounce counter would never end (open scene: all end)."""
+    print(f"small pass: spheres, {vertices} vertices", flush=True)
+    gs = wr.GpuScene(gpu_device, SCENES["spheres"]((33, 17)))
+    a, b = _films(gs, wr.render_nee, 33 * 17, 1, num_path_vertices=vertices)
+    np.testing.assert_array_equal(a[0], b[0])
+    assert a[2:] == b[2:]
+
+
 @pytest.mark.parametrize("spp", [16, 17])
 def test_shares_up_to_the_limit_of_a_tiny_scene(gpu_device, spp):
     print(f"small pass: cornell 512x512 spp={spp}", flush=True)

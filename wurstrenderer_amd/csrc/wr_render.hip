@@ -2930,8 +2930,11 @@ static int render_impl(wr_scene *s, wr_film *f, const wr_render_params *prm, wr_
     const int g_infer = std::max(1, std::min<int>((P + kInferBlock - 1) / kInferBlock,
                                                   s->dev->n_cu * occupancy(s->dev, infer_fn, kInferBlock)));
     // passes that k_small_pass takes: the plain estimators, unless traversal
-    // counters, per-kernel times or graph replays of the iterations are asked for
-    const bool small_passes = est != kEstLight && !g && !medium && !count && !prof && !use_graph;
+    // counters, per-kernel times or graph replays of the iterations are asked for.
+    // A path's bounce is kept in 8 bits: with more vertices than that nothing but
+    // the limit on iterations ends the paths of a closed scene, and only the
+    // queues have one.
+    const bool small_passes = est != kEstLight && !g && !medium && !count && !prof && !use_graph && N <= int(kBounceMask);
     const void *small_fn = env ? reinterpret_cast<const void *>(&k_small_pass<true>) : reinterpret_cast<const void *>(&k_small_pass<false>);
     const uint32_t small_blocks = uint32_t(s->dev->n_cu * occupancy(s->dev, small_fn, 2 * kBlock));
     const uint32_t small_slices = uint32_t(fixed ? fixed->trav_blocks : s->max_trav_blocks) / 2;
