@@ -181,6 +181,7 @@ struct wr_device {
     int n_cu = 256;
     // resident blocks per CU of each kernel (HIP occupancy API), used to size persistent grids
     int occ_rays = 8, occ_shade = 8, occ_generate = 8, occ_trace = 8;
+    std::mutex occ_mutex;  // guards occ_cache
     std::map<const void *, int> occ_cache;  // other kernels, filled on first use
     BlockPool spills{2, size_t(1) << 30};       // traversal stack spill regions, one per scene
     BlockPool geometry{3, size_t(512) << 20, true};  // nodes (both copies) and triangles of GPU-built scenes

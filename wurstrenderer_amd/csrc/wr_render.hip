@@ -1897,6 +1897,7 @@ __global__ __launch_bounds__(kBlock, 4) void k_bdpt(DScene s, uint32_t wh, uint3
 
 // Resident blocks per CU of a kernel (HIP occupancy API), cached per device.
 static int occupancy(wr_device *d, const void *fn, int block) {
+    std::lock_guard<std::mutex> lock(d->occ_mutex);  // scenes of one device may render in several threads
     auto it = d->occ_cache.find(fn);
     if (it != d->occ_cache.end()) return it->second;
     int nb = 0;
