@@ -181,8 +181,12 @@ __global__ void k_init(PathBuffers pb, RenderArgs a) {
 // launch gap aside).  Thread 0 did its block's appends and holds their
 // results, so they are done when it takes a ticket, and no fence (which would
 // write back and invalidate the XCD's L2) is needed: what the last block reads
-// is either older than this kernel or read with an atomic.
+// is either older than this kernel or read with an atomic.  The barrier keeps
+// the block's other waves ahead of its ticket: each wave reads the number of
+// active paths, two words that the last block rewrites, when it starts, and in a
+// block without work no append's barrier follows that read.
 __device__ __forceinline__ void end_iteration(const PathBuffers &pb, const RenderArgs &a) {
+    __syncthreads();
     if (threadIdx.x != 0) return;
     uint32_t *c = pb.counters;
     if (atomicAdd(&c[kTicket], 1u) != gridDim.x - 1) return;
