@@ -1327,10 +1327,10 @@ __device__ __forceinline__ void shadow_rays(DScene s1, const BatchJob *__restric
                     atomicAdd(dst + 1, double(c.y));
                     atomicAdd(dst + 2, double(c.z));
                 } else {
-                    float4 *r = (target & ~kTargetMask) == kToSample ? pb.sample_rad + idx : pb.cur.rad + idx;
-                    float4 rr = *r;
-                    rr.x += c.x; rr.y += c.y; rr.z += c.z;
-                    *r = rr;
+                    // the three sums alone: other waves of this launch read a path's fourth word, its job
+                    float *r = &((target & ~kTargetMask) == kToSample ? pb.sample_rad + idx : pb.cur.rad + idx)->x;
+                    const float rx = r[0] + c.x, ry = r[1] + c.y, rz = r[2] + c.z;
+                    r[0] = rx; r[1] = ry; r[2] = rz;
                 }
             }
         }
