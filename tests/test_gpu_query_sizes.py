@@ -1,0 +1,64 @@
+"""Ray queries at the sizes where their route changes: up to 32,768 rays are read from
+pinned memory by the kernel, up to 1,310,720 hits and 15,728,640 flags are written
+there.  Everything is exact, so comparisons are too."""
+import time
+
+import numpy as np
+import pytest
+
+import wurstrenderer_amd as wr
+from wurstrenderer_amd import scenes
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n", [1, 64, 32_767, 32_768, 32_769, 87_382, 349_526, 1_310_720, 1_310_721])
+def test_hits_equal_those_of_parts(gpu_device, n):
+    """A query gives what the same rays give in pieces of 10,007."""
+    print(f"query: {n} rays", flush=True)
+    sc = scenes.icospheres(2, n_spheres=6, level=3, resolution=(8, 8))
+    gs = wr.GpuScene(gpu_device, sc)
+    rays = np.concatenate([scenes.random_rays(sc, (n + 1) // 2, seed=1), scenes.random_rays(sc, n // 2, seed=2, inside=True)])
+    rays[:, 7] = np.where(np.arange(n) % 3 == 0, 4.0, np.inf)
+    whole, flags = gs.trace_closest(rays), gs.trace_any(rays)
+    for at in range(0, n, 10_007):
+        part = rays[at:at + 10_007]
+        for a, b in zip(whole, gs.trace_closest(part)):
+            np.testing.assert_array_equal(a[at:at + 10_007], b)
+        np.testing.assert_array_equal(flags[at:at + 10_007], gs.trace_any(part))
+    assert 0 < flags.sum() < n or n == 1
+
+
+def test_flags_above_the_pinned_limit(gpu_device):
+    n = 15 * (1 << 20) + 1
+    print(f"query: {n} flags", flush=True)
+    sc = scenes.cornell(1, (8, 8))
+    gs = wr.GpuScene(gpu_device, sc)
+    part = scenes.random_rays(sc, 30_011, seed=3)
+    part[:, 7] = 3.0
+    rays = np.resize(part, (n, 8))
+    want = gs.trace_any(part)
+    for m in (n - 1, n):
+        np.testing.assert_array_equal(gs.trace_any(rays[:m]), np.resize(want, m))
+
+
+def test_a_small_query_is_one_launch_and_one_wait(gpu_device):
+    """1,000 hits take 28 us and a plain copy of 31 KB (Guide.get_params) 13 us; with
+    a wait for each array's own transfer the query took 102, with two waits and the
+    host's lookup 61.  Shortest of many, so that other load does not count."""
+    sc = scenes.cornell(1, (8, 8))
+    gs = wr.GpuScene(gpu_device, sc)
+    guide = wr.Guide(gs)
+    rays = scenes.random_rays(sc, 1000, seed=1)
+
+    def shortest(call):
+        best = np.inf
+        for _ in range(300):
+            t = time.perf_counter()
+            call()
+            best = min(best, time.perf_counter() - t)
+        return best
+
+    query, copy = shortest(lambda: gs.trace_closest(rays)), shortest(guide.get_params)
+    print(f"query {query * 1e6:.1f} us, copy {copy * 1e6:.1f} us", flush=True)
+    assert query < 4 * copy

@@ -32,6 +32,7 @@ struct TransferRing {
     static constexpr int kSlots = 16, kThreads = 8;
     static constexpr size_t kChunk = size_t(1) << 20, kThreadedBytes = size_t(3) << 20;
     static_assert(kSlots % kThreads == 0, "a slot belongs to one thread");
+    static int threads_for(size_t bytes) { return bytes < kThreadedBytes ? 1 : kThreads; }
 
     std::mutex busy;
     char *pinned = nullptr;
@@ -52,8 +53,30 @@ struct TransferRing {
     template <class Issue>
     hipError_t download(int ordinal, hipStream_t stream, void *dst, size_t bytes, Issue &&issue) {
         char *out = static_cast<char *>(dst);
-        return run(ordinal, stream, bytes, true, issue,
+        return run(ordinal, stream, bytes, threads_for(bytes), true, issue,
                    [out](size_t off, size_t n, char *slot) { std::memcpy(out + off, slot, n); });
+    }
+    // The same for arrays in device memory, each to its own place on the host, in
+    // one transfer: the host copies one array while the device copies the next.
+    struct Out { void *dst; const void *src; size_t bytes; };
+    hipError_t download(int ordinal, hipStream_t stream, std::initializer_list<Out> parts) {
+        size_t total = 0;
+        for (const Out &p : parts) total += p.bytes;
+        return run(
+            ordinal, stream, total, threads_for(total), true,
+            [&parts, stream](size_t off, size_t n, char *slot) {
+                hipError_t e = hipSuccess;
+                pieces(parts, off, n, slot, [&](const Out &p, size_t at, char *piece, size_t m) {
+                    if (e == hipSuccess)
+                        e = hipMemcpyAsync(piece, static_cast<const char *>(p.src) + at, m, hipMemcpyDeviceToHost, stream);
+                });
+                return e;
+            },
+            [&parts](size_t off, size_t n, char *slot) {
+                pieces(parts, off, n, slot, [](const Out &p, size_t at, char *piece, size_t m) {
+                    std::memcpy(static_cast<char *>(p.dst) + at, piece, m);
+                });
+            });
     }
     // Host to device on `stream`: the parts, one behind the other.  The sources
     // may be reused when it returns, and the copies are complete.
@@ -63,42 +86,93 @@ struct TransferRing {
         size_t total = 0;
         for (const Part &p : parts) total += p.bytes;
         return run(
-            ordinal, stream, total, false,
+            ordinal, stream, total, threads_for(total), false,
             [out, stream](size_t off, size_t n, char *slot) {
                 return hipMemcpyAsync(out + off, slot, n, hipMemcpyHostToDevice, stream);
             },
             [&parts](size_t off, size_t n, char *slot) {
-                for (const Part &p : parts) {  // the piece of each part that lies in [off, off + n)
-                    const size_t m = off < p.bytes ? std::min(n, p.bytes - off) : 0;
-                    if (m) std::memcpy(slot, static_cast<const char *>(p.src) + off, m);
-                    slot += m;
-                    n -= m;
-                    off = off < p.bytes ? 0 : off - p.bytes;
-                }
+                pieces(parts, off, n, slot, [](const Part &p, size_t at, char *piece, size_t m) {
+                    std::memcpy(piece, static_cast<const char *>(p.src) + at, m);
+                });
             });
     }
-    hipError_t upload(int ordinal, hipStream_t stream, void *device, const void *src, size_t bytes) {
-        return upload(ordinal, stream, device, {Part{src, bytes}});
+    // The ring for one caller, whose kernel reads and writes pinned memory directly:
+    // a chunk `in` and kSlots - 1 chunks `out`, until the lease dies.  The caller
+    // waits for its stream before that.
+    static constexpr size_t kLeaseIn = kChunk, kLeaseOut = (kSlots - 1) * kChunk;
+    struct Lease {
+        std::unique_lock<std::mutex> lock;
+        char *in = nullptr, *out = nullptr;
+    };
+    hipError_t lease(Lease *l) {
+        l->lock = std::unique_lock<std::mutex>(busy);
+        const hipError_t e = allocate();
+        if (e != hipSuccess) return e;
+        l->in = pinned;
+        l->out = pinned + kLeaseIn;
+        return hipSuccess;
+    }
+    // Host copies of the parts, by several threads from kThreadedBytes on.
+    static void copy(std::initializer_list<Out> parts) {
+        constexpr size_t kPiece = kChunk / 4;
+        size_t total = 0;
+        for (const Out &p : parts) total += p.bytes;
+        const int threads = threads_for(total);
+        on_threads(threads, [&](int t) {
+            for (size_t off = size_t(t) * kPiece; off < total; off += size_t(threads) * kPiece)
+                pieces(parts, off, std::min(kPiece, total - off), nullptr, [](const Out &p, size_t at, char *, size_t m) {
+                    std::memcpy(static_cast<char *>(p.dst) + at, static_cast<const char *>(p.src) + at, m);
+                });
+        });
     }
 
 private:
+    // The ring's memory, on first use; `busy` is held.
+    hipError_t allocate() {
+        if (pinned) return hipSuccess;
+        const hipError_t e = hipHostMalloc(reinterpret_cast<void **>(&pinned), kSlots * kChunk, hipHostMallocDefault);
+        if (e != hipSuccess) pinned = nullptr;
+        return e;
+    }
+    // work(0) ... work(threads - 1), on the calling thread and as many others as can be had.
+    template <class Work>
+    static void on_threads(int threads, Work &&work) {
+        std::vector<std::thread> pool;
+        int started = 1;
+        try {
+            pool.reserve(size_t(threads));
+            for (; started < threads; started++) pool.emplace_back([&work, started] { work(started); });
+        } catch (const std::exception &) {  // no thread to be had: the calling one does the rest
+        }
+        work(0);
+        for (int t = started; t < threads; t++) work(t);
+        for (std::thread &t : pool) t.join();
+    }
+    // Calls f(part, offset in the part, slot address, bytes) for the piece of each
+    // part that lies in bytes [off, off + n) of all parts laid end to end.
+    template <class P, class F>
+    static void pieces(std::initializer_list<P> parts, size_t off, size_t n, char *slot, F &&f) {
+        for (const P &p : parts) {
+            const size_t m = off < p.bytes ? std::min(n, p.bytes - off) : 0;
+            if (m) f(p, off, slot, m);
+            if (slot) slot += m;
+            n -= m;
+            off = off < p.bytes ? 0 : off - p.bytes;
+        }
+    }
     // Per chunk, device(offset, bytes, slot) enqueues its device work and
     // host(offset, bytes, slot) does its host copy; `down`: device first.
     template <class Device, class Host>
-    hipError_t run(int ordinal, hipStream_t stream, size_t bytes, bool down, Device &&device, Host &&host) {
+    hipError_t run(int ordinal, hipStream_t stream, size_t bytes, int threads, bool down, Device &&device, Host &&host) {
         if (bytes == 0) return hipSuccess;
         std::lock_guard<std::mutex> lock(busy);
-        if (!pinned) {
-            hipError_t e = hipHostMalloc(reinterpret_cast<void **>(&pinned), kSlots * kChunk, hipHostMallocDefault);
-            if (e != hipSuccess) { pinned = nullptr; return e; }
-        }
+        if (const hipError_t e = allocate(); e != hipSuccess) return e;
         const size_t chunks = (bytes + kChunk - 1) / kChunk;
         for (size_t k = 0; k < std::min<size_t>(chunks, kSlots); k++)
             if (!done[k]) {
                 hipError_t e = hipEventCreateWithFlags(&done[k], hipEventDisableTiming);
                 if (e != hipSuccess) { done[k] = nullptr; return e; }
             }
-        const int threads = bytes < kThreadedBytes ? 1 : kThreads;
         std::atomic<int> first_error{hipSuccess};
         auto note = [&](hipError_t e) {
             int none = hipSuccess;
@@ -136,16 +210,7 @@ private:
                 for (; next < issued; next += threads) (void)wait(next);
             }
         };
-        std::vector<std::thread> pool;
-        int started = 1;
-        try {
-            pool.reserve(size_t(threads));
-            for (; started < threads; started++) pool.emplace_back(work, started);
-        } catch (const std::exception &) {  // no thread to be had: the calling one does the rest
-        }
-        work(0);
-        for (int t = started; t < threads; t++) work(t);
-        for (std::thread &t : pool) t.join();
+        on_threads(threads, work);
         return hipError_t(first_error.load());
     }
 };
