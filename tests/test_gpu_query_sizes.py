@@ -1,6 +1,9 @@
-"""Ray queries at the sizes where their route changes: up to 32,768 rays are read from
-pinned memory by the kernel, up to 1,310,720 hits and 15,728,640 flags are written
-there.  Everything is exact, so comparisons are too."""
+"""Ray queries and film reads at the sizes where their route changes.
+
+Rays: up to 32,768 are read from pinned memory by the kernel; up to 1,310,720 hits
+and 15,728,640 flags are written there.  Films: arrays up to 16 KB and from 1.2 MB
+on (26^2 and 27^2, 223^2 and 224^2 pixels) come through the pinned ring, those in
+between by plain copies.  Everything is exact, so comparisons are too."""
 import time
 
 import numpy as np
@@ -40,6 +43,21 @@ def test_flags_above_the_pinned_limit(gpu_device):
     want = gs.trace_any(part)
     for m in (n - 1, n):
         np.testing.assert_array_equal(gs.trace_any(rays[:m]), np.resize(want, m))
+
+
+@pytest.mark.parametrize("size", [1, 26, 27, 40, 223, 224, 361])
+def test_film_reads_equal_single_arrays(gpu_device, size):
+    print(f"film read: {size}", flush=True)
+    gs = wr.GpuScene(gpu_device, scenes.cornell(1, (size, size)))
+    film = wr.Film(gs)
+    wr.render_nee(gs, film, 2, num_path_vertices=4, seed=1)
+    base, splat = film.read()
+    alone = np.empty_like(base)
+    for want, args in ((base, (alone.ctypes.data, None)), (splat, (None, alone.ctypes.data))):
+        alone[:] = -1.0
+        assert wr.lib().wr_film_read(film.h, *args) == 0
+        np.testing.assert_array_equal(alone, want)
+    np.testing.assert_array_equal(film.image(), base / 2 + splat / (2 * size * size))
 
 
 def test_a_small_query_is_one_launch_and_one_wait(gpu_device):

@@ -2567,13 +2567,7 @@ int wr_film_read(wr_film *f, double *base, double *splat) {
     if (rc) return rc;
     const size_t bytes = sizeof(double) * 3 * size_t(f->W) * f->H;
     hipStream_t st = f->scene->stream;
-    for (auto &[dst, src] : {std::make_pair(base, f->d_base), std::make_pair(splat, f->d_splat)}) {
-        if (!dst) continue;
-        const char *from = reinterpret_cast<const char *>(src);
-        WR_HIP(dev->ring.download(dev->ordinal, st, dst, bytes, [&](size_t off, size_t n, char *slot) {
-            return hipMemcpyAsync(slot, from + off, n, hipMemcpyDeviceToHost, st);
-        }));
-    }
+    WR_HIP(dev->ring.download(dev->ordinal, st, {{base, f->d_base, base ? bytes : 0}, {splat, f->d_splat, splat ? bytes : 0}}));
     WR_HIP(hipStreamSynchronize(st));
     return WR_OK;
 }
