@@ -200,8 +200,8 @@ private:
             return note(device(c * kChunk, size_of(c), slot_of(c))) && note(hipEventRecord(done[c % kSlots], stream));
         };
         auto wait = [&](size_t c) { return note(hipEventSynchronize(done[c % kSlots])); };
-        // chunks t, t + threads, ...; whatever happens, every event the thread
-        // recorded is waited for before it returns
+        // chunks t, t + threads, ...; every event the thread recorded is waited for
+        // before it returns
         auto work = [&](int t) {
             if (!note(hipSetDevice(ordinal))) return;
             size_t issued = size_t(t), next = size_t(t);
@@ -216,7 +216,7 @@ private:
             } else {
                 for (; issued < chunks && first_error == hipSuccess; issued += threads) {
                     if (issued >= size_t(kSlots)) {
-                        (void)wait(next);
+                        if (!wait(next)) break;  // the slot may still be read
                         next += threads;
                     }
                     host(issued * kChunk, size_of(issued), slot_of(issued));
@@ -226,6 +226,9 @@ private:
             }
         };
         on_threads(threads, work);
+        // after a failure there may be device work that no event stands for: nothing
+        // may use the slots or the caller's memory once this returns
+        if (first_error != hipSuccess) (void)hipStreamSynchronize(stream);
         return hipError_t(first_error.load());
     }
 };
