@@ -27,3 +27,14 @@ def transfer_check(tmp_path_factory):
 def test_transfers_that_fail_leave_nothing_in_flight(transfer_check, direction, what, call, megabytes):
     r = subprocess.run([transfer_check, direction, what, str(call), str(megabytes)], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, (r.returncode, r.stdout)
+
+
+@pytest.fixture(scope="module")
+def pool_check(tmp_path_factory):
+    return _build(tmp_path_factory, "pool_check")
+
+
+@pytest.mark.parametrize("check", ["give_without_host_memory", "keeps_the_largest", "close_fit", "full_device"])
+def test_blocks_kept_by_a_device_handle(pool_check, check):
+    r = subprocess.run([pool_check, check], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, (r.returncode, r.stdout, r.stderr)

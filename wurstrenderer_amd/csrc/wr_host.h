@@ -13,6 +13,7 @@
 #include "../../include/wurst_amd.h"
 #include "wr_device.h"
 #include "wr_layout.h"
+#include "wr_memory.h"
 #include "wr_transfer.h"
 
 namespace wr {
@@ -116,100 +117,13 @@ struct RenderArgs {
 };
 
 // ============================================================== host objects
-// Device memory that outlives the calls which use it, kept by a device handle.
-// A caller takes a block and gives it back when its stream has finished with
-// it; blocks are handed to one caller at a time, so streams and threads never
-// share one, and at most `keep` free blocks of at most `most` bytes are held.
-struct BlockPool {
-    struct Block { void *p = nullptr; size_t bytes = 0; };
-    int keep;
-    size_t most;
-    bool close_fit;  // blocks of more than twice the size asked for are not handed out
-    std::mutex m;
-    std::vector<Block> free_blocks;
-    BlockPool(int keep_, size_t most_, bool close_fit_ = false) : keep(keep_), most(most_), close_fit(close_fit_) {}
-    ~BlockPool() {
-        for (Block &b : free_blocks) (void)hipFree(b.p);
-    }
-    // the smallest free block of at least `bytes`, else a new one
-    hipError_t take(size_t bytes, Block *out) {
-        {
-            std::lock_guard<std::mutex> lock(m);
-            size_t best = free_blocks.size();
-            for (size_t i = 0; i < free_blocks.size(); i++)
-                if (free_blocks[i].bytes >= bytes && (!close_fit || free_blocks[i].bytes / 2 <= bytes) &&
-                    (best == free_blocks.size() || free_blocks[i].bytes < free_blocks[best].bytes))
-                    best = i;
-            if (best < free_blocks.size()) {
-                *out = free_blocks[best];
-                free_blocks.erase(free_blocks.begin() + long(best));
-                return hipSuccess;
-            }
-        }
-        const hipError_t e = hipMalloc(&out->p, bytes);
-        if (e != hipSuccess) out->p = nullptr;
-        out->bytes = e == hipSuccess ? bytes : 0;
-        return e;
-    }
-    // gives every free block back to the runtime
-    void trim() {
-        std::lock_guard<std::mutex> lock(m);
-        for (Block &b : free_blocks) (void)hipFree(b.p);
-        free_blocks.clear();
-    }
-    void give(Block b) {
-        if (!b.p) return;
-        Block drop = b;
-        if (b.bytes <= most) {
-            std::lock_guard<std::mutex> lock(m);
-            free_blocks.push_back(b);
-            drop = Block{};
-            if (int(free_blocks.size()) > keep) {  // the smallest goes
-                size_t k = 0;
-                for (size_t i = 1; i < free_blocks.size(); i++)
-                    if (free_blocks[i].bytes < free_blocks[k].bytes) k = i;
-                drop = free_blocks[k];
-                free_blocks.erase(free_blocks.begin() + long(k));
-            }
-        }
-        if (drop.p) (void)hipFree(drop.p);
-    }
-};
-
-struct wr_device {
+struct wr_device : wr::DeviceMemory {
     int ordinal = 0;
     int n_cu = 256;
     // resident blocks per CU of each kernel (HIP occupancy API), used to size persistent grids
     int occ_rays = 8, occ_shade = 8, occ_generate = 8, occ_trace = 8;
     std::mutex occ_mutex;  // guards occ_cache
     std::map<const void *, int> occ_cache;  // other kernels, filled on first use
-    BlockPool spills{2, size_t(1) << 30};       // traversal stack spill regions, one per scene
-    BlockPool geometry{3, size_t(512) << 20, true};  // nodes (both copies) and triangles of GPU-built scenes
-    BlockPool build_memory{1, size_t(1) << 30}; // mesh copies and scratch of BVH builds
-    void trim() {
-        spills.trim();
-        geometry.trim();
-        build_memory.trim();
-    }
-    // hipMalloc that frees the pools' idle blocks where memory runs out
-    hipError_t alloc(void **p, size_t bytes) {
-        hipError_t e = hipMalloc(p, bytes);
-        if (e == hipErrorOutOfMemory) {
-            (void)hipGetLastError();
-            trim();
-            e = hipMalloc(p, bytes);
-        }
-        return e;
-    }
-    hipError_t take(BlockPool &pool, size_t bytes, BlockPool::Block *b) {
-        hipError_t e = pool.take(bytes, b);
-        if (e == hipErrorOutOfMemory) {
-            (void)hipGetLastError();
-            trim();
-            e = pool.take(bytes, b);
-        }
-        return e;
-    }
     TransferRing ring;        // pinned buffers of large host transfers
     void *scratch = nullptr;  // device address of wr_render_nee_noalloc's fixed region on this GPU
 };
