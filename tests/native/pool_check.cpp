@@ -62,7 +62,7 @@ static int full_device() {
     mem.geometry.give(b);
     mem.build_memory.give(c);
     void *p = nullptr;
-    if (mem.alloc(&p, 950) != hipSuccess || fake::used != 950) return 2;
+    if (mem.idle() != 900 || mem.alloc(&p, 950) != hipSuccess || mem.idle() != 0 || fake::used != 950) return 2;
     if (mem.alloc(&p, 100) != hipErrorOutOfMemory) return 3;
     return 0;
 }

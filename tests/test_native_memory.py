@@ -38,3 +38,11 @@ def pool_check(tmp_path_factory):
 def test_blocks_kept_by_a_device_handle(pool_check, check):
     r = subprocess.run([pool_check, check], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, (r.returncode, r.stdout, r.stderr)
+
+
+def test_every_device_allocation_can_use_idle_blocks():
+    """hipMalloc is called in wr_memory.h alone: an allocation elsewhere would fail
+    while a device handle holds idle blocks that it could have had."""
+    csrc = os.path.join(os.path.dirname(HERE), "wurstrenderer_amd", "csrc")
+    users = {f for f in os.listdir(csrc) if "hipMalloc(" in open(os.path.join(csrc, f)).read()}
+    assert users == {"wr_memory.h"}

@@ -713,7 +713,7 @@ int mesh_check_gpu(const BuildBuffers &b, uint32_t n, uint32_t n_verts, uint32_t
 }
 
 // The Node4 of a scene without triangles.
-static int empty_bvh(GpuBvhResult *res) {
+static int empty_bvh(wr_device *dev, GpuBvhResult *res) {
     Node4 nd;
     for (int i = 0; i < 4; i++) {
         nd.lo_x[i] = nd.lo_y[i] = nd.lo_z[i] = FLT_MAX;
@@ -721,8 +721,8 @@ static int empty_bvh(GpuBvhResult *res) {
         nd.child[i] = kEmptyChild;
         nd.count[i] = 0;
     }
-    WR_HIP(hipMalloc(&res->nodes, sizeof(Node4)));
-    WR_HIP(hipMalloc(&res->tris, 128));
+    WR_HIP(dev->alloc(reinterpret_cast<void **>(&res->nodes), sizeof(Node4)));
+    WR_HIP(dev->alloc(reinterpret_cast<void **>(&res->tris), 128));
     WR_HIP(hipMemcpy(res->nodes, &nd, sizeof(Node4), hipMemcpyHostToDevice));
     res->n_nodes = 1;
     res->max_stack = 1;
@@ -734,7 +734,7 @@ int build_bvh4_gpu(wr_device *dev, const BuildBuffers &b, uint32_t n, hipStream_
     *res = GpuBvhResult{};
     const int R = radius > 0 ? std::min(radius, kPlocRadiusMax) : kPlocRadius;
     const auto t0 = std::chrono::steady_clock::now();
-    if (n == 0) return empty_bvh(res);
+    if (n == 0) return empty_bvh(dev, res);
     const size_t nn = 2 * size_t(n) - 1, node_cap = n;
     const float *d_verts = b.verts;
     const uint32_t *d_tris = b.tris, *d_tri_geom = b.tri_geom;

@@ -88,14 +88,16 @@ __global__ void k_debug_camera_we1(DCamera cam, const float *org, const float *w
 
 // Device staging for one call: inputs copied in, outputs copied out, all freed.
 struct Staging {
+    wr_device *dev;
     std::vector<void *> ptrs;
+    explicit Staging(wr_device *d) : dev(d) {}
     ~Staging() {
         for (void *p : ptrs) (void)hipFree(p);
     }
     template <class T>
     int in(T **dst, const void *src, size_t bytes) {
         *dst = nullptr;
-        WR_HIP(hipMalloc(reinterpret_cast<void **>(dst), bytes ? bytes : 4));
+        WR_HIP(dev->alloc(reinterpret_cast<void **>(dst), bytes ? bytes : 4));
         ptrs.push_back(*dst);
         if (bytes) WR_HIP(hipMemcpy(*dst, src, bytes, hipMemcpyHostToDevice));
         return WR_OK;
@@ -103,7 +105,7 @@ struct Staging {
     template <class T>
     int out(T **dst, size_t bytes) {
         *dst = nullptr;
-        WR_HIP(hipMalloc(reinterpret_cast<void **>(dst), bytes ? bytes : 4));
+        WR_HIP(dev->alloc(reinterpret_cast<void **>(dst), bytes ? bytes : 4));
         ptrs.push_back(*dst);
         return WR_OK;
     }
@@ -156,7 +158,7 @@ int wr_debug_bsdf_eval(wr_device *dev, const wr_material *mats, const float *wi,
     std::vector<DMat> dm;
     if (int rc = to_dmats(mats, n, dm)) return rc;
     if (int rc = set_device(dev)) return rc;
-    Staging S;
+    Staging S(dev);
     DMat *d_m; float *d_wi, *d_wo, *d_f, *d_p;
     const size_t v3 = sizeof(float) * 3 * size_t(n);
     if (int rc = S.in(&d_m, dm.data(), sizeof(DMat) * n)) return rc;
@@ -179,7 +181,7 @@ int wr_debug_bsdf_sample(wr_device *dev, const wr_material *mats, const float *w
     std::vector<DMat> dm;
     if (int rc = to_dmats(mats, n, dm)) return rc;
     if (int rc = set_device(dev)) return rc;
-    Staging S;
+    Staging S(dev);
     DMat *d_m; float *d_wi, *d_u, *d_wo, *d_w, *d_p;
     const size_t v3 = sizeof(float) * 3 * size_t(n);
     if (int rc = S.in(&d_m, dm.data(), sizeof(DMat) * n)) return rc;
@@ -201,7 +203,7 @@ int wr_debug_light_sample(wr_scene *s, const float *u, uint32_t n, float *pos, f
     if (s->ds.n_lights == 0) return set_error(WR_ERR_INVALID_ARGUMENT, "scene has no area lights");
     if (n == 0) return WR_OK;
     if (int rc = set_device(s->dev)) return rc;
-    Staging S;
+    Staging S(s->dev);
     float *d_u, *d_pos, *d_n, *d_c, *d_p;
     const size_t v3 = sizeof(float) * 3 * size_t(n);
     if (int rc = S.in(&d_u, u, sizeof(float) * 2 * size_t(n))) return rc;
@@ -228,7 +230,7 @@ int wr_debug_camera_ray(wr_scene *s, const uint32_t *pixel, const float *ulens, 
             return set_error(WR_ERR_INVALID_ARGUMENT, "pixel outside the film");
     if (n == 0) return WR_OK;
     if (int rc = set_device(s->dev)) return rc;
-    Staging S;
+    Staging S(s->dev);
     uint32_t *d_px;
     float *d_ul, *d_up, *d_o, *d_d, *d_p;
     const size_t v2 = sizeof(float) * 2 * size_t(n), v3 = sizeof(float) * 3 * size_t(n);
@@ -250,7 +252,7 @@ int wr_debug_camera_we1(wr_scene *s, const float *org, const float *w, uint32_t 
     if (!s || (n && (!org || !w || !we1 || !raster))) return set_error(WR_ERR_INVALID_ARGUMENT, "null argument");
     if (n == 0) return WR_OK;
     if (int rc = set_device(s->dev)) return rc;
-    Staging S;
+    Staging S(s->dev);
     float *d_o, *d_w, *d_we, *d_r;
     const size_t v3 = sizeof(float) * 3 * size_t(n);
     if (int rc = S.in(&d_o, org, v3)) return rc;
@@ -277,7 +279,7 @@ int wr_debug_l1_request_probe(wr_device *dev, uint64_t footprint, uint32_t loads
     WR_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void *>(&k_debug_l1_probe),
                                                         kDebugBlock, 0));
     const uint32_t grid = uint32_t(dev->n_cu) * uint32_t(std::max(1, per_cu));
-    Staging S;
+    Staging S(dev);
     uint4 *d_buf;
     uint32_t *d_sink;
     if (int rc = S.out(&d_buf, size_t(footprint))) return rc;

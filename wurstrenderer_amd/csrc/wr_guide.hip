@@ -851,7 +851,7 @@ int guide_reserve_draws(wr_guide *g, uint32_t capacity) {
     g->d_draw_dir = nullptr;
     g->d_draw_qnee = nullptr;
     g->draw_capacity = 0;
-    WR_HIP(hipMalloc(reinterpret_cast<void **>(&g->d_draw_dir), (sizeof(float4) + sizeof(float)) * size_t(capacity)));
+    WR_HIP(g->scene->dev->alloc(reinterpret_cast<void **>(&g->d_draw_dir), (sizeof(float4) + sizeof(float)) * size_t(capacity)));
     g->d_draw_qnee = reinterpret_cast<float *>(g->d_draw_dir + capacity);
     g->draw_capacity = capacity;
     return WR_OK;
@@ -896,20 +896,20 @@ static int guide_create_impl(wr_guide *g) {
     if (rc) return rc;
     int ndev_blocks = g->scene->dev->n_cu;
     g->train_blocks = std::min(kMaxTrainBlocks, ndev_blocks);
-    WR_HIP(hipMalloc(reinterpret_cast<void **>(&g->d_params), sizeof(float) * kNumParams));
-    WR_HIP(hipMalloc(reinterpret_cast<void **>(&g->d_m), sizeof(float) * kNumParams));
-    WR_HIP(hipMalloc(reinterpret_cast<void **>(&g->d_v), sizeof(float) * kNumParams));
-    WR_HIP(hipMalloc(reinterpret_cast<void **>(&g->d_avg), sizeof(float) * kNumParams));
-    WR_HIP(hipMalloc(reinterpret_cast<void **>(&g->d_fwd), sizeof(u32x4) * kFwdOps));
-    WR_HIP(hipMalloc(reinterpret_cast<void **>(&g->d_bwd), sizeof(u32x4) * kBwdOps));
-    WR_HIP(hipMalloc(reinterpret_cast<void **>(&g->d_bias), sizeof(float) * kBiasPacked));
-    WR_HIP(hipMalloc(reinterpret_cast<void **>(&g->d_fwd8), sizeof(u32x2) * kFwdOps));
-    WR_HIP(hipMalloc(reinterpret_cast<void **>(&g->d_wscale), sizeof(float) * kLayers));
-    WR_HIP(hipMalloc(reinterpret_cast<void **>(&g->d_partials), sizeof(float) * kNumParams * size_t(g->train_blocks)));
-    WR_HIP(hipMalloc(reinterpret_cast<void **>(&g->d_loss), sizeof(float) * g->train_blocks));
-    WR_HIP(hipMalloc(reinterpret_cast<void **>(&g->d_wsum), sizeof(double)));
+    WR_HIP(g->scene->dev->alloc(reinterpret_cast<void **>(&g->d_params), sizeof(float) * kNumParams));
+    WR_HIP(g->scene->dev->alloc(reinterpret_cast<void **>(&g->d_m), sizeof(float) * kNumParams));
+    WR_HIP(g->scene->dev->alloc(reinterpret_cast<void **>(&g->d_v), sizeof(float) * kNumParams));
+    WR_HIP(g->scene->dev->alloc(reinterpret_cast<void **>(&g->d_avg), sizeof(float) * kNumParams));
+    WR_HIP(g->scene->dev->alloc(reinterpret_cast<void **>(&g->d_fwd), sizeof(u32x4) * kFwdOps));
+    WR_HIP(g->scene->dev->alloc(reinterpret_cast<void **>(&g->d_bwd), sizeof(u32x4) * kBwdOps));
+    WR_HIP(g->scene->dev->alloc(reinterpret_cast<void **>(&g->d_bias), sizeof(float) * kBiasPacked));
+    WR_HIP(g->scene->dev->alloc(reinterpret_cast<void **>(&g->d_fwd8), sizeof(u32x2) * kFwdOps));
+    WR_HIP(g->scene->dev->alloc(reinterpret_cast<void **>(&g->d_wscale), sizeof(float) * kLayers));
+    WR_HIP(g->scene->dev->alloc(reinterpret_cast<void **>(&g->d_partials), sizeof(float) * kNumParams * size_t(g->train_blocks)));
+    WR_HIP(g->scene->dev->alloc(reinterpret_cast<void **>(&g->d_loss), sizeof(float) * g->train_blocks));
+    WR_HIP(g->scene->dev->alloc(reinterpret_cast<void **>(&g->d_wsum), sizeof(double)));
     const size_t cap = g->cfg.record_capacity;
-    WR_HIP(hipMalloc(&g->rec_pool, 2 * (sizeof(float4) * 6 * cap + 256)));
+    WR_HIP(g->scene->dev->alloc(&g->rec_pool, 2 * (sizeof(float4) * 6 * cap + 256)));
     for (int k = 0; k < 2; k++) {
         float4 *b = reinterpret_cast<float4 *>(static_cast<char *>(g->rec_pool) + k * (sizeof(float4) * 6 * cap + 256));
         Records &r = g->recs[k];
@@ -926,7 +926,7 @@ static int guide_create_impl(wr_guide *g) {
     const size_t fwd_b = (sizeof(u32x4) * kFwdOps + 255) / 256 * 256, bias_b = (sizeof(float) * kBiasPacked + 255) / 256 * 256;
     const size_t fwd8_b = (sizeof(u32x2) * kFwdOps + 255) / 256 * 256, ws_b = 256;
     const size_t set_b = fwd_b + bias_b + fwd8_b + ws_b;
-    WR_HIP(hipMalloc(&g->infer_pool, 2 * set_b));
+    WR_HIP(g->scene->dev->alloc(&g->infer_pool, 2 * set_b));
     for (int k = 0; k < 2; k++) {
         char *b = static_cast<char *>(g->infer_pool) + k * set_b;
         g->d_ifwd[k] = reinterpret_cast<u32x4 *>(b);
@@ -1004,7 +1004,7 @@ static int forward_impl(wr_guide *g, const float *pos, const float *nrm, const f
     hipStream_t st = g->scene->stream;
     float *d = nullptr;
     const size_t in_bytes = sizeof(float) * 9 * size_t(n), out_bytes = sizeof(float) * kOut * size_t(n);
-    WR_HIP(hipMalloc(reinterpret_cast<void **>(&d), in_bytes + out_bytes));
+    WR_HIP(g->scene->dev->alloc(reinterpret_cast<void **>(&d), in_bytes + out_bytes));
     float *dp = d, *dn = d + 3 * size_t(n), *dw = d + 6 * size_t(n), *dout = d + 9 * size_t(n);
     hipError_t e = hipMemcpyAsync(dp, pos, in_bytes / 3, hipMemcpyHostToDevice, st);
     if (e == hipSuccess) e = hipMemcpyAsync(dn, nrm, in_bytes / 3, hipMemcpyHostToDevice, st);
@@ -1040,7 +1040,7 @@ int wr_guide_gradient(wr_guide *g, const float *pos, const float *nrm, const flo
     rc = dr.upload(g->scene->dev, g->scene->stream, pos, nrm, wo, wi, weight, n);
     if (rc) return rc;
     float *dg = nullptr;
-    WR_HIP(hipMalloc(reinterpret_cast<void **>(&dg), sizeof(float) * kNumParams));
+    WR_HIP(g->scene->dev->alloc(reinterpret_cast<void **>(&dg), sizeof(float) * kNumParams));
     rc = train_step(g, dr.pos, dr.nrm, dr.wo, dr.wi, n, 0, n, 1.f / float(n), dg, loss, g->scene->stream);
     hipError_t e = hipSuccess;
     if (!rc) {
@@ -1082,7 +1082,7 @@ int wr_guide_mixture(wr_guide *g, const float *raw, const float *dirs, const flo
     hipStream_t st = g->scene->stream;
     float *d = nullptr;
     const size_t N = n;
-    WR_HIP(hipMalloc(reinterpret_cast<void **>(&d), sizeof(float) * N * (kOut + 3 + 3 + 1 + 3 + 1)));
+    WR_HIP(g->scene->dev->alloc(reinterpret_cast<void **>(&d), sizeof(float) * N * (kOut + 3 + 3 + 1 + 3 + 1)));
     float *draw = d, *ddir = d + kOut * N, *du = ddir + 3 * N, *dpd = du + 3 * N, *ds = dpd + N, *dsp = ds + 3 * N;
     hipError_t e = hipMemcpyAsync(draw, raw, sizeof(float) * kOut * N, hipMemcpyHostToDevice, st);
     if (e == hipSuccess) e = hipMemcpyAsync(ddir, dirs, sizeof(float) * 3 * N, hipMemcpyHostToDevice, st);

@@ -47,6 +47,13 @@ struct BlockPool {
         out->bytes = e == hipSuccess ? bytes : 0;
         return e;
     }
+    // bytes of the free blocks
+    size_t idle() {
+        std::lock_guard<std::mutex> lock(m);
+        size_t bytes = 0;
+        for (int i = 0; i < n; i++) bytes += held[i].bytes;
+        return bytes;
+    }
     // gives every free block back to the runtime
     void trim() {
         std::lock_guard<std::mutex> lock(m);
@@ -72,7 +79,8 @@ struct BlockPool {
     }
 };
 
-// The pools of a device handle, and allocations that may use what they hold idle.
+// The pools of a device handle, and the allocations of everything that belongs to
+// it, which get what the pools hold idle before they fail.
 struct DeviceMemory {
     BlockPool spills{2, size_t(1) << 30};       // traversal stack spill regions, one per scene
     BlockPool geometry{3, size_t(512) << 20, true};  // nodes (both copies) and triangles of GPU-built scenes
@@ -82,6 +90,7 @@ struct DeviceMemory {
         geometry.trim();
         build_memory.trim();
     }
+    size_t idle() { return spills.idle() + geometry.idle() + build_memory.idle(); }
     // hipMalloc that frees the pools' idle blocks where memory runs out
     hipError_t alloc(void **p, size_t bytes) {
         hipError_t e = hipMalloc(p, bytes);

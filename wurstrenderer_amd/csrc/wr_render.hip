@@ -2034,8 +2034,8 @@ int wr_bvh_selftest(const wr_scene_desc *d, uint64_t *n_nodes, uint32_t *max_sta
 }
 
 template <typename T>
-static int upload(T **dst, const void *src, size_t bytes, uint64_t &total) {
-    WR_HIP(hipMalloc(reinterpret_cast<void **>(dst), std::max<size_t>(bytes, 128)));
+static int upload(wr_device *dev, T **dst, const void *src, size_t bytes, uint64_t &total) {
+    WR_HIP(dev->alloc(reinterpret_cast<void **>(dst), std::max<size_t>(bytes, 128)));
     if (bytes) WR_HIP(hipMemcpy(*dst, src, bytes, hipMemcpyHostToDevice));
     total += bytes;
     return WR_OK;
@@ -2060,8 +2060,8 @@ static int bvh_host(wr_scene *s, const wr_scene_desc *d) {
     s->n_nodes = bvh.n_nodes;
     s->max_stack = bvh.max_stack;
     s->bvh_depth = bvh.depth;
-    int rc = upload(&s->d_nodes, bvh.nodes, sizeof(Node4) * bvh.n_nodes, s->device_bytes);
-    if (!rc) rc = upload(&s->d_tris, bvh.tris, sizeof(TriRecord) * bvh.n_tris, s->device_bytes);
+    int rc = upload(s->dev, &s->d_nodes, bvh.nodes, sizeof(Node4) * bvh.n_nodes, s->device_bytes);
+    if (!rc) rc = upload(s->dev, &s->d_tris, bvh.tris, sizeof(TriRecord) * bvh.n_tris, s->device_bytes);
     free_bvh(&bvh);
     s->build_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
     return rc;
@@ -2501,8 +2501,8 @@ int wr_scene_set_envmap(wr_scene *s, const float *rgb, uint32_t width, uint32_t 
     float4 *d_tex = nullptr;
     float *d_cp = nullptr;
     uint64_t bytes = 0;
-    rc = upload(&d_tex, tex.data(), sizeof(float4) * n, bytes);
-    if (!rc) rc = upload(&d_cp, cp.data(), sizeof(float) * 2 * n, bytes);
+    rc = upload(s->dev, &d_tex, tex.data(), sizeof(float4) * n, bytes);
+    if (!rc) rc = upload(s->dev, &d_cp, cp.data(), sizeof(float) * 2 * n, bytes);
     if (rc) {
         (void)hipFree(d_tex);
         return rc;
@@ -2669,13 +2669,14 @@ constexpr uint64_t kMaxSamplesPerPass = uint64_t(1) << 27;
 constexpr uint64_t kDefaultPool = uint64_t(1) << 27;
 // The default pool of a scene whose pool has to grow: `want` paths, but no
 // more than a quarter of the device memory that is free (counting the scene's
-// current pool, which the growth releases) -- many scenes can then keep their
+// current pool, which the growth releases, and the blocks that the device handle
+// holds idle, which an allocation gets where memory runs out) -- many scenes can then keep their
 // pools in one process -- and never below the current pool or 2^20 paths.
 static uint64_t default_pool_fit(const wr_scene *s, uint64_t want, uint64_t samples) {
     if (want <= s->capacity && samples <= s->sample_capacity) return want;
     size_t free_b = 0, total_b = 0;
     if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) return want;
-    uint64_t avail = free_b + (s->pool ? pool_bytes(s->capacity, s->sample_capacity) : 0);
+    uint64_t avail = free_b + s->dev->idle() + (s->pool ? pool_bytes(s->capacity, s->sample_capacity) : 0);
     const uint64_t per_path = pool_bytes(1 << 20, 0) >> 20;
     const uint64_t budget = avail / 4 > 16 * samples ? (avail / 4 - 16 * samples) / per_path : 0;
     const uint64_t floor = std::min<uint64_t>(want, std::max<uint64_t>(s->capacity, uint64_t(1) << 20));
@@ -3269,7 +3270,7 @@ int wr_render_batch(const wr_batch_job *jobs, uint32_t n_jobs, const wr_render_p
     pb.film_base = nullptr;  // per job, from the table
     pb.film_splat = nullptr;
     BatchJob *d_tab = nullptr;
-    WR_HIP(hipMalloc(reinterpret_cast<void **>(&d_tab), sizeof(BatchJob) * n_jobs));
+    WR_HIP(s0->dev->alloc(reinterpret_cast<void **>(&d_tab), sizeof(BatchJob) * n_jobs));
     struct Free { BatchJob *p; ~Free() { if (p) (void)hipFree(p); } } free_tab{d_tab};
     k_fill_u32<<<1, 64, 0, s0->stream>>>(reinterpret_cast<uint32_t *>(pb.stats), 0u, 12);
     WR_HIP(hipGetLastError());
