@@ -2630,6 +2630,13 @@ static unsigned long long *progress_word(wr_scene *s) {
 
 static int ensure_capacity(wr_scene *s, uint32_t cap, uint32_t samples) {
     if (s->capacity >= cap && s->sample_capacity >= samples) return WR_OK;
+    // first: a scene with a capacity has the counters' copy and the progress word, which the device writes
+    if (!s->h_counters) {
+        void *p = nullptr;
+        WR_HIP(hipHostMalloc(&p, sizeof(uint32_t) * kCounterStride * (kNumCounterLines + 1), hipHostMallocDefault));
+        s->h_counters = static_cast<uint32_t *>(p);
+        *progress_word(s) = 0;
+    }
     cap = std::max(cap, s->capacity);
     samples = std::max(samples, s->sample_capacity);
     if (s->pool) {
@@ -2645,11 +2652,6 @@ static int ensure_capacity(wr_scene *s, uint32_t cap, uint32_t samples) {
     pool_layout(p, cap, samples, &s->pb);
     s->capacity = cap;
     s->sample_capacity = samples;
-    if (!s->h_counters) {
-        WR_HIP(hipHostMalloc(reinterpret_cast<void **>(&s->h_counters),
-                             sizeof(uint32_t) * kCounterStride * (kNumCounterLines + 1), hipHostMallocDefault));
-        *progress_word(s) = 0;
-    }
     return WR_OK;
 }
 
