@@ -1,0 +1,40 @@
+"""Scenes with a vertex so far out that box areas overflow FP32 (from about 1e19 on).
+Every finite vertex is accepted, so the builders must still make a valid tree: a
+subtree of more triangles than a leaf holds stays a subtree, whatever its cost."""
+import dataclasses
+
+import numpy as np
+import pytest
+
+import wurstrenderer_amd as wr
+from wurstrenderer_amd import scenes
+
+FAR = [1e15, 3e18, 2e19, 1e20, 1e25, 1e30, 3e33, 1e34, 1e36, 1e38]
+
+
+def far_scene(far, sides=(1, 1, 1), near=None):
+    """A small scene and, behind its geometries, a triangle that reaches out to `far` on each axis."""
+    sc = near if near is not None else scenes.icospheres(2, n_spheres=4, level=2, resolution=(8, 8))
+    a = np.float32(far) * np.asarray(sides, np.float32)
+    verts = np.concatenate([sc.verts, [a, a * np.float32([1, 0.5, 1]), a * np.float32([1, 1, 0.5])]]).astype(np.float32)
+    nv = len(sc.verts)
+    return dataclasses.replace(sc, verts=verts, tris=np.concatenate([sc.tris, [[nv, nv + 1, nv + 2]]]).astype(np.uint32),
+                               tri_geom=np.append(sc.tri_geom, len(sc.geom_material)).astype(np.uint32),
+                               geom_material=np.append(sc.geom_material, 0).astype(np.int32),
+                               geom_light=np.append(sc.geom_light, -1).astype(np.int32))
+
+
+@pytest.mark.parametrize("far", FAR)
+def test_host_tree_is_valid(far):
+    wr.bvh_selftest(far_scene(far))
+    wr.bvh_selftest(far_scene(-far))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("far", FAR[:7])
+@pytest.mark.parametrize("builder", ["gpu", "host"])
+def test_device_tree_is_valid(gpu_device, builder, far):
+    print(f"far vertices: {builder} {far}", flush=True)
+    for sc in (far_scene(far), far_scene(-far)):
+        gs = wr.GpuScene(gpu_device, sc, builder=builder)
+        gs.bvh_check(sc)

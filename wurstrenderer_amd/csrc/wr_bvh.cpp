@@ -207,9 +207,11 @@ struct Collapser {
                 }
             }
             const float inner = kTraversalCost * A + dist[4];
-            const float leaf = cnt[q] <= uint32_t(kMaxLeafTris) ? kTriangleCost * A * float(cnt[q]) : FLT_MAX;
+            // more triangles than a leaf ref counts never become one leaf, also where the costs overflow
+            const bool fits = cnt[q] <= uint32_t(kMaxLeafTris);
+            const float leaf = fits ? kTriangleCost * A * float(cnt[q]) : FLT_MAX;
             c[0] = std::min(inner, leaf);
-            sp[0] = leaf <= inner ? 1 : 0;
+            sp[0] = fits && leaf <= inner ? 1 : 0;
             for (int i = 2; i <= 4; i++) {
                 if (dist[i] < c[i - 2]) { c[i - 1] = dist[i]; sp[i - 1] = dk[i]; }
                 else { c[i - 1] = c[i - 2]; sp[i - 1] = 0; }

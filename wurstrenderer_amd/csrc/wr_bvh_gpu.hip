@@ -333,9 +333,11 @@ __device__ __forceinline__ void merge_nodes(uint32_t a, uint32_t b, float4 la, f
             }
         }
         const float wide_inner = kCt * A + dist[4];
-        const float wide_leaf = cnt <= uint32_t(kMaxLeafTris) ? leaf_cost : INFINITY;
+        // more triangles than a leaf ref counts never become one leaf, also where the costs overflow
+        const bool fits = cnt <= uint32_t(kMaxLeafTris);
+        const float wide_leaf = fits ? leaf_cost : INFINITY;
         float c[4];
-        uint32_t w = wide_leaf <= wide_inner ? kWideLeaf : 0u;
+        uint32_t w = fits && wide_leaf <= wide_inner ? kWideLeaf : 0u;
         c[0] = fminf(wide_inner, wide_leaf);
 #pragma unroll
         for (int i = 2; i <= 4; i++) {
