@@ -2366,6 +2366,7 @@ int wr_scene_bvh_check(wr_scene *s, const wr_scene_desc *d, wr_bvh_stats *st) {
                     return set_error(WR_ERR_DEVICE, "BVH invariant violated: quantised node refs differ");
                 if (a.child[c] == kEmptyChild) continue;
                 for (int k = 0; k < 3; k++) {
+                    if (std::isinf(sc[k])) continue;  // spacing * 2^24 overflows: the axis encloses everything
                     const uint32_t w = pl[2 * k + (c >> 1)] >> (8 * (c & 1));
                     const double sp = double(sc[k]) * 0x1p-24;
                     if (!((w & 0xFFu) * sp <= double(lo[k][c]) - double(b.org[k]) &&

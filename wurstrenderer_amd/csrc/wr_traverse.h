@@ -229,9 +229,10 @@ struct LaneStack {
 // watertight test places a hit along the axis to about 2^-22 of the same sum.
 // b is therefore lowered for near planes and raised for far planes by
 // 2^-20 (|b| + 255 |g|), so a box the ray touches always has entry <= exit.
-// Where g overflows, that margin is infinite and every plane of the axis
-// becomes -inf / +inf or NaN, which max and min pass over: the axis culls
-// nothing.  An empty slot is rejected by its ref (kEmptyChild).
+// Where g or the stored spacing overflows, that margin is infinite and every
+// plane of the axis becomes -inf / +inf or NaN, which max and min pass over: the
+// axis culls nothing, and an exit that is NaN, on all three axes, does not
+// either.  An empty slot is rejected by its ref (kEmptyChild).
 // Returns the refs; tn holds the entry distances and hit[i] marks the
 // children whose box is entered before `far_limit`.
 //
@@ -273,7 +274,7 @@ __device__ __forceinline__ uint4 node_test(uint4 r0, uint4 r1, uint4 r2, uint4 r
 #pragma unroll
     for (int i = 0; i < 4; i++) {
         tn[i] = max3(n[0][i], n[1][i], fmaxf(n[2][i], r.tmin));
-        hit[i] = (c[i] != kEmptyChild) & (tn[i] <= min3(f[0][i], f[1][i], f[2][i])) & (tn[i] <= far_limit);
+        hit[i] = (c[i] != kEmptyChild) & !(tn[i] > min3(f[0][i], f[1][i], f[2][i])) & (tn[i] <= far_limit);
     }
     return ch;
 }
