@@ -1540,9 +1540,13 @@ __global__ void k_film_image(const double *__restrict__ base, const double *__re
 // Hits leave as (leaf triangle, t) pairs, or, with IDS, as what the host API
 // returns: the geometry, the triangle within it and t in three arrays of n
 // (a triangle record holds its input index and geometry; geom_first is each
-// geometry's first triangle).
+// geometry's first triangle).  A block takes tiles of 64 rays in a stride of the
+// grid, which is what is resident (8M any-hit rays among 1.31M triangles: 228 us,
+// 264 with 8,192 blocks of which 7,168 are).  Closest hit runs 8 waves per SIMD
+// (8M rays in a 40,000-triangle clutter 742 us, 7 waves 850), any hit, whose
+// registers fit 7 without spills, 7 (2M rays 104 us, 8 waves 116).
 template <bool ANY, bool IDS = false>
-__global__ __launch_bounds__(kBlock) void k_trace(DScene s, const float4 *__restrict__ rays, uint32_t n, uint2 *hits,
+__global__ __launch_bounds__(kBlock) WR_EXTEND_ATTR(ANY ? 7 : 8) void k_trace(DScene s, const float4 *__restrict__ rays, uint32_t n, uint2 *hits,
                                                   uint8_t *occ, const uint32_t *__restrict__ geom_first, uint2 *spill) {
     __shared__ uint64_t st_ent[kLdsSlots * kBlock];
     TraversalCounters cnt;
@@ -1939,7 +1943,6 @@ int wr_device_create(int ordinal, wr_device **out) {
     occ(reinterpret_cast<const void *>(&k_shade<false>), kShadeBlock, d->occ_shade);
 
     occ(reinterpret_cast<const void *>(&k_regen<false>), kShadeBlock, d->occ_generate);
-    occ(reinterpret_cast<const void *>(&k_trace<false>), kBlock, d->occ_trace);
     if (int rc = scratch_setup(d)) {
         delete d;
         return rc;
@@ -3143,7 +3146,9 @@ int wr_render_visualize(wr_scene *s, wr_film *f, const wr_render_params *prm, wr
     wr_render_stats st{};
     const uint32_t wh = uint32_t(s->W) * uint32_t(s->H);
     if (prm->spp > 0) {
-        const int grid = trav_grid(s, wh, s->dev->occ_trace);
+        // as many blocks as there are spill slices, 8,192, of which 5,120 are resident: the 1.31M-triangle scene
+        // at 1920 x 1080 takes 323 us (7,168, the residency of k_trace: 372), at 1280 x 720 187 (5,120: 234)
+        const int grid = trav_grid(s, wh, kMaxTraversalBlocksPerCU);
         if (prm->profile) WR_HIP(hipEventRecord(s->ev[0], s->stream));
         k_visualize<<<grid, kBlock, 0, s->stream>>>(s->ds, wh, uint32_t(prm->spp), uint32_t(prm->first_sample),
                                                     prm->seed, f->d_base, s->d_spill);
@@ -3472,7 +3477,10 @@ static int trace_impl(wr_scene *s, const float *d_rays, uint32_t n, void *d_hits
     int rc = set_device(s->dev);
     if (rc) return rc;
     if (n == 0) { if (ms) *ms = 0.f; return WR_OK; }
-    const int grid = trav_grid(s, n, s->dev->occ_trace);
+    const void *fn = any ? reinterpret_cast<const void *>(&k_trace<true>)
+                    : ids ? reinterpret_cast<const void *>(&k_trace<false, true>)
+                          : reinterpret_cast<const void *>(&k_trace<false>);
+    const int grid = trav_grid(s, n, occupancy(s->dev, fn, kBlock));
     if (ms) WR_HIP(hipEventRecord(s->ev[0], s->stream));
     const float4 *rays = reinterpret_cast<const float4 *>(d_rays);
     uint2 *hits = reinterpret_cast<uint2 *>(d_hits);
