@@ -60,6 +60,15 @@ def test_film_reads_equal_single_arrays(gpu_device, size):
     np.testing.assert_array_equal(film.image(), base / 2 + splat / (2 * size * size))
 
 
+def _shortest(call, times):
+    best = np.inf
+    for _ in range(times):
+        t = time.perf_counter()
+        call()
+        best = min(best, time.perf_counter() - t)
+    return best
+
+
 def test_a_small_query_is_one_launch_and_one_wait(gpu_device):
     """1,000 hits take 28 us and a plain copy of 31 KB (Guide.get_params) 13 us; with
     a wait for each array's own transfer the query took 102, with two waits and the
@@ -68,15 +77,27 @@ def test_a_small_query_is_one_launch_and_one_wait(gpu_device):
     gs = wr.GpuScene(gpu_device, sc)
     guide = wr.Guide(gs)
     rays = scenes.random_rays(sc, 1000, seed=1)
-
-    def shortest(call):
-        best = np.inf
-        for _ in range(300):
-            t = time.perf_counter()
-            call()
-            best = min(best, time.perf_counter() - t)
-        return best
-
-    query, copy = shortest(lambda: gs.trace_closest(rays)), shortest(guide.get_params)
+    query, copy = _shortest(lambda: gs.trace_closest(rays), 300), _shortest(guide.get_params, 300)
     print(f"query {query * 1e6:.1f} us, copy {copy * 1e6:.1f} us", flush=True)
     assert query < 4 * copy
+
+
+def test_uploads_grow_evenly_with_their_size(gpu_device):
+    """Gradients of 60,000 and 80,000 records (3.1 and 4.2 MB up): the larger takes at
+    most 4/3 of the smaller (and 5%), where threads started for it made it 1.5 at best
+    and 2.3 at the median (278 us and 650)."""
+    sc = scenes.cornell(1, (8, 8))
+    guide = wr.Guide(wr.GpuScene(gpu_device, sc))
+    rng = np.random.default_rng(1)
+
+    def records(n):
+        v = rng.normal(size=(4, n, 3)).astype(np.float32)
+        v[1:] /= np.linalg.norm(v[1:], axis=2, keepdims=True)
+        return (*v, np.ones(n, np.float32))
+
+    times = []
+    for n in (60_000, 80_000):
+        r = records(n)
+        times.append(_shortest(lambda: guide.gradient(*r), 100))
+        print(f"gradient of {n}: {times[-1] * 1e6:.0f} us", flush=True)
+    assert times[1] < 1.4 * times[0]

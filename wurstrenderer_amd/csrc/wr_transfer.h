@@ -1,15 +1,18 @@
 // wr_transfer.h -- large host <-> device transfers through a small ring of
-// pinned buffers, filled or emptied by several host threads.
+// pinned buffers, for downloads emptied by several host threads.
 //
 // A hipMemcpy of pageable memory is one host thread's work: 50 MB into a fresh
 // array measured 11.3 ms (4.4 GB/s: the thread also takes the array's page
-// faults), 40 MB from host arrays 1.5 to 7.9 ms, while the link moves 55 GB/s
-// and eight threads touch and copy a fresh 50 MB in 2.3 ms.  So a transfer is
-// cut into chunks of 1 MB; chunk c uses ring slot c mod kSlots and host thread
-// c mod threads, and because kSlots is a multiple of the thread count a slot
-// belongs to one thread, which alone waits for its event, copies, and issues
-// the slot's next chunk.  Transfers below kThreadedBytes run on the calling
-// thread (starting one costs about 30 us).
+// faults), while the link moves 55 GB/s and eight threads touch and copy a fresh
+// 50 MB in 2.3 ms.  So a transfer is cut into chunks of 1 MB; chunk c uses ring
+// slot c mod kSlots and host thread c mod threads, and because kSlots is a
+// multiple of the thread count a slot belongs to one thread, which alone waits
+// for its event, copies, and issues the slot's next chunk.  Downloads below
+// kThreadedBytes run on the calling thread (starting the others costs about
+// 100 us), and so do all uploads: their sources are written already, and one
+// thread's copies keep up with the link's (records of a gradient, 4 MB, 310 us
+// with the call, 650 with eight threads; 13.6 MB 620 and 710; scene of 41 MB 4.05
+// and 4.35 ms).
 //
 // The ring (16 MB) belongs to a device handle, is allocated on its first
 // transfer and freed with the handle; a mutex lets one transfer use it at a
@@ -101,7 +104,7 @@ struct TransferRing {
         size_t total = 0;
         for (const Part &p : parts) total += p.bytes;
         return run(
-            ordinal, stream, total, threads_for(total), false,
+            ordinal, stream, total, 1, false,
             [out, stream](size_t off, size_t n, char *slot) {
                 return hipMemcpyAsync(out + off, slot, n, hipMemcpyHostToDevice, stream);
             },
