@@ -114,13 +114,23 @@ struct TransferRing {
                 });
             });
     }
-    // The ring for one caller, whose kernel reads and writes pinned memory directly:
-    // a chunk `in` and kSlots - 1 chunks `out`, until the lease dies.  The caller
-    // waits for its stream before that.
+    // The ring for one caller, whose device work reads and writes pinned memory
+    // itself: a chunk `in` and kSlots - 1 chunks `out`, until the lease is given back
+    // or dies.  The caller waits for that work before, or marks the lease behind it.
     static constexpr size_t kLeaseIn = kChunk, kLeaseOut = (kSlots - 1) * kChunk;
     struct Lease {
         std::unique_lock<std::mutex> lock;
         char *in = nullptr, *out = nullptr;
+        hipEvent_t used = nullptr;
+        Lease() = default;
+        Lease(const Lease &) = delete;
+        Lease &operator=(const Lease &) = delete;
+        ~Lease() { give(); }
+        void give() {
+            if (used) (void)hipEventSynchronize(used);
+            used = nullptr;
+            if (lock.owns_lock()) lock.unlock();
+        }
     };
     hipError_t lease(Lease *l) {
         l->lock = std::unique_lock<std::mutex>(busy);
@@ -129,6 +139,15 @@ struct TransferRing {
         l->in = pinned;
         l->out = pinned + kLeaseIn;
         return hipSuccess;
+    }
+    // Giving the lease back waits for what `stream` holds now, and no more.
+    hipError_t mark(Lease *l, hipStream_t stream) {
+        hipError_t e = done[0] ? hipSuccess : hipEventCreateWithFlags(&done[0], hipEventDisableTiming);
+        if (e != hipSuccess) done[0] = nullptr;
+        if (e == hipSuccess) e = hipEventRecord(done[0], stream);
+        if (e == hipSuccess) l->used = done[0];
+        else (void)hipStreamSynchronize(stream);
+        return e;
     }
     // Host copies of the parts, by several threads from kThreadedBytes on.
     static void copy(std::initializer_list<Out> parts) {
