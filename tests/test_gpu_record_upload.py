@@ -1,5 +1,5 @@
-"""Records of up to one chunk of the pinned ring (20,164) go up without a wait of
-their own, larger ones chunk by chunk.  Weightless records add nothing and the factors are
+"""Records of up to what the pinned ring holds (322,638) go up without a wait of their
+own, in chunks of 20,164, more of them through the ring's slots in turn.  Weightless records add nothing and the factors are
 powers of two, so a gradient over n records equals one over 2n bit for bit."""
 import threading
 
@@ -57,3 +57,26 @@ def test_training_and_transfers_of_several_threads(gpu_device):
     [t.start() for t in threads]
     [t.join(60) for t in threads]
     assert not bad and not any(t.is_alive() for t in threads)
+
+
+@pytest.mark.parametrize("n", [322_638, 322_639, 400_000])
+def test_uploads_around_the_size_of_the_ring(guide_scene, n):  # noqa: F811
+    """The last 4,096 records count and the rest are weightless, so the sums are those
+    of a gradient over the 4,096 alone, FP32 sums of the same products in another order
+    (the bars of the gradient test: loss 1e-3, gradient 1e-2 in relative L2 norm)."""
+    sc, gs = guide_scene
+    print(f"record upload: {n}", flush=True)
+    g = wr.Guide(gs)
+    rng = np.random.default_rng(n)
+    g.set_params(params(rng, scale_out=1.0))
+    few = records(rng, 4096, scene_box(sc))
+    pos, nrm, wo, wi = (np.resize(a, (n, 3)) for a in few[:4])
+    w = np.zeros(n, np.float32)
+    w[-4096:] = np.resize(few[4], n)[-4096:]
+    last = [np.ascontiguousarray(a[-4096:]) for a in (pos, nrm, wo, wi, w)]
+    loss, grad = g.gradient(pos, nrm, wo, wi, w)
+    loss1, grad1 = g.gradient(*last)
+    # means over n and over 4,096 records
+    np.testing.assert_allclose(loss * n, loss1 * 4096, rtol=1e-4)
+    a, b = grad * np.float32(n), grad1 * np.float32(4096)
+    assert np.linalg.norm(a - b) < 1e-2 * np.linalg.norm(b)

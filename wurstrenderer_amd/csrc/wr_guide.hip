@@ -696,9 +696,9 @@ int train_step(wr_guide *g, const float4 *pos, const float4 *nrm, const float4 *
 }
 
 // Host records -> temporary device arrays (float4 each): the caller's arrays go
-// up as they are and k_unpack spreads them.  Up to a chunk of the ring, 20,164
-// records, nothing waits for the copy but the kernels behind it: the caller gives
-// the ring back once it has enqueued its first step (2 steps on 1,000 records:
+// up as they are and k_unpack spreads them.  Up to what the ring holds, 322,638
+// records, nothing waits for the copies but the kernels behind them: the caller
+// gives the ring back once it has enqueued its first step (2 steps on 1,000 records:
 // 172 us, with a wait of the copy's own 186).
 struct DeviceRecords {
     float4 *buf = nullptr;
@@ -714,15 +714,9 @@ struct DeviceRecords {
         WR_HIP(dev->alloc(reinterpret_cast<void **>(&buf), 4 * sizeof(float4) * size_t(n) + raw));
         pos = buf; nrm = buf + n; wo = buf + 2 * size_t(n); wi = buf + 3 * size_t(n);
         float *d_raw = reinterpret_cast<float *>(buf + 4 * size_t(n));
-        if (raw <= TransferRing::kLeaseIn) {
-            WR_HIP(dev->ring.lease(&staged));
-            TransferRing::copy({{staged.in, p, row}, {staged.in + row, nr, row}, {staged.in + 2 * row, o, row},
-                                {staged.in + 3 * row, i, row}, {staged.in + 4 * row, w, raw - 4 * row}});
-            WR_HIP(hipMemcpyAsync(d_raw, staged.in, raw, hipMemcpyHostToDevice, st));
-            WR_HIP(dev->ring.mark(&staged, st));
-        } else {
-            WR_HIP(dev->ring.upload(dev->ordinal, st, d_raw, {{p, row}, {nr, row}, {o, row}, {i, row}, {w, raw - 4 * row}}));
-        }
+        const std::initializer_list<TransferRing::Part> parts = {{p, row}, {nr, row}, {o, row}, {i, row}, {w, raw - 4 * row}};
+        if (raw <= TransferRing::kLeaseAll) WR_HIP(dev->ring.stage(&staged, st, d_raw, parts));
+        else WR_HIP(dev->ring.upload(dev->ordinal, st, d_raw, parts));
         k_unpack<<<(n + 255) / 256, 256, 0, st>>>(d_raw, n, buf);
         WR_HIP(hipGetLastError());
         return WR_OK;

@@ -116,7 +116,7 @@ struct TransferRing {
     }
     // The ring for one caller, whose device work reads and writes pinned memory
     // itself: a chunk `in` and kSlots - 1 chunks `out`, until the lease is given back
-    // or dies.  The caller waits for that work before, or marks the lease behind it.
+    // or dies.  The caller waits for that work before (stage() has its own wait).
     static constexpr size_t kLeaseIn = kChunk, kLeaseOut = (kSlots - 1) * kChunk;
     struct Lease {
         std::unique_lock<std::mutex> lock;
@@ -140,10 +140,25 @@ struct TransferRing {
         l->out = pinned + kLeaseIn;
         return hipSuccess;
     }
-    // Giving the lease back waits for what `stream` holds now, and no more.
-    hipError_t mark(Lease *l, hipStream_t stream) {
-        hipError_t e = done[0] ? hipSuccess : hipEventCreateWithFlags(&done[0], hipEventDisableTiming);
-        if (e != hipSuccess) done[0] = nullptr;
+    // Host to device through a lease of the whole ring, for parts of up to
+    // kLeaseAll bytes: enqueued on `stream` when it returns, and the sources may be
+    // reused.  Giving the lease back waits for the copies.
+    static constexpr size_t kLeaseAll = kSlots * kChunk;
+    hipError_t stage(Lease *l, hipStream_t stream, void *device, std::initializer_list<Part> parts) {
+        hipError_t e = lease(l);
+        size_t total = 0;
+        for (const Part &p : parts) total += p.bytes;
+        for (size_t off = 0; off < total && e == hipSuccess; off += kChunk) {
+            const size_t n = std::min(kChunk, total - off);
+            pieces(parts, off, n, pinned + off, [](const Part &p, size_t at, char *piece, size_t m) {
+                std::memcpy(piece, static_cast<const char *>(p.src) + at, m);
+            });
+            e = hipMemcpyAsync(static_cast<char *>(device) + off, pinned + off, n, hipMemcpyHostToDevice, stream);
+        }
+        if (e == hipSuccess && !done[0]) {
+            e = hipEventCreateWithFlags(&done[0], hipEventDisableTiming);
+            if (e != hipSuccess) done[0] = nullptr;
+        }
         if (e == hipSuccess) e = hipEventRecord(done[0], stream);
         if (e == hipSuccess) l->used = done[0];
         else (void)hipStreamSynchronize(stream);
