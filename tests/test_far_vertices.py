@@ -67,3 +67,30 @@ def test_near_triangles_are_hit_whatever_lies_far_out(gpu_device, builder, far):
         short = rays.copy()
         short[:, 7] = np.where(hit, t0 * np.float32(1.01), 1.0)
         assert gs.trace_any(short)[hit].all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("value", [np.nan, np.inf, -np.inf])
+def test_rays_that_are_not_finite_miss_at_the_root(gpu_device, value):
+    """One component or all of an origin or a direction; the finite rays between them
+    keep their hits, and a wave of such rays costs what a wave of misses costs, not
+    the whole tree (300,000 nodes one after the other, a microsecond each)."""
+    import time
+
+    print(f"rays that are not finite: {value}", flush=True)
+    sc = scenes.icospheres(2, n_spheres=64, level=5, resolution=(8, 8))
+    gs = wr.GpuScene(gpu_device, sc)
+    rays = scenes.random_rays(sc, 640, seed=3)
+    want = gs.trace_closest(rays)
+    assert (want[0] != 0xFFFFFFFF).sum() > 50
+    broken = np.arange(640) % 5 == 0
+    for where in ([0], [0, 1, 2], [4], [6], [4, 5, 6], [0, 1, 2, 4, 5, 6]):
+        r = rays.copy()
+        r[np.ix_(broken, where)] = value
+        g, p, t = gs.trace_closest(r)
+        assert (g[broken] == 0xFFFFFFFF).all() and np.isinf(t[broken]).all() and not gs.trace_any(r)[broken].any()
+        for a, b in zip((g, p, t), want):
+            np.testing.assert_array_equal(a[~broken], b[~broken])
+        start = time.perf_counter()
+        gs.trace_closest(r)
+        assert time.perf_counter() - start < 0.02

@@ -332,7 +332,10 @@ struct TravState {
 
 __device__ __forceinline__ void trav_begin(TravState &ts, const RaySetup &r, float tmax) {
     ts.r = r;
-    ts.t = tmax;
+    // A ray that is not a number gets that as its far limit, so that no box is
+    // entered and it misses at the root: NaN planes alone cull nothing and would
+    // take it through the whole tree.
+    ts.t = fmaf(r.ix, 0.f, fmaf(r.iy, 0.f, fmaf(r.iz, 0.f, fmaf(r.o.x, 0.f, fmaf(r.o.y, 0.f, fmaf(r.o.z, 0.f, tmax))))));
     ts.hit = kInvalid;
     ts.cur = 0;  // root (internal node 0)
 }
