@@ -781,12 +781,13 @@ int build_bvh4_gpu(wr_device *dev, const BuildBuffers &b, uint32_t n, hipStream_
     }
     k_ploc_tail<<<1, kTailBlock, 0, stream>>>(d_state, cl, R, nlo, nhi, kids, wc, wd, tail);
     WR_HIP(hipGetLastError());
+    // (taken before the copy to the stack: running out of memory leaves nothing in flight to a frame that is gone)
+    WR_HIP(dev->take(dev->geometry, std::max<size_t>(sizeof(TriRecord) * n, 128), &res->tris_block));
+    res->tris = static_cast<TriRecord *>(res->tris_block.p);
     uint32_t ended[4];
     WR_HIP(hipMemcpyAsync(ended, tail, sizeof ended, hipMemcpyDeviceToHost, stream));
 
     // collapse, level by level (breadth-first node order: children after parents)
-    WR_HIP(dev->take(dev->geometry, std::max<size_t>(sizeof(TriRecord) * n, 128), &res->tris_block));
-    res->tris = static_cast<TriRecord *>(res->tris_block.p);
     WR_HIP(hipStreamSynchronize(stream));
     if (ended[3]) return set_error(WR_ERR_DEVICE, "GPU BVH build: clustering made no progress (non-finite vertices?)");
     if (ended[1] != nn) return set_error(WR_ERR_DEVICE, "GPU BVH build: node count mismatch");
@@ -818,10 +819,10 @@ int build_bvh4_gpu(wr_device *dev, const BuildBuffers &b, uint32_t n, hipStream_
         depth++;
     }
     const uint32_t n_nodes = level_base;
-    uint32_t ms = 0;
-    WR_HIP(hipMemcpyAsync(&ms, max_stack, sizeof ms, hipMemcpyDeviceToHost, stream));
     WR_HIP(dev->take(dev->geometry, sizeof(Node4) * n_nodes, &res->nodes_block));
     res->nodes = static_cast<Node4 *>(res->nodes_block.p);
+    uint32_t ms = 0;
+    WR_HIP(hipMemcpyAsync(&ms, max_stack, sizeof ms, hipMemcpyDeviceToHost, stream));
     WR_HIP(hipMemcpyAsync(res->nodes, nodes_tmp, sizeof(Node4) * n_nodes, hipMemcpyDeviceToDevice, stream));
     WR_HIP(hipStreamSynchronize(stream));
     res->n_nodes = n_nodes;
