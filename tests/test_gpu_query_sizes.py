@@ -4,6 +4,7 @@ Rays: up to 32,768 are read from pinned memory by the kernel; up to 1,310,720 hi
 and 15,728,640 flags are written there.  Films: arrays up to 16 KB and from 1.2 MB
 on (26^2 and 27^2, 223^2 and 224^2 pixels) come through the pinned ring, those in
 between by plain copies.  Everything is exact, so comparisons are too."""
+import threading
 import time
 
 import numpy as np
@@ -101,3 +102,27 @@ def test_uploads_grow_evenly_with_their_size(gpu_device):
         times.append(_shortest(lambda: guide.gradient(*r), 100))
         print(f"gradient of {n}: {times[-1] * 1e6:.0f} us", flush=True)
     assert times[1] < 1.4 * times[0]
+
+
+def test_queries_of_several_threads(gpu_device):
+    """Four scenes of one device, queried at the same time: some calls find the pinned
+    ring free and some do not, and all answer what they answer alone."""
+    print("queries of several threads", flush=True)
+    work, bad = [], []
+    for k, n in enumerate((1000, 30_000, 40_000, 1_400_000)):
+        sc = scenes.icospheres(2 + k, n_spheres=6, level=3, resolution=(8, 8))
+        gs = wr.GpuScene(gpu_device, sc)
+        rays = scenes.random_rays(sc, n, seed=k)
+        work.append((gs, rays, gs.trace_closest(rays), gs.trace_any(rays)))
+
+    def query(gs, rays, hits, flags):
+        for _ in range(400_000 // len(rays) + 2):
+            if not all(np.array_equal(a, b) for a, b in zip(gs.trace_closest(rays), hits)):
+                bad.append(len(rays))
+            if not np.array_equal(gs.trace_any(rays), flags):
+                bad.append(len(rays))
+
+    threads = [threading.Thread(target=query, args=w) for w in work]
+    [t.start() for t in threads]
+    [t.join(60) for t in threads]
+    assert not bad and not any(t.is_alive() for t in threads)

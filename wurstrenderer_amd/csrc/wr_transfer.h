@@ -73,13 +73,7 @@ struct TransferRing {
             total += p.bytes;
             most = std::max(most, p.bytes);
         }
-        if (most > kPlainAbove && most < kPlainBelow) {
-            hipError_t e = hipSuccess;
-            for (const Out &p : parts)
-                if (e == hipSuccess && p.bytes) e = hipMemcpyAsync(p.dst, p.src, p.bytes, hipMemcpyDeviceToHost, stream);
-            const hipError_t w = hipStreamSynchronize(stream);
-            return e != hipSuccess ? e : w;
-        }
+        if (most > kPlainAbove && most < kPlainBelow) return plain(stream, parts);
         return run(
             ordinal, stream, total, threads_for(most), true,
             [&parts, stream](size_t off, size_t n, char *slot) {
@@ -95,6 +89,14 @@ struct TransferRing {
                     std::memcpy(static_cast<char *>(p.dst) + at, piece, m);
                 });
             });
+    }
+    // By the runtime's own copies, without the ring.
+    static hipError_t plain(hipStream_t stream, std::initializer_list<Out> parts) {
+        hipError_t e = hipSuccess;
+        for (const Out &p : parts)
+            if (e == hipSuccess && p.bytes) e = hipMemcpyAsync(p.dst, p.src, p.bytes, hipMemcpyDeviceToHost, stream);
+        const hipError_t w = hipStreamSynchronize(stream);
+        return e != hipSuccess ? e : w;
     }
     // Host to device on `stream`: the parts, one behind the other.  The sources
     // may be reused when it returns, and the copies are complete.
@@ -134,11 +136,12 @@ struct TransferRing {
     };
     hipError_t lease(Lease *l) {
         l->lock = std::unique_lock<std::mutex>(busy);
-        const hipError_t e = allocate();
-        if (e != hipSuccess) return e;
-        l->in = pinned;
-        l->out = pinned + kLeaseIn;
-        return hipSuccess;
+        return leased(l);
+    }
+    // The same if no other transfer has the ring; `in` stays null where one has.
+    hipError_t try_lease(Lease *l) {
+        l->lock = std::unique_lock<std::mutex>(busy, std::try_to_lock);
+        return l->lock.owns_lock() ? leased(l) : hipSuccess;
     }
     // Host to device through a lease of the whole ring, for parts of up to
     // kLeaseAll bytes: enqueued on `stream` when it returns, and the sources may be
@@ -179,6 +182,13 @@ struct TransferRing {
     }
 
 private:
+    hipError_t leased(Lease *l) {
+        const hipError_t e = allocate();
+        if (e != hipSuccess) return e;
+        l->in = pinned;
+        l->out = pinned + kLeaseIn;
+        return hipSuccess;
+    }
     // The ring's memory, on first use; `busy` is held.
     hipError_t allocate() {
         if (pinned) return hipSuccess;
