@@ -62,7 +62,6 @@ struct DScene {
     const DLight *lights;
     const float4 *ltris;      // 3 float4 per emitter triangle
     uint32_t n_lights;
-    uint32_t n_nodes;
     DCamera cam;
     DMedium med;
     // envmap light (EnvmapLight over an equirectangular image, light/envmap.h):

@@ -121,7 +121,7 @@ struct wr_device : wr::DeviceMemory {
     int ordinal = 0;
     int n_cu = 256;
     // resident blocks per CU of each kernel (HIP occupancy API), used to size persistent grids
-    int occ_rays = 8, occ_shade = 8, occ_generate = 8;
+    int occ_rays = 8, occ_generate = 8;
     std::mutex occ_mutex;  // guards occ_cache
     std::map<const void *, int> occ_cache;  // other kernels, filled on first use
     TransferRing ring;        // pinned buffers of large host transfers

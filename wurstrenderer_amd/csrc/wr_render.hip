@@ -73,17 +73,6 @@ __device__ __forceinline__ uint32_t mbcnt64(unsigned long long mask) {
     return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
 }
 
-// Wave-aggregated append: one atomic per wave.  All lanes must call it.
-__device__ __forceinline__ uint32_t wave_append(uint32_t *counter, bool pred) {
-    const unsigned long long mask = __ballot(pred);
-    if (mask == 0) return kInvalid;
-    const uint32_t leader = __ffsll((long long)mask) - 1;
-    uint32_t base = 0;
-    if (lane_id() == leader) base = atomicAdd(counter, (uint32_t)__popcll(mask));
-    base = __shfl(base, leader);
-    return pred ? base + mbcnt64(mask) : kInvalid;
-}
-
 // Block-aggregated append: one atomic per block of up to kShadeBlock threads.
 // All threads of the block must call it (it synchronises the block).
 constexpr int kShadeBlock = 512;
@@ -1279,7 +1268,7 @@ __global__ __launch_bounds__(kShadeBlock) void k_shade_ext(DScene s, PathBuffers
 // this iteration's regeneration) filled; a visible connection adds its
 // contribution to the radiance of its path (continuing: by then in the
 // current state; finished: its sample), or to the FP64 splat film for
-// light->camera (t = 1) connections.  `st_node` is the block's LDS stack of
+// light->camera (t = 1) connections.  `st_ent` is the block's LDS stack, here of
 // node refs (any hit keeps no entry distances).
 template <bool COUNT, bool BATCH>
 __device__ __forceinline__ void shadow_rays(DScene s1, const BatchJob *__restrict__ jobs, PathBuffers pb, uint2 *spill,
@@ -1396,8 +1385,8 @@ __global__ __launch_bounds__(kBlock) WR_EXTEND_ATTR(WR_BATCH_WAVES) void k_trace
 //   spheres, 1.31M         1.54 / 0.59  2.27 / 0.95  2.34 / 1.27  3.09 / 2.40
 //   gap room, 1.0M         2.31 / 1.33  2.99 / 1.68  3.21 / 3.04  7.70 / 10.4
 // (16,777,216 in the Cornell box 14.2 / 14.2), hence small_pass_samples.  Six
-// waves per SIMD: the registers still hold everything, and 262,144 samples of
-// the gap room take 3.6 ms at four.  Restarting at 1 / 8 / 16 / 32 idle lanes:
+// waves per SIMD, at which 132 bytes a lane spill to scratch (192 with an envmap):
+// 262,144 samples of the gap room take 3.04 ms, 3.6 at four.  Restarting at 1 / 8 / 16 / 32 idle lanes:
 // 3.91 / 3.78 / 3.72 / 3.96 ms in the box at 4,194,304 samples.
 constexpr uint32_t kRestartLanes = 16;
 // Largest pass of k_small_pass in a scene of n_tris triangles; passes of at most
@@ -1940,8 +1929,6 @@ int wr_device_create(int ordinal, wr_device **out) {
         out_blocks = std::min(out_blocks, kMaxTraversalBlocksPerCU);
     };
     occ(reinterpret_cast<const void *>(&k_trace_bounce_fast), kBlock, d->occ_rays);
-    occ(reinterpret_cast<const void *>(&k_shade<false>), kShadeBlock, d->occ_shade);
-
     occ(reinterpret_cast<const void *>(&k_regen<false>), kShadeBlock, d->occ_generate);
     if (int rc = scratch_setup(d)) {
         delete d;
@@ -2284,7 +2271,6 @@ static int scene_create_impl(wr_device *dev, const wr_scene_desc *d, int builder
     dc.focal = c.focal_distance;
     s->ds.nodes = s->d_qnodes;
     s->ds.fnodes = s->d_nodes;
-    s->ds.n_nodes = uint32_t(s->n_nodes);
     s->ds.tris = s->d_tris;
     s->ds.geom_info = s->d_geom;
     s->ds.mats = s->d_mats;

@@ -26,7 +26,7 @@ struct RaySetup {
     int kz;                    // watertight test: the axis of the largest direction component
     float Sx, Sy, Sz;
     uint32_t onx, ony, onz;    // byte offsets of the near-plane rows in a Node4 (the far row is at offset ^ 16)
-    uint32_t snx, sny, snz;    // byte selectors of the near planes in a NodeQ plane word (kSelNear / kSelFar)
+    uint32_t snx, sny, snz;    // byte selectors of the near planes in a NodeQ plane word (kSelLow / kSelHigh)
 };
 
 // v_perm_b32 selectors that spread two planes of a NodeQ plane word (child a's
@@ -341,7 +341,7 @@ __device__ __forceinline__ void trav_begin(TravState &ts, const RaySetup &r, flo
 }
 
 // Orders the children near to far, pushes the entered ones but the nearest,
-// farthest first, and returns the nearest (kInvalid if none is entered).  A
+// farthest first, and returns the nearest (kPopRef if none is entered).  A
 // key is the 64-bit stack entry (child ref low, entry distance bits high), its
 // high word kNoEntry for a child whose box is not entered.  Read as doubles,
 // keys order by their high words (an FP32 pattern up to infinity is the high
