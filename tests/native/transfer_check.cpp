@@ -1,5 +1,5 @@
 // Transfers through the pinned ring against a runtime whose events can fail.
-//   transfer_check <up|down> <record|sync|none> <call that fails> <MB>
+//   transfer_check <up|down|stage> <record|sync|none> <call that fails> <MB>
 // Exit 0: a transfer that succeeds has moved every byte; one that fails says so, has
 // nothing in flight that could still touch the caller's memory or the ring, never
 // filled a slot whose copy was still to run, and the next transfer works.
@@ -12,7 +12,7 @@
 
 int main(int argc, char **argv) {
     if (argc != 5) return 64;
-    const bool up = std::string(argv[1]) == "up";
+    const bool stage = std::string(argv[1]) == "stage", up = stage || std::string(argv[1]) == "up";
     const std::string what = argv[2];
     const size_t bytes = (size_t(std::atoi(argv[4])) << 20) + 12345;
     std::vector<char> host(bytes), device(bytes, 0);
@@ -22,12 +22,17 @@ int main(int argc, char **argv) {
     hipStream_t st = reinterpret_cast<hipStream_t>(&ring);
     auto once = [&] {
         const size_t half = bytes / 3;
+        if (stage) {
+            wr::TransferRing::Lease lease;  // given back, with its copies done, when the lambda returns
+            return ring.stage(&lease, st, device.data(), {{host.data(), half}, {host.data() + half, bytes - half}});
+        }
         return up ? ring.upload(0, st, device.data(), {{host.data(), half}, {host.data() + half, bytes - half}})
                   : ring.download(0, st, {{host.data(), device.data(), half}, {host.data() + half, device.data() + half, bytes - half}});
     };
     (what == "record" ? fake::record_fails_at : fake::sync_fails_at) = what == "none" ? -1 : std::atoi(argv[3]);
     const hipError_t e = once();
-    const bool failed = what != "none" && (what == "record" ? fake::records : fake::syncs) > std::atoi(argv[3]);
+    // (the wait of a lease has nobody to tell, and falls back on the stream's)
+    const bool failed = what != "none" && !(stage && what == "sync") && (what == "record" ? fake::records : fake::syncs) > std::atoi(argv[3]);
     if (failed != (e != hipSuccess)) return std::puts("the error is not reported"), 1;
     if (fake::pending()) return std::puts("work is still in flight"), 2;
     // bytes that arrived are the right ones (a slot filled too early sends another chunk's)

@@ -123,13 +123,14 @@ struct TransferRing {
     struct Lease {
         std::unique_lock<std::mutex> lock;
         char *in = nullptr, *out = nullptr;
-        hipEvent_t used = nullptr;
+        hipEvent_t used = nullptr;      // behind the copies of stage(), on `stream`
+        hipStream_t stream = nullptr;
         Lease() = default;
         Lease(const Lease &) = delete;
         Lease &operator=(const Lease &) = delete;
         ~Lease() { give(); }
         void give() {
-            if (used) (void)hipEventSynchronize(used);
+            if (used && hipEventSynchronize(used) != hipSuccess) (void)hipStreamSynchronize(stream);
             used = nullptr;
             if (lock.owns_lock()) lock.unlock();
         }
@@ -163,6 +164,7 @@ struct TransferRing {
             if (e != hipSuccess) done[0] = nullptr;
         }
         if (e == hipSuccess) e = hipEventRecord(done[0], stream);
+        l->stream = stream;
         if (e == hipSuccess) l->used = done[0];
         else (void)hipStreamSynchronize(stream);
         return e;
